@@ -394,9 +394,9 @@ struct mce_plan {
   uint8_t *d_stacks = nullptr;
   ShareRec *d_recs = nullptr;
   unsigned int *d_users = nullptr;
-  unsigned int *d_idle = nullptr;  // kIdleCopies copies of the idle count, kIdleStride apart
   unsigned long long *d_has_work = nullptr;
   unsigned long long *d_ctr = nullptr;  // see Ctr
+  unsigned long long *d_work = nullptr; // see kWorkWords
   unsigned long long *d_hist = nullptr;
   unsigned long long *d_root_nodes = nullptr;
   unsigned long long *d_root_cycles = nullptr;
@@ -446,8 +446,16 @@ struct mce_batch {
 };
 
 namespace {
-enum Ctr { kCount, kHash, kNodes, kNext, kListCursor, kNDeferred, kDeferNeed, kDeferStackNeed, kShared, kActive,
-           kIdle, kErr, kWords, kBuild, kPublished, kOwnerTasks, kNext2, kNext3, kNWide1, kNWide2, kPoolUsed, kNumCtr };
+// Words of d_ctr: the collected sums (Sum), then the others.
+enum Ctr { kCount = sCount, kHash = sHash, kNodes = sNodes, kWords = sWords, kBuild = sBuild, kShared = sShared,
+           kPublished = sPublished, kOwnerTasks = sOwner, kListCursor = kNumSums, kNDeferred, kDeferNeed,
+           kDeferStackNeed, kErr, kNWide1, kNWide2, kPoolUsed, kNumCtr };
+// Words of d_work, the per-run counters kept in copies: dispatch counters of
+// up to three launches, the work state, the sums and the clique sizes.
+constexpr uint64_t kNextWords = (uint64_t)kShards * kShardWords;
+constexpr uint64_t kStateAt = 3 * kNextWords, kSumsAt = kStateAt + (uint64_t)kStateShards * kShardWords,
+                   kHistAt = kSumsAt + (uint64_t)kShards * kShardWords,
+                   kWorkWords = kHistAt + (uint64_t)kShards * kLdsHist;
 
 template <class T>
 hipError_t dalloc(T **p, uint64_t count) {
@@ -470,7 +478,7 @@ void plan_release(mce_plan *p) {
                   p->d_root_nodes, p->d_root_cycles, p->d_list,     p->d_deferred,    p->d_deferred2,
                   p->d_slots2,   p->d_stacks,      p->d_stacks2,    p->d_recs,        p->d_users,
                   p->d_has_work, p->d_root_graph,  p->d_gcount,     p->d_ghash,       p->d_ghist,
-                  p->d_idle,     p->d_pk_stack,    p->d_pk_plist,   p->d_wide[0],     p->d_wide[1],
+                  p->d_work,     p->d_pk_stack,    p->d_pk_plist,   p->d_wide[0],     p->d_wide[1],
                   p->d_wide_h,   p->d_pool,        p->d_rfirst,     p->d_gstart};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
@@ -702,7 +710,7 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
   PTRY(dalloc(&p->d_recs, p->max_waves));
   PTRY(dalloc(&p->d_users, p->max_waves + 2));  // zeroed in whole 8-byte words
   PTRY(dalloc(&p->d_has_work, (p->max_waves + 63) / 64));
-  PTRY(dalloc(&p->d_idle, (uint64_t)kIdleCopies * kIdleStride));
+  PTRY(dalloc(&p->d_work, kWorkWords));
   set_config(p, wpc, opt.share_bound == 0 ? 24 : opt.share_bound, opt.lds_tier ? 1 : 0);
 
   PTRY(dalloc(&p->d_ctr, kNumCtr));
@@ -738,21 +746,14 @@ KArgs make_args(const mce_plan *p) {
   a.n_dispatch = p->n_dispatch;
   a.reverse = p->d_perm ? 0 : 1;
   a.root_mode = p->opt.root_mode;
-  a.count = p->d_ctr + kCount;
-  a.hash = p->d_ctr + kHash;
-  a.total_nodes = p->d_ctr + kNodes;
-  a.search_words = p->d_ctr + kWords;
-  a.build_bytes = p->d_ctr + kBuild;
-  a.next_root = p->d_ctr + kNext;
+  a.next_root = p->d_work;
+  a.state = p->d_work + kStateAt;
+  a.sums = p->d_work + kSumsAt;
+  a.hist_sh = p->d_work + kHistAt;
   a.list_cursor = p->d_ctr + kListCursor;
   a.n_deferred = p->d_ctr + kNDeferred;
   a.deferred_need = p->d_ctr + kDeferNeed;
   a.deferred_stack_need = p->d_ctr + kDeferStackNeed;
-  a.shared_tasks = p->d_ctr + kShared;
-  a.published_levels = p->d_ctr + kPublished;
-  a.owner_tasks = p->d_ctr + kOwnerTasks;
-  a.active = (unsigned int *)(p->d_ctr + kActive);
-  a.idle_hint = p->d_idle;
   a.err = (unsigned int *)(p->d_ctr + kErr);
   a.hist = p->d_hist;
   a.hist_len = p->hist_len;
@@ -827,28 +828,62 @@ uint32_t pack_waves(const mce_plan *p) {
   return (uint32_t)std::min<uint64_t>(p->pack_waves_alloc, std::max<uint64_t>(1, (uint64_t)p->cus * p->pack_wpc));
 }
 
-// Resets every counter, result and sharing word of a run with fill kernels
-// (graph-capturable) and launches the enumeration kernels: with the packed
+// Ranges zeroed before a run: counters and results ...
+void result_fills(const mce_plan *p, FillList &f) {
+  f.add(p->d_ctr, kNumCtr);
+  f.add(p->d_hist, p->hist_len);
+  if (p->d_gcount) f.add(p->d_gcount, p->n_graphs);
+  if (p->d_ghash) f.add(p->d_ghash, p->n_graphs);
+  if (p->d_ghist) f.add(p->d_ghist, p->n_graphs * p->g_hist_stride);
+}
+// ... and before each launch of the one-root-per-wave kernel: its sharing
+// words.
+void share_fills(const mce_plan *p, uint64_t waves, FillList &f) {
+  f.add(p->d_recs, sizeof(ShareRec) / 8 * waves);
+  f.add(p->d_users, (waves + 1) / 2);
+  f.add(p->d_has_work, (waves + 63) / 64);
+}
+
+hipError_t collect(const mce_plan *p, hipStream_t s) {
+  return launch_collect(p->d_work + kSumsAt, p->d_work + kHistAt, p->d_ctr, p->d_hist, p->hist_len, s);
+}
+
+// Whether a level can ever be exposed: |P| >= share_bound takes a root with
+// that many candidates (at most the largest out-degree), or an eager root.
+bool can_share(const mce_plan *p, const KArgs &a) {
+  return a.share_bound > 0 && ((uint64_t)a.share_bound <= p->max_out || a.eager);
+}
+// Waves of the one-root-per-wave kernel: those beyond the root count could
+// only take shared tasks.
+uint32_t mce_waves(const mce_plan *p, KArgs &a) {
+  if (can_share(p, a)) return p->waves;
+  a.share_bound = -1;
+  return (uint32_t)std::min<uint64_t>(p->waves, std::max<uint64_t>(a.n_dispatch, 1));
+}
+
+// Resets every counter, result and sharing word of a run with one fill kernel
+// (graph-capturable; one launch per buffer took 11 launches, 2 us each) and
+// launches the enumeration kernels: with the packed
 // search on, pack<1,1> over the dispatch list, pack<2,2> over the roots it
 // found too wide (derived from the vertex bitmaps pack<1,1> kept for them),
 // and the one-root-per-wave kernel over the rest (each
 // later launch reads its list length from the counter the earlier one
 // filled, so the sequence needs no host round trip).
-hipError_t enqueue_run(const mce_plan *p, const KArgs &a, hipStream_t s) {
-  hipError_t e = launch_fill_zero(p->d_ctr, kNumCtr, s);
-  if (e == hipSuccess) e = launch_fill_zero(p->d_hist, p->hist_len, s);
-  if (e == hipSuccess) e = launch_fill_zero(p->d_recs, sizeof(ShareRec) / 8 * p->waves, s);
-  if (e == hipSuccess) e = launch_fill_zero(p->d_users, (p->waves + 1) / 2, s);
-  if (e == hipSuccess) e = launch_fill_zero(p->d_has_work, (p->waves + 63) / 64, s);
-  if (e == hipSuccess) e = launch_fill_zero(p->d_idle, (uint64_t)kIdleCopies * kIdleStride / 2, s);
-  if (e == hipSuccess && p->d_root_nodes) e = launch_fill_zero(p->d_root_nodes, p->n_roots, s);
-  if (e == hipSuccess && p->d_root_cycles) e = launch_fill_zero(p->d_root_cycles, p->n_roots, s);
-  if (e == hipSuccess && p->d_gcount) e = launch_fill_zero(p->d_gcount, p->n_graphs, s);
-  if (e == hipSuccess && p->d_ghash) e = launch_fill_zero(p->d_ghash, p->n_graphs, s);
-  if (e == hipSuccess && p->d_ghist) e = launch_fill_zero(p->d_ghist, p->n_graphs * p->g_hist_stride, s);
+hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
+  KArgs a = a0;
+  FillList f;
+  result_fills(p, f);
+  share_fills(p, p->waves, f);
+  f.add(p->d_work, kWorkWords);
+  if (p->d_root_nodes) f.add(p->d_root_nodes, p->n_roots);
+  if (p->d_root_cycles) f.add(p->d_root_cycles, p->n_roots);
+  hipError_t e = launch_fill_zero(f, s);
   if (e != hipSuccess) return e;
-  if (!p->pack) return launch_mce(a, p->waves, (uint32_t)p->waves_per_cu, s);
-  const uint32_t pw = pack_waves(p);
+  if (!p->pack) {
+    e = launch_mce(a, mce_waves(p, a), (uint32_t)p->waves_per_cu, s);
+    return e == hipSuccess ? collect(p, s) : e;
+  }
+  const uint64_t units = a.pk_gstart ? a.pk_ngroups : a.n_dispatch;
   for (int v = 0; v < 2 && e == hipSuccess; ++v) {
     const uint32_t nw = v == 0 ? 1 : 2, nx = nw;
     KArgs b = a;
@@ -884,8 +919,11 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a, hipStream_t s) {
       b.perm = p->d_wide[0];
       b.reverse = 0;
       b.n_dispatch_dev = p->d_ctr + kNWide1;
-      b.next_root = p->d_ctr + kNext2;
+      b.next_root = p->d_work + kNextWords;
     }
+    // the first launch hands out `units` runs; the second one's list length is
+    // not known here
+    const uint32_t pw = v == 0 ? (uint32_t)std::min<uint64_t>(pack_waves(p), std::max<uint64_t>(units, 1)) : pack_waves(p);
     e = launch_pack(b, v, pw, (uint32_t)p->pack_wpc, s);
   }
   if (e != hipSuccess) return e;
@@ -894,8 +932,10 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a, hipStream_t s) {
   c.reverse = 0;
   c.eager = nullptr;
   c.n_dispatch_dev = p->d_ctr + kNWide2;
-  c.next_root = p->d_ctr + kNext3;
-  return launch_mce(c, p->waves, (uint32_t)p->waves_per_cu, s);
+  c.next_root = p->d_work + 2 * kNextWords;
+  if (!can_share(p, c)) c.share_bound = -1;
+  e = launch_mce(c, p->waves, (uint32_t)p->waves_per_cu, s);
+  return e == hipSuccess ? collect(p, s) : e;
 }
 
 struct RunOut {
@@ -913,13 +953,9 @@ mce_status run_core(mce_plan *p, const KArgs &a0, bool allow_graph, RunOut &ro) 
   ro.passes = 0;
   ro.kernel_ms = 0;
   if (a.n_dispatch == 0) {
-    HIP_TRY(launch_fill_zero(p->d_ctr, kNumCtr, s));
-    HIP_TRY(launch_fill_zero(p->d_hist, p->hist_len, s));
-    if (p->d_gcount) {
-      HIP_TRY(launch_fill_zero(p->d_gcount, p->n_graphs, s));
-      HIP_TRY(launch_fill_zero(p->d_ghash, p->n_graphs, s));
-      HIP_TRY(launch_fill_zero(p->d_ghist, p->n_graphs * p->g_hist_stride, s));
-    }
+    FillList f;
+    result_fills(p, f);
+    HIP_TRY(launch_fill_zero(f, s));
     HIP_TRY(hipStreamSynchronize(s));
     std::memset(ro.ctr, 0, sizeof(ro.ctr));
     return MCE_OK;
@@ -982,13 +1018,11 @@ mce_status run_core(mce_plan *p, const KArgs &a0, bool allow_graph, RunOut &ro) 
     }
     if (!p->d_deferred2) HIP_TRY(dalloc(&p->d_deferred2, p->deferred_cap));
     HIP_TRY(hipMemcpyAsync(p->d_deferred2, p->d_deferred, nd * 8, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(launch_fill_zero(p->d_ctr + kNext, 1, s));
-    HIP_TRY(launch_fill_zero(p->d_ctr + kNDeferred, 3, s));
-    HIP_TRY(launch_fill_zero(p->d_ctr + kActive, 2, s));
-    HIP_TRY(launch_fill_zero(p->d_recs, sizeof(ShareRec) / 8 * waves2, s));
-    HIP_TRY(launch_fill_zero(p->d_users, (waves2 + 1) / 2, s));
-    HIP_TRY(launch_fill_zero(p->d_has_work, (waves2 + 63) / 64, s));
-    HIP_TRY(launch_fill_zero(p->d_idle, (uint64_t)kIdleCopies * kIdleStride / 2, s));
+    FillList f;
+    f.add(p->d_ctr + kNDeferred, 3);
+    f.add(p->d_work, kSumsAt);
+    share_fills(p, waves2, f);
+    HIP_TRY(launch_fill_zero(f, s));
     KArgs b = a;
     b.perm = p->d_deferred2;
     b.eager = nullptr;
@@ -1001,6 +1035,7 @@ mce_status run_core(mce_plan *p, const KArgs &a0, bool allow_graph, RunOut &ro) 
     b.n_waves = (uint32_t)waves2;
     HIP_TRY(hipEventRecord(p->ev[2], s));
     HIP_TRY(launch_mce(b, (uint32_t)waves2, (uint32_t)p->waves_per_cu, s));
+    HIP_TRY(collect(p, s));
     HIP_TRY(hipEventRecord(p->ev[3], s));
     HIP_TRY(hipEventSynchronize(p->ev[3]));
     HIP_TRY(hipEventElapsedTime(&ms, p->ev[2], p->ev[3]));

@@ -121,23 +121,18 @@ __device__ __forceinline__ void or64(uint64_t *p, uint64_t v) {
   __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Per-wave accumulators (lane 0 flushes them at exit).  `words` counts the
-// 64-bit bitmap words the search reads; `build` the bytes the subproblem
-// build moves (both adjacency lists, the candidate list, the bitmap).
+// Per-wave accumulators (flushed at exit).  `words` counts the 64-bit bitmap
+// words the search reads; `build` the bytes the subproblem build moves (both
+// adjacency lists, the candidate list, the bitmap).
 struct Acc {
   unsigned long long count;
   unsigned long long hash;
   unsigned long long words;
   unsigned long long build;
   unsigned long long scan;  // per lane: adjacency entries of the bitmap rows' runs
+  unsigned long long nodes;
+  uint32_t shared, published, owner;  // sharing: see Sum
 };
-
-// Sum over the wave of a per-lane 64-bit value (uniform result).
-__device__ __forceinline__ uint64_t wave_sum64(uint64_t v) {
-  uint64_t s = 0;
-  for (uint32_t k = 0; k < 64; ++k) s += readlane64(v, k);
-  return s;
-}
 
 __device__ __forceinline__ unsigned int ld_relaxed(unsigned int *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -154,8 +149,32 @@ __device__ __forceinline__ void nap(uint32_t n) {
 }
 __device__ __forceinline__ uint32_t bcast32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 __device__ __forceinline__ uint64_t bcast64(uint64_t v) {
-  return ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) |
-         __builtin_amdgcn_readfirstlane((uint32_t)v);
+  return ((uint64_t)bcast32((uint32_t)(v >> 32)) << 32) | bcast32((uint32_t)v);  // (the builtin's result is signed)
+}
+
+// Number of dispatch entries, as a uniform value (a loaded one would make
+// every branch on it divergent).
+__device__ __forceinline__ uint64_t dispatch_count(const KArgs &a) {
+  return a.n_dispatch_dev ? bcast64(ld_relaxed((unsigned long long *)a.n_dispatch_dev)) : a.n_dispatch;
+}
+
+// Takes the next dispatch entry of counter `sh` (this wave's own to begin
+// with).  kHop: that one has run out, `sh` now names the nearest one that has
+// not, ask again; kNone: all have run out.  With n_dispatch entries, counter
+// k holds entries k, k + kShards, ...
+enum Claim { kNone, kGot, kHop };
+__device__ __forceinline__ Claim next_entry(const KArgs &a, uint64_t n_dispatch, uint32_t &sh, uint64_t &entry) {
+  const uint32_t l = lane();
+  unsigned long long i = 0;
+  if (l == 0) i = atomicAdd(&a.next_root[(uint64_t)sh * kShardWords], 1ull);
+  entry = bcast64(i) * kShards + sh;
+  if (entry < n_dispatch) return kGot;
+  // lane k looks at counter k; the first with entries left after sh
+  const uint64_t at = ld_relaxed(&a.next_root[(uint64_t)l * kShardWords]) * kShards + l;
+  const uint64_t m = __ballot(at < n_dispatch);
+  const uint64_t rot = (m >> sh) | (sh ? m << (64 - sh) : 0);
+  sh = (sh + (m ? (uint32_t)__builtin_ctzll(rot) : 0u)) & (kShards - 1);
+  return m ? kHop : kNone;
 }
 
 // LDS pointers (address space 3): the LDS tiers and the per-wave clique-size
@@ -176,6 +195,14 @@ __device__ __forceinline__ uint32_t wave_scan_add_u32(uint32_t v) {
   t = __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xC, 0xF, false); v += t;
   return v;
 }
+// Sum over the wave of a per-lane 64-bit value (uniform result): three
+// 22-bit pieces, whose sums over 64 lanes fit 28 bits.
+__device__ __forceinline__ uint64_t wave_sum64(uint64_t v) {
+  const uint32_t a = __builtin_amdgcn_readlane(wave_scan_add_u32((uint32_t)v & 0x3FFFFF), 63);
+  const uint32_t b = __builtin_amdgcn_readlane(wave_scan_add_u32((uint32_t)(v >> 22) & 0x3FFFFF), 63);
+  const uint32_t c = __builtin_amdgcn_readlane(wave_scan_add_u32((uint32_t)(v >> 44)), 63);
+  return (uint64_t)a + ((uint64_t)b << 22) + ((uint64_t)c << 44);
+}
 __device__ __forceinline__ uint32_t wave_scan_max_u32(uint32_t v) {
   uint32_t t;
   t = __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xF, 0xF, false); v = v > t ? v : t;
@@ -186,6 +213,26 @@ __device__ __forceinline__ uint32_t wave_scan_max_u32(uint32_t v) {
   t = __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xC, 0xF, false); v = v > t ? v : t;
   return v;
 }
+// Adds this wave's sums and its clique-size histogram to its copies of the
+// results: lane k adds Sum word k and the sizes k.
+__device__ __forceinline__ void flush_sums(const KArgs &a, uint32_t me, const Acc &acc, const ldsu64 *s_hist) {
+  const uint32_t l = lane(), sh = me % kShards;
+  const uint64_t cnt = bcast64(acc.count), hsh = bcast64(acc.hash);  // kept by lane 0
+  uint64_t v = 0;
+  v = l == sCount ? cnt : v;
+  v = l == sHash ? hsh : v;
+  v = l == sNodes ? acc.nodes : v;
+  v = l == sWords ? acc.words : v;
+  v = l == sBuild ? acc.build : v;
+  v = l == sShared ? (uint64_t)acc.shared : v;
+  v = l == sPublished ? (uint64_t)acc.published : v;
+  v = l == sOwner ? (uint64_t)acc.owner : v;
+  if (v) atomicAdd(&a.sums[(uint64_t)sh * kShardWords + l], (unsigned long long)v);
+  const unsigned long long h = s_hist[l];
+  if (h) atomicAdd(&a.hist_sh[(uint64_t)sh * kLdsHist + l], h);
+}
+static_assert(kLdsHist == 64, "one clique size per lane");
+
 // Relaxed 64-bit OR into an LDS word.
 __device__ __forceinline__ void or64_lds(lds64 *p, uint64_t v) {
   __hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);

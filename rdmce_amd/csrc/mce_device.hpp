@@ -10,8 +10,15 @@ constexpr uint32_t kMaxP = 4096;
 constexpr uint32_t kMaxW = kMaxP / 64;
 // Per-wave LDS histogram of clique sizes below this bound.
 constexpr uint32_t kLdsHist = 64;
-constexpr uint32_t kIdleCopies = 64;  // copies of the idle count, one per 128-byte line
-constexpr uint32_t kIdleStride = 32;  // u32 between copies
+// Counters that every wave touches are kept in kShards copies, one per
+// 128-byte line (kShardWords words); wave w uses copy w % kShards.  Atomics on
+// one address take 12 ns each however many waves issue them (4,096 waves: 53
+// us per increment), on 64 lines 0.25 ns.
+constexpr uint32_t kShards = 64;
+constexpr uint32_t kShardWords = 16;
+// Copies of the work state (see KArgs::state): few, so that a poll for idle
+// waves is one load of 16 lines; 256 waves a copy change state in 3 us.
+constexpr uint32_t kStateShards = 16;
 constexpr uint32_t kPollSteps = 128;  // descents (tree nodes) between polls for idle waves (a power of two)
 
 // Error flags raised by the kernels (bit mask in KArgs::err).
@@ -20,6 +27,14 @@ constexpr uint32_t kErrHistOverflow = 2u;    // clique larger than hist_len - 1
 constexpr uint32_t kErrDeferFull = 4u;       // deferred-root list full
 constexpr uint32_t kErrListFull = 8u;        // clique list capacity exceeded
 constexpr uint32_t kErrPackStack = 16u;      // packed search: record stack full
+
+// Words of a copy of KArgs::sums.
+enum Sum { sCount, sHash, sNodes, sWords, sBuild, sShared, sPublished, sOwner, kNumSums };
+// sWords: bitmap words read by the search; sBuild: bytes moved building
+// subproblems; sShared: tasks taken by a wave other than the publisher;
+// sPublished: levels exposed; sOwner: tasks of exposed levels run by their
+// publisher.
+static_assert(kNumSums <= kShardWords, "one line per copy");
 
 // One root's subproblem, as every wavefront working on it sees it.  The
 // pointers are HBM copies (the owner may work on an LDS copy of bm and gP).
@@ -62,20 +77,21 @@ struct KArgs {
   uint64_t n_dispatch;
   int32_t reverse;
   int32_t root_mode;            // 1 vertex, 2 edge
-  // Results.
-  unsigned long long *count;
-  unsigned long long *hash;
+  // Results.  Waves add their sums to their copy of `sums` (kShards copies of
+  // the Sum words) and of the clique sizes below kLdsHist (`hist_sh`, kShards x
+  // kLdsHist); launch_collect adds the copies up.  Larger sizes go straight
+  // to hist.
+  unsigned long long *sums;
+  unsigned long long *hist_sh;
   unsigned long long *hist;     // hist_len entries
   uint32_t hist_len;
-  unsigned long long *total_nodes;
-  unsigned long long *search_words;  // bitmap words read by the search
-  unsigned long long *build_bytes;   // bytes moved building subproblems
   unsigned long long *root_nodes;   // per canonical root, nullable
   unsigned long long *root_cycles;  // per canonical root, nullable
   uint32_t *list;                   // nullable
   unsigned long long *list_cursor;
   uint64_t list_cap;
-  // Work distribution.
+  // Work distribution: kShards counters, kShardWords apart; counter k hands
+  // out dispatch entries k, k + kShards, k + 2 kShards, ...
   unsigned long long *next_root;
   // Per-wave HBM scratch: data (candidate lists + bitmap) and DFS stack.
   uint8_t *slots;
@@ -86,11 +102,8 @@ struct KArgs {
   ShareRec *recs;                   // one per wave
   unsigned int *users;              // per wave: other waves reading its data region
   unsigned long long *has_work;     // bit per wave: record has unclaimed tasks
-  unsigned int *active;             // waves running a root or a task
-  unsigned int *idle_hint;          // kIdleCopies copies (kIdleStride apart) of the number of waves looking for work
-  unsigned long long *shared_tasks; // tasks taken by a wave other than the publisher
-  unsigned long long *published_levels;  // levels exposed
-  unsigned long long *owner_tasks;       // tasks of exposed levels run by their publisher
+  unsigned long long *state;        // kStateShards copies (kShardWords apart) of: waves running a root or a task
+                                    // (low 32 bits), waves looking for work (high 32 bits)
   int32_t share_bound;              // |P| threshold for exposing a level; <= 0: off
   uint32_t n_waves;
   // LDS tier: subproblems whose bitmap, label hashes and stack fit in
@@ -180,5 +193,23 @@ hipError_t launch_copy_probe(const void *src, void *dst, uint64_t bytes, hipStre
 // Zero-fills n 64-bit words with a kernel (safe inside captured hipGraphs,
 // unlike memset nodes).
 hipError_t launch_fill_zero(void *p, uint64_t n_words, hipStream_t stream);
+// The same for several ranges in one launch.
+constexpr uint32_t kMaxFill = 16;
+struct FillList {
+  uint64_t *p[kMaxFill];
+  uint64_t end[kMaxFill];  // running total of words up to and including range i
+  uint32_t n = 0;
+  void add(void *ptr, uint64_t words) {
+    if (!words) return;
+    p[n] = (uint64_t *)ptr;
+    end[n] = (n ? end[n - 1] : 0) + words;
+    ++n;
+  }
+};
+hipError_t launch_fill_zero(const FillList &f, hipStream_t stream);
+// out[Sum] += the copies of `sums`, hist[k] += the copies of hist_sh (k <
+// min(hist_len, kLdsHist)); the copies are left zeroed for the next pass.
+hipError_t launch_collect(unsigned long long *sums, unsigned long long *hist_sh, unsigned long long *out,
+                          unsigned long long *hist, uint32_t hist_len, hipStream_t stream);
 
 }  // namespace rdmce

@@ -263,15 +263,37 @@ __device__ __forceinline__ void publish_bit(const KArgs &a, uint32_t w, bool set
   else atomicAnd(&a.has_work[w >> 6], ~(1ull << (w & 63)));
 }
 
-// The number of waves looking for work is kept in kIdleCopies copies, one
-// per 128-byte line: a wave changing state updates every copy (one vector
-// atomic, lane i on copy i), and a searching wave polls only copy me % 64,
-// so the polls of thousands of waves do not queue on one address.
-__device__ __forceinline__ void idle_add(const KArgs &a, int d) {
-  atomicAdd(&a.idle_hint[lane() * kIdleStride], (unsigned int)d);
+// The numbers of working and of looking waves are kept in kStateShards
+// copies: a wave changing state updates its own copy (one atomic; updating
+// every one of 64 copies at each change cost an empty launch of 4,096 waves
+// 174 us, this 12 us), and a poll reads all of them (lane i copy i).
+constexpr unsigned long long kWorking = 1ull, kLooking = 1ull << 32;
+__device__ __forceinline__ void state_add(const KArgs &a, uint32_t me, unsigned long long d) {
+  if (lane() == 0) atomicAdd(&a.state[(uint64_t)(me % kStateShards) * kShardWords], d);
 }
-__device__ __forceinline__ bool any_idle(const KArgs &a, uint32_t me) {
-  return ld_relaxed(&a.idle_hint[(me % kIdleCopies) * kIdleStride]) != 0;
+// A poll reads this wave's own copy first: a few thousand waves polling all
+// copies would saturate the lines they share with the updates.
+__device__ __forceinline__ bool state_any(const KArgs &a, uint32_t me, bool looking) {
+  const uint32_t l = lane(), own = me % kStateShards;
+  unsigned long long v = 0;
+  if (l == own) v = ld_relaxed(&a.state[(uint64_t)l * kShardWords]);
+  bool any = __ballot((looking ? v >> 32 : v & 0xFFFFFFFFull) != 0) != 0;
+  if (!any) {
+    if (l < kStateShards) v = ld_relaxed(&a.state[(uint64_t)l * kShardWords]);
+    any = __ballot((looking ? v >> 32 : v & 0xFFFFFFFFull) != 0) != 0;
+  }
+  return any;
+}
+__device__ __forceinline__ bool any_idle(const KArgs &a, uint32_t me) { return state_any(a, me, true); }
+__device__ __forceinline__ bool any_working(const KArgs &a, uint32_t me) { return state_any(a, me, false); }
+// Whether to expose a level now: at once for an eager root's top level,
+// otherwise when some wave looks for work; never while an earlier
+// publication's takers still read its levels.
+__device__ __forceinline__ bool may_expose(const KArgs &a, uint32_t me, ShareRec *my, bool at_once) {
+  if (!at_once && !any_idle(a, me)) return false;
+  bool go = false;
+  if (lane() == 0) go = ld_relaxed(&my->pending) == 0;
+  return bcast32(go);
 }
 
 // Evaluates node L (the record at `rec`): a leaf is emitted; otherwise the
@@ -383,7 +405,7 @@ __device__ __forceinline__ uint64_t run_dfs(const KArgs &a, const Sub &s, BmP bm
           return nodes;
         }
         if (bcast32(last) && l == 0) publish_bit(a, me, false);
-        if (l == 0) atomicAdd(a.owner_tasks, 1ull);
+        ++acc.owner;
         level = S + 1;
         L = materialize(s, stk + (uint64_t)S * LS, (uint32_t)idx, stk + (uint64_t)level * LS, bm, gP, acc);
         if (l == 0) __hip_atomic_fetch_sub(&my->pending, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
@@ -401,9 +423,7 @@ __device__ __forceinline__ uint64_t run_dfs(const KArgs &a, const Sub &s, BmP bm
     // once; otherwise exposure waits for idle waves, polled every kPollSteps
     // descents - a poll is a round trip past this XCD's L2).
     if (S < Lstar && S + 1 < level && ((eager_top && S < 0) || ((++tick & (kPollSteps - 1)) == 0))) {
-      bool go = false;
-      if (l == 0) go = ((eager_top && S < 0) || any_idle(a, me)) && ld_relaxed(&my->pending) == 0;
-      if (bcast32(go)) {
+      if (may_expose(a, me, my, eager_top && S < 0)) {
         const uint32_t lp = (uint32_t)(S + 1);
         StP src = stk + (uint64_t)lp * LS;
         uint32_t n = set_popc(wl ? (uint64_t)src[3 * W + l] : 0ull, W);
@@ -432,8 +452,8 @@ __device__ __forceinline__ uint64_t run_dfs(const KArgs &a, const Sub &s, BmP bm
             __hip_atomic_store(&my->ctl, ((unsigned long long)ep << 32) | ((unsigned long long)n << 16),
                                __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
             publish_bit(a, me, true);
-            atomicAdd(a.published_levels, 1ull);
           }
+          ++acc.published;
           published = true;
         }
         S = (int)lp;
@@ -774,7 +794,7 @@ __device__ __forceinline__ uint64_t run_dfsr(const KArgs &a, const Sub &s, const
           return nodes;
         }
         if (bcast32(last) && l == 0) publish_bit(a, me, false);
-        if (l == 0) atomicAdd(a.owner_tasks, 1ull);
+        ++acc.owner;
         // candidate idx of the frozen V, with P and XP as sequential DFS
         // holds them when it reaches it (as materialize does)
         wave_fence();
@@ -813,9 +833,7 @@ __device__ __forceinline__ uint64_t run_dfsr(const KArgs &a, const Sub &s, const
     if (!task) {
       // Exposure: the shallowest level above this one that is not frozen.
       if (S < Lstar && S + 1 < level && ((eager_top && S < 0) || ((++tick & (kPollSteps - 1)) == 0))) {
-        bool go = false;
-        if (l == 0) go = ((eager_top && S < 0) || any_idle(a, me)) && ld_relaxed(&my->pending) == 0;
-        if (bcast32(go)) {
+        if (may_expose(a, me, my, eager_top && S < 0)) {
           const uint32_t lp = (uint32_t)(S + 1);
           const uint64_t *src = stk + (uint64_t)lp * LS;
           wave_fence();  // lane 0 wrote the record
@@ -846,8 +864,8 @@ __device__ __forceinline__ uint64_t run_dfsr(const KArgs &a, const Sub &s, const
               __hip_atomic_store(&my->ctl, ((unsigned long long)ep << 32) | ((unsigned long long)n << 16),
                                  __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
               publish_bit(a, me, true);
-              atomicAdd(a.published_levels, 1ull);
             }
+            ++acc.published;
             published = true;
           }
           S = (int)lp;
@@ -875,7 +893,9 @@ __device__ __forceinline__ uint64_t run_dfsr(const KArgs &a, const Sub &s, const
   }
 }
 
-__device__ void defer_root(const KArgs &a, uint64_t canon, uint64_t data_need, uint64_t stack_need) {
+// (Always inlined, as everything here that takes KArgs: a call would put the
+// arguments in scratch memory and make all values read from them divergent.)
+__device__ __forceinline__ void defer_root(const KArgs &a, uint64_t canon, uint64_t data_need, uint64_t stack_need) {
   if (lane() == 0) {
     unsigned long long pos = atomicAdd(a.n_deferred, 1ull);
     if (pos < a.deferred_cap) a.deferred[pos] = canon;
@@ -1155,8 +1175,7 @@ __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk
   if (idx < 0) return false;
   if (l == 0 && last) publish_bit(a, (uint32_t)victim, false);
   if (is_idle) {  // looking for work -> working
-    idle_add(a, -1);
-    if (l == 0) atomicAdd(a.active, 1u);
+    state_add(a, me, kWorking - kLooking);
     is_idle = false;
   }
   Sub s = r->sub;
@@ -1193,10 +1212,10 @@ __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk
   if (l == 0) {
     if (a.root_nodes && nodes) atomicAdd(&a.root_nodes[s.canon], (unsigned long long)nodes);
     if (a.root_cycles) atomicAdd(&a.root_cycles[s.canon], (unsigned long long)(clock64() - t0));
-    atomicAdd(a.total_nodes, (unsigned long long)nodes);
-    atomicAdd(a.shared_tasks, 1ull);
     __hip_atomic_fetch_sub(&a.users[s.bm_owner], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   }
+  acc.nodes += nodes;
+  ++acc.shared;
   return true;
 }
 
@@ -1206,25 +1225,29 @@ __device__ __forceinline__ void mce_main(const KArgs &a) {
   ldsu64 *s_hist = (ldsu64 *)lds_dyn;
   lds64 *lds = (lds64 *)lds_dyn + kLdsHist;
   const uint32_t l = lane();
+  const uint64_t n_dispatch = dispatch_count(a);
+  if (n_dispatch == 0) return;  // no root, so nothing is ever published either
   for (uint32_t i = l; i < kLdsHist; i += 64) s_hist[i] = 0;
   __syncthreads();
   const uint32_t me = blockIdx.x;
   uint8_t *slot = a.slots + (uint64_t)me * a.slot_bytes;
   uint64_t *stk = (uint64_t *)(a.stacks + (uint64_t)me * a.stack_bytes);
-  Acc acc{0, 0, 0, 0, 0};
-  unsigned long long nodes_total = 0;
-  // A wave is working (counted in `active`) until it finds neither a root
-  // nor a task; it is then looking for work (counted in the idle copies)
-  // until it gets either.  Only these transitions touch the shared
-  // counters, not every root.  The run ends for a wave that is looking for
-  // work when no roots are left and no wave is working: only working waves
-  // publish tasks, and a thief becomes working before the publisher it
-  // took from can finish.
-  const uint64_t n_dispatch = a.n_dispatch_dev ? ld_relaxed((unsigned long long *)a.n_dispatch_dev) : a.n_dispatch;
+  Acc acc{};
+  // A wave is working until it finds neither a root nor a task; it is then
+  // looking for work until it gets either.  Only these transitions touch the
+  // shared state, not every root.  The run ends for a wave that is looking
+  // for work when no roots are left and no wave is working: only working
+  // waves publish tasks, and a thief becomes working before the publisher it
+  // took from can finish.  (The copies of the state are not read in one
+  // instant, so a wave may see no worker while a task passes from one copy's
+  // wave to another's and end early; its part of the remaining tasks then
+  // falls to the others - a publisher runs every task nobody takes.)
   bool roots_left = true, is_idle = false;
   bool published = false;  // others may be reading this wave's data region
   uint32_t backoff = 1;
-  if (l == 0) atomicAdd(a.active, 1u);
+  uint32_t shard = me % kShards;
+  const bool sharing = a.share_bound > 0;
+  if (sharing) state_add(a, me, kWorking);
   for (;;) {
     bool did = false;
     if (roots_left) {
@@ -1238,20 +1261,19 @@ __device__ __forceinline__ void mce_main(const KArgs &a) {
         }
       }
       if (free_slot) {
-        unsigned long long i = 0;
-        if (l == 0) i = atomicAdd(a.next_root, 1ull);
-        i = bcast64(i);
-        if (i < n_dispatch) {
+        uint64_t i = 0;
+        const Claim claim = next_entry(a, n_dispatch, shard, i);
+        if (claim == kHop) continue;
+        if (claim == kGot) {
           if (is_idle) {
-            idle_add(a, -1);
-            if (l == 0) atomicAdd(a.active, 1u);
+            state_add(a, me, kWorking - kLooking);
             is_idle = false;
           }
           uint64_t canon = a.perm ? a.perm[i] : (a.reverse ? n_dispatch - 1 - i : i);
           uint64_t t0 = clock64();
           const bool eager = a.eager && a.eager[i];
           uint64_t nodes = solve_root(a, slot, stk, lds, me, canon, acc, s_hist, published, eager);
-          nodes_total += nodes;
+          acc.nodes += nodes;
           if (a.root_graph) flush_graph(a, a.root_graph[canon], acc, s_hist);
           if (l == 0) {
             if (a.root_nodes && nodes) atomicAdd(&a.root_nodes[canon], (unsigned long long)nodes);
@@ -1265,32 +1287,22 @@ __device__ __forceinline__ void mce_main(const KArgs &a) {
       }
     }
     if (did) continue;
-    if (!is_idle) {  // working -> looking for work
-      idle_add(a, 1);
-      if (l == 0) atomicSub(a.active, 1u);
+    if (!sharing) break;  // no root left, and nothing is ever published
+    if (!is_idle) {       // working -> looking for work
+      state_add(a, me, kLooking - kWorking);
       is_idle = true;
     }
-    if (a.share_bound > 0 && steal(a, me, stk, lds, acc, s_hist, is_idle)) {
+    if (steal(a, me, stk, lds, acc, s_hist, is_idle)) {
       backoff = 1;
       continue;
     }
-    bool done = false;
-    if (l == 0) done = !roots_left && ld_relaxed(a.active) == 0;
-    if (bcast32(done)) break;
+    if (!roots_left && !any_working(a, me)) break;
     if (l == 0) nap(backoff);
     backoff = backoff < 64 ? backoff * 2 : 64;
   }
   __syncthreads();
   acc.build += 4 * wave_sum64(acc.scan);
-  if (l == 0) {
-    if (acc.count) atomicAdd(a.count, acc.count);
-    if (acc.hash) atomicAdd(a.hash, acc.hash);
-    if (nodes_total) atomicAdd(a.total_nodes, nodes_total);
-    if (acc.words) atomicAdd(a.search_words, acc.words);
-    if (acc.build) atomicAdd(a.build_bytes, acc.build);
-  }
-  for (uint32_t i = l; i < kLdsHist && i < a.hist_len; i += 64)
-    if (s_hist[i]) atomicAdd(&a.hist[i], s_hist[i]);
+  flush_sums(a, me, acc, s_hist);
 }
 
 // One persistent kernel per occupancy target: the register budget that
@@ -1331,16 +1343,59 @@ __global__ __launch_bounds__(256) void copy_probe_kernel(const uint4 *__restrict
 }  // namespace
 
 namespace {
-__global__ __launch_bounds__(256) void fill_zero_kernel(uint64_t *p, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-    p[i] = 0;
+__global__ __launch_bounds__(256) void fill_zero_kernel(FillList f) {
+  const uint64_t n = f.end[f.n - 1];
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    // uniform scan of the ranges: the list sits in scalar registers
+    uint64_t *p = f.p[0] + i;
+    for (uint32_t k = 1; k < kMaxFill; ++k)
+      if (k < f.n && i >= f.end[k - 1]) p = f.p[k] + (i - f.end[k - 1]);
+    *p = 0;
+  }
+}
+
+// One block: thread t < kLdsHist sums clique size t over the copies, the next
+// kNumSums threads one Sum word each; kShards independent loads per thread.
+__global__ __launch_bounds__(kLdsHist + 64) void collect_kernel(unsigned long long *sums, unsigned long long *hist_sh,
+                                                                unsigned long long *out, unsigned long long *hist,
+                                                                uint32_t hist_len) {
+  const uint32_t t = threadIdx.x;
+  const bool h = t < kLdsHist;
+  const uint32_t k = h ? t : t - kLdsHist;
+  if (!h && k >= (uint32_t)kNumSums) return;
+  unsigned long long *src = h ? hist_sh + k : sums + k;
+  const uint32_t stride = h ? kLdsHist : kShardWords;
+  unsigned long long s = 0;
+#pragma unroll 16
+  for (uint32_t i = 0; i < kShards; ++i) {
+    s += src[(uint64_t)i * stride];
+    src[(uint64_t)i * stride] = 0;
+  }
+  if (h) {
+    if (k < hist_len) hist[k] += s;
+  } else {
+    out[k] += s;
+  }
 }
 }  // namespace
 
+hipError_t launch_fill_zero(const FillList &f, hipStream_t stream) {
+  if (f.n == 0) return hipSuccess;
+  const uint64_t n = f.end[f.n - 1];
+  uint32_t blocks = (uint32_t)std::min<uint64_t>(2048, (n + 255) / 256);
+  hipLaunchKernelGGL(fill_zero_kernel, dim3(blocks), dim3(256), 0, stream, f);
+  return hipGetLastError();
+}
+
 hipError_t launch_fill_zero(void *p, uint64_t n_words, hipStream_t stream) {
-  if (n_words == 0) return hipSuccess;
-  uint32_t blocks = (uint32_t)std::min<uint64_t>(2048, (n_words + 255) / 256);
-  hipLaunchKernelGGL(fill_zero_kernel, dim3(blocks), dim3(256), 0, stream, (uint64_t *)p, n_words);
+  FillList f;
+  f.add(p, n_words);
+  return launch_fill_zero(f, stream);
+}
+
+hipError_t launch_collect(unsigned long long *sums, unsigned long long *hist_sh, unsigned long long *out,
+                          unsigned long long *hist, uint32_t hist_len, hipStream_t stream) {
+  hipLaunchKernelGGL(collect_kernel, dim3(1), dim3(kLdsHist + 64), 0, stream, sums, hist_sh, out, hist, hist_len);
   return hipGetLastError();
 }
 

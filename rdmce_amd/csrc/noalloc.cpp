@@ -29,9 +29,11 @@ constexpr uint32_t kWavesPerCu = 4;     // few waves, large per-wave regions
 constexpr uint32_t kDeferCap = 1024;
 constexpr uint32_t kScanThreads = 1024;
 
-// Counters in the array (u64 each).
-enum Ctr { cCount, cHash, cNodes, cNext, cList, cNDeferred, cDeferNeed, cDeferStackNeed, cShared, cActive, cErr,
-           cWords, cBuild, cPublished, cOwner, cNum };
+// Counters in the array (u64 each): the collected sums (Sum), the others,
+// then those kept in copies (dispatch, work state, sums, clique sizes).
+enum Ctr { cCount = sCount, cHash = sHash, cNodes = sNodes, cList = kNumSums, cNDeferred, cDeferNeed, cDeferStackNeed,
+           cErr, cNext = 32, cState = cNext + kShards * kShardWords, cSums = cState + kStateShards * kShardWords,
+           cHistSh = cSums + kShards * kShardWords, cNum = cHistSh + kShards * kLdsHist };
 
 std::mutex g_mu;
 uint8_t *g_scratch[kMaxDevices] = {};
@@ -160,8 +162,7 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
   const uint64_t o_ctr = take(8ull * cNum), o_hist = take(8ull * hist_len), o_outoff = take(8 * (n + 1)),
                  o_rfirst = take(8 * (n + 1)), o_roots = take(8 * std::max<uint64_t>(m, 1)),
                  o_defer = take(8ull * kDeferCap), o_recs = take(sizeof(ShareRec) * (uint64_t)waves),
-                 o_users = take(8ull * ((waves + 2) / 2)), o_work = take(8ull * ((waves + 63) / 64)),
-                 o_idle = take(4ull * kIdleCopies * kIdleStride);
+                 o_users = take(8ull * ((waves + 2) / 2)), o_work = take(8ull * ((waves + 63) / 64));
   if (off >= kScratchBytes) return fail(MCE_ERR_UNSUPPORTED, "graph too large for the no-alloc scratch array");
   const uint64_t per_wave = (kScratchBytes - off) / waves / 512 * 256;  // data region and stack, each
   if (per_wave < 4096)
@@ -176,13 +177,14 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
   unsigned long long *hist = (unsigned long long *)(base + o_hist);
   uint64_t *outoff = (uint64_t *)(base + o_outoff), *rfirst = (uint64_t *)(base + o_rfirst);
   uint64_t *roots = (uint64_t *)(base + o_roots);
-  // Resets with fill kernels (no memset nodes if the caller captures this).
-  hipError_t e = launch_fill_zero(ctr, cNum, s);
-  if (e == hipSuccess) e = launch_fill_zero(hist, hist_len, s);
-  if (e == hipSuccess) e = launch_fill_zero(base + o_recs, sizeof(ShareRec) / 8 * (uint64_t)waves, s);
-  if (e == hipSuccess) e = launch_fill_zero(base + o_users, (waves + 2) / 2, s);
-  if (e == hipSuccess) e = launch_fill_zero(base + o_work, (waves + 63) / 64, s);
-  if (e == hipSuccess) e = launch_fill_zero(base + o_idle, (uint64_t)kIdleCopies * kIdleStride / 2, s);
+  // Resets with a fill kernel (no memset nodes if the caller captures this).
+  FillList f;
+  f.add(ctr, cNum);
+  f.add(hist, hist_len);
+  f.add(base + o_recs, sizeof(ShareRec) / 8 * (uint64_t)waves);
+  f.add(base + o_users, (waves + 2) / 2);
+  f.add(base + o_work, (waves + 63) / 64);
+  hipError_t e = launch_fill_zero(f, s);
   if (e != hipSuccess) return fail(MCE_ERR_DEVICE, std::string("reset: ") + hipGetErrorString(e));
   if (m) {
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(4096, (n + 255) / 256);
@@ -203,20 +205,14 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
     a.n_dispatch = m;
     a.reverse = 1;  // high core first, BkPivotBitBalance.cuh:429-431
     a.root_mode = MCE_ROOT_EDGE;
-    a.count = ctr + cCount;
-    a.hash = ctr + cHash;
-    a.total_nodes = ctr + cNodes;
-    a.search_words = ctr + cWords;
-    a.build_bytes = ctr + cBuild;
     a.next_root = ctr + cNext;
+    a.state = ctr + cState;
+    a.sums = ctr + cSums;
+    a.hist_sh = ctr + cHistSh;
     a.list_cursor = ctr + cList;
     a.n_deferred = ctr + cNDeferred;
     a.deferred_need = ctr + cDeferNeed;
     a.deferred_stack_need = ctr + cDeferStackNeed;
-    a.shared_tasks = ctr + cShared;
-    a.published_levels = ctr + cPublished;
-    a.owner_tasks = ctr + cOwner;
-    a.active = (unsigned int *)(ctr + cActive);
     a.err = (unsigned int *)(ctr + cErr);
     a.hist = hist;
     a.hist_len = hist_len;
@@ -227,7 +223,6 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
     a.recs = (ShareRec *)(base + o_recs);
     a.users = (unsigned int *)(base + o_users);
     a.has_work = (unsigned long long *)(base + o_work);
-    a.idle_hint = (unsigned int *)(base + o_idle);
     a.share_bound = 24;
     a.n_waves = waves;
     a.lds_tier = 1;
@@ -239,6 +234,7 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
     a.deferred = (uint64_t *)(base + o_defer);
     a.deferred_cap = kDeferCap;
     e = launch_mce(a, waves, kWavesPerCu, s);
+    if (e == hipSuccess) e = launch_collect(a.sums, a.hist_sh, ctr, hist, hist_len, s);
     if (e != hipSuccess) return fail(MCE_ERR_DEVICE, std::string("enumeration: ") + hipGetErrorString(e));
   }
   hipLaunchKernelGGL(copy_out_kernel, dim3(1), dim3(256), 0, s, (const unsigned long long *)ctr,

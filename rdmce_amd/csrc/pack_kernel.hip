@@ -585,10 +585,11 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
   w.L.meta = w.L.map + 32;
   w.L.bhist = w.L.meta + kPackMetaWords * S;
   w.L.slots = w.L.bhist + (a.root_graph ? C::HS * S : 0);
+  const uint64_t n_dispatch = dispatch_count(a);
+  if (n_dispatch == 0) return;
   for (uint32_t i = l; i < kLdsHist; i += 64) w.L.hist[i] = 0;
   wave_fence();
-
-  const uint64_t n_dispatch = a.n_dispatch_dev ? ld_relaxed((unsigned long long *)a.n_dispatch_dev) : a.n_dispatch;
+  uint32_t shard = w.me % kShards;
   uint8_t *scratch = a.slots + (uint64_t)w.me * a.slot_bytes;
   // The wave's record stack, field-major: field f of record r is
   // stk[f * cap + r], so lanes touching neighbouring records touch
@@ -598,7 +599,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
   constexpr bool lists = LISTS;  // clique lists: R is kept in the records
   auto fld = [stk, cap](uint32_t f, uint32_t r) -> uint64_t & { return stk[(uint64_t)f * cap + r]; };
   ldsu32 *map32 = (ldsu32 *)w.L.map;
-  Acc acc{0, 0, 0, 0, 0};
+  Acc acc{};
   uint64_t cnt = 0, hsh = 0, words = 0, nodes = 0;  // per lane
   uint32_t top = 0;                                  // records in the stack
   uint64_t pending = 0;                              // candidates (tasks) in the stack
@@ -647,10 +648,10 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
           }
           nwide = 0;
         }
-        unsigned long long gi = 0;
-        if (l == 0) gi = atomicAdd(a.next_root, 1ull);
-        gi = bcast64(gi);
-        if (a.pk_gstart ? gi >= a.pk_ngroups : gi >= n_dispatch) {
+        uint64_t gi = 0;
+        const Claim claim = next_entry(a, a.pk_gstart ? a.pk_ngroups : n_dispatch, shard, gi);
+        if (claim == kHop) continue;
+        if (claim == kNone) {
           roots_left = false;
           break;
         }
@@ -1046,18 +1047,13 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
   }
 
   // Exit: the wave's sums.
-  const uint64_t wc = wave_sum64(cnt), wh = wave_sum64(hsh), ww = wave_sum64(words), wn = wave_sum64(nodes);
+  acc.count = wave_sum64(cnt);
+  acc.hash = wave_sum64(hsh);
+  acc.words = wave_sum64(words);
+  acc.nodes = wave_sum64(nodes);
   acc.build += 4 * wave_sum64(acc.scan);
-  if (l == 0) {
-    if (wc) atomicAdd(a.count, (unsigned long long)wc);
-    if (wh) atomicAdd(a.hash, (unsigned long long)wh);
-    if (wn) atomicAdd(a.total_nodes, (unsigned long long)wn);
-    if (ww) atomicAdd(a.search_words, (unsigned long long)ww);
-    if (acc.build) atomicAdd(a.build_bytes, acc.build);
-  }
   wave_fence();
-  for (uint32_t i = l; i < kLdsHist && i < a.hist_len; i += 64)
-    if (w.L.hist[i]) atomicAdd(&a.hist[i], (unsigned long long)w.L.hist[i]);
+  flush_sums(a, w.me, acc, w.L.hist);
 }
 
 // One kernel per variant and occupancy target (WPE waves per SIMD: the
