@@ -373,7 +373,7 @@ struct mce_plan {
   uint32_t waves = 0;
   uint32_t max_waves = 0;
   uint32_t lds_bytes = 0;
-  uint32_t lds_per_cu = 160u << 10;
+  uint32_t lds_per_cu = kCuLds;
   uint32_t lds_per_block_max = 64u << 10;
   int share_bound = 24;
   int lds_tier = 1;
@@ -572,7 +572,7 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
   hipDeviceProp_t prop;
   PTRY(hipGetDeviceProperties(&prop, opt.device));
   p->cus = prop.multiProcessorCount;
-  if (prop.sharedMemPerMultiprocessor) p->lds_per_cu = (uint32_t)prop.sharedMemPerMultiprocessor;
+  p->lds_per_cu = lds_of_cu(prop.sharedMemPerMultiprocessor);
   if (prop.sharedMemPerBlock) p->lds_per_block_max = (uint32_t)prop.sharedMemPerBlock - 1024;
   PTRY(hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking));
   for (auto &e : p->ev) PTRY(hipEventCreate(&e));

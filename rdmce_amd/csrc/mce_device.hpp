@@ -21,6 +21,15 @@ constexpr uint32_t kShardWords = 16;
 constexpr uint32_t kStateShards = 16;
 constexpr uint32_t kPollSteps = 128;  // descents (tree nodes) between polls for idle waves (a power of two)
 
+// LDS of a compute unit.  Some HIP runtimes report the whole device's LDS (40
+// MB: 256 CUs x 160 KB) in hipDeviceProp_t::sharedMemPerMultiprocessor - the
+// one that PyTorch's wheel brings, so every process that imports torch; taken
+// as one CU's, a wave asked for all of a CU's LDS and had the CU to itself.
+constexpr uint32_t kCuLds = 160u << 10;
+inline uint32_t lds_of_cu(uint64_t reported) {
+  return reported && reported < kCuLds ? (uint32_t)reported : kCuLds;
+}
+
 // Error flags raised by the kernels (bit mask in KArgs::err).
 constexpr uint32_t kErrPTooLarge = 1u;       // a root has |P| > kMaxP
 constexpr uint32_t kErrHistOverflow = 2u;    // clique larger than hist_len - 1

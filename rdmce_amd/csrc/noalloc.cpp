@@ -142,7 +142,7 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
       if (e != hipSuccess) return fail(MCE_ERR_DEVICE, std::string("hipGetDeviceProperties: ") + hipGetErrorString(e));
       g_scratch[device] = (uint8_t *)p;
       g_cus[device] = (uint32_t)prop.multiProcessorCount;
-      g_lds_cu[device] = (uint32_t)prop.sharedMemPerMultiprocessor;
+      g_lds_cu[device] = lds_of_cu(prop.sharedMemPerMultiprocessor);
       g_lds_block[device] = (uint32_t)prop.sharedMemPerBlock;
     }
     base = g_scratch[device];
@@ -226,7 +226,7 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
     a.share_bound = 24;
     a.n_waves = waves;
     a.lds_tier = 1;
-    uint64_t lds = (uint64_t)(lds_cu ? lds_cu : (160u << 10)) / kWavesPerCu;
+    uint64_t lds = (uint64_t)lds_cu / kWavesPerCu;
     lds = lds > 1024 ? lds - 1024 : 0;
     lds = std::min<uint64_t>(lds, (lds_block ? lds_block : (64u << 10)) - 2048);
     a.lds_bytes = (uint32_t)(lds / 256 * 256);
