@@ -426,6 +426,8 @@ struct mce_plan {
   uint64_t *d_pk_stack = nullptr;
   uint32_t *d_pk_plist = nullptr;
   uint64_t *d_wide[2] = {nullptr, nullptr};
+  uint64_t *d_mail = nullptr;       // packed search: per-wave mail (work handed to idle waves)
+  unsigned long long *d_pk_idle = nullptr;
   uint64_t *d_wide_h = nullptr;     // per entry of the first list: its kept vertex bitmap in d_pool
   uint64_t *d_pool = nullptr;
   uint64_t pool_words = 0;
@@ -450,10 +452,11 @@ namespace {
 enum Ctr { kCount = sCount, kHash = sHash, kNodes = sNodes, kWords = sWords, kBuild = sBuild, kShared = sShared,
            kPublished = sPublished, kOwnerTasks = sOwner, kListCursor = kNumSums, kNDeferred, kDeferNeed,
            kDeferStackNeed, kErr, kNWide1, kNWide2, kPoolUsed, kNumCtr };
-// Words of d_work, the per-run counters kept in copies: dispatch counters of
-// up to three launches, the work state, the sums and the clique sizes.
+// Words of d_work, the per-run counters kept in copies: dispatch counters and
+// work state of up to three launches, the sums and the clique sizes.
 constexpr uint64_t kNextWords = (uint64_t)kShards * kShardWords;
-constexpr uint64_t kStateAt = 3 * kNextWords, kSumsAt = kStateAt + (uint64_t)kStateShards * kShardWords,
+constexpr uint64_t kStateWords = (uint64_t)kStateShards * kShardWords;
+constexpr uint64_t kStateAt = 3 * kNextWords, kSumsAt = kStateAt + 3 * kStateWords,
                    kHistAt = kSumsAt + (uint64_t)kShards * kShardWords,
                    kWorkWords = kHistAt + (uint64_t)kShards * kLdsHist;
 
@@ -479,7 +482,7 @@ void plan_release(mce_plan *p) {
                   p->d_slots2,   p->d_stacks,      p->d_stacks2,    p->d_recs,        p->d_users,
                   p->d_has_work, p->d_root_graph,  p->d_gcount,     p->d_ghash,       p->d_ghist,
                   p->d_work,     p->d_pk_stack,    p->d_pk_plist,   p->d_wide[0],     p->d_wide[1],
-                  p->d_wide_h,   p->d_pool,        p->d_rfirst,     p->d_gstart};
+                  p->d_wide_h,   p->d_mail,    p->d_pk_idle,  p->d_pool,        p->d_rfirst,     p->d_gstart};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   for (auto &e : p->ev)
@@ -810,6 +813,8 @@ mce_status ensure_pack(mce_plan *p) {
     HIP_TRY(dalloc(&p->d_wide[0], p->wide_cap));
     HIP_TRY(dalloc(&p->d_wide[1], p->wide_cap));
     HIP_TRY(dalloc(&p->d_wide_h, p->wide_cap));
+    HIP_TRY(dalloc(&p->d_mail, (uint64_t)kPackMailWords * waves));
+    HIP_TRY(dalloc(&p->d_pk_idle, (waves + 63) / 64));
     // Kept vertex bitmaps: at most one per vertex with two or more edge
     // roots, within a quarter of the free device memory.
     size_t free_b = 0, total_b = 0;
@@ -877,6 +882,7 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
   f.add(p->d_work, kWorkWords);
   if (p->d_root_nodes) f.add(p->d_root_nodes, p->n_roots);
   if (p->d_root_cycles) f.add(p->d_root_cycles, p->n_roots);
+  if (p->pack) f.add(p->d_pk_idle, (p->pack_waves_alloc + 63) / 64);
   hipError_t e = launch_fill_zero(f, s);
   if (e != hipSuccess) return e;
   if (!p->pack) {
@@ -884,6 +890,7 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
     return e == hipSuccess ? collect(p, s) : e;
   }
   const uint64_t units = a.pk_gstart ? a.pk_ngroups : a.n_dispatch;
+  const bool share = can_share(p, a);
   for (int v = 0; v < 2 && e == hipSuccess; ++v) {
     const uint32_t nw = v == 0 ? 1 : 2, nx = nw;
     KArgs b = a;
@@ -921,9 +928,15 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
       b.n_dispatch_dev = p->d_ctr + kNWide1;
       b.next_root = p->d_work + kNextWords;
     }
-    // the first launch hands out `units` runs; the second one's list length is
-    // not known here
-    const uint32_t pw = v == 0 ? (uint32_t)std::min<uint64_t>(pack_waves(p), std::max<uint64_t>(units, 1)) : pack_waves(p);
+    // Without sharing, waves beyond the runs the first launch hands out have
+    // nothing to do (the second one's list length is not known here).
+    uint32_t pw = pack_waves(p);
+    if (v == 0 && !share) pw = (uint32_t)std::min<uint64_t>(pw, std::max<uint64_t>(units, 1));
+    b.state = p->d_work + kStateAt + v * kStateWords;
+    b.pk_share = share;
+    b.pk_nwaves = pw;
+    b.pk_idle = p->d_pk_idle;
+    b.pk_mail = p->d_mail;
     e = launch_pack(b, v, pw, (uint32_t)p->pack_wpc, s);
   }
   if (e != hipSuccess) return e;
@@ -933,6 +946,7 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
   c.eager = nullptr;
   c.n_dispatch_dev = p->d_ctr + kNWide2;
   c.next_root = p->d_work + 2 * kNextWords;
+  c.state = p->d_work + kStateAt + 2 * kStateWords;
   if (!can_share(p, c)) c.share_bound = -1;
   e = launch_mce(c, p->waves, (uint32_t)p->waves_per_cu, s);
   return e == hipSuccess ? collect(p, s) : e;

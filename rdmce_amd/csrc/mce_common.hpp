@@ -11,10 +11,48 @@ namespace {
 
 __device__ __forceinline__ uint32_t lane() { return __lane_id(); }
 
+// lane(), as a value the compiler knows nothing about: what is computed from
+// it stays where it is instead of being moved out of the caller's loop into
+// registers that live through it (rarely run parts of a persistent kernel).
+__device__ __forceinline__ uint32_t cold_lane() {
+  uint32_t l = __lane_id();
+#ifdef __AMDGCN__
+  asm volatile("" : "+v"(l));
+#endif
+  return l;
+}
+
+// The kernel's arguments, read from the argument segment where they are used
+// (every kernel here takes one KArgs): the same for uniform values, which
+// otherwise fill the scalar registers for the whole kernel.
+__device__ __forceinline__ const KArgs &cold_args(const KArgs &a) {
+#ifdef __AMDGCN__
+  auto p = (const __attribute__((address_space(4))) KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const KArgs *)p;
+#else
+  return a;
+#endif
+}
+
 __device__ __forceinline__ uint64_t readlane64(uint64_t v, uint32_t l) {
   uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, l);
   uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), l);
   return ((uint64_t)hi << 32) | lo;
+}
+
+// A value that is the same in every lane, as the compiler can see (lane 0's).
+// Loads through plain pointers, atomics' results and what loops over them
+// leave behind count as divergent otherwise: held in vector registers, and
+// every branch on them runs as exec-mask arithmetic.
+__device__ __forceinline__ uint32_t bcast32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint64_t bcast64(uint64_t v) {
+  return ((uint64_t)bcast32((uint32_t)(v >> 32)) << 32) | bcast32((uint32_t)v);  // (the builtin's result is signed)
+}
+
+template <class T>
+__device__ __forceinline__ T *bcastp(T *p) {
+  return (T *)bcast64((uint64_t)p);
 }
 
 // Wave-wide reductions with DPP (row_shr 1/2/4/8 inside each 16-lane row,
@@ -147,11 +185,6 @@ __device__ __forceinline__ unsigned int ld_acquire(unsigned int *p) {
 __device__ __forceinline__ void nap(uint32_t n) {
   for (uint32_t i = 0; i < n; ++i) __builtin_amdgcn_s_sleep(4);
 }
-__device__ __forceinline__ uint32_t bcast32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ uint64_t bcast64(uint64_t v) {
-  return ((uint64_t)bcast32((uint32_t)(v >> 32)) << 32) | bcast32((uint32_t)v);  // (the builtin's result is signed)
-}
-
 // Number of dispatch entries, as a uniform value (a loaded one would make
 // every branch on it divergent).
 __device__ __forceinline__ uint64_t dispatch_count(const KArgs &a) {
@@ -182,6 +215,60 @@ __device__ __forceinline__ Claim next_entry(const KArgs &a, uint64_t n_dispatch,
 using lds64 = __attribute__((address_space(3))) uint64_t;
 using ldsu64 = __attribute__((address_space(3))) unsigned long long;
 using ldsu32 = __attribute__((address_space(3))) uint32_t;
+
+// The numbers of working and of looking waves are kept in kStateShards
+// copies: a wave changing state updates its own copy (one atomic; updating
+// every one of 64 copies at each change cost an empty launch of 4,096 waves
+// 174 us, this 12 us), and a poll reads all of them (lane i copy i).
+constexpr unsigned long long kWorking = 1ull, kLooking = 1ull << 32;
+__device__ __forceinline__ void state_add(const KArgs &a, uint32_t me, unsigned long long d) {
+  if (lane() == 0) atomicAdd(&a.state[(uint64_t)(me % kStateShards) * kShardWords], d);
+}
+// A poll reads this wave's own copy first: a few thousand waves polling all
+// copies would saturate the lines they share with the updates.
+__device__ __forceinline__ bool state_any(const KArgs &a, uint32_t me, bool looking) {
+  const uint32_t l = lane(), own = me % kStateShards;
+  unsigned long long v = 0;
+  if (l == own) v = ld_relaxed(&a.state[(uint64_t)l * kShardWords]);
+  bool any = __ballot((looking ? v >> 32 : v & 0xFFFFFFFFull) != 0) != 0;
+  if (!any) {
+    if (l < kStateShards) v = ld_relaxed(&a.state[(uint64_t)l * kShardWords]);
+    any = __ballot((looking ? v >> 32 : v & 0xFFFFFFFFull) != 0) != 0;
+  }
+  return any;
+}
+__device__ __forceinline__ bool any_idle(const KArgs &a, uint32_t me) { return state_any(a, me, true); }
+__device__ __forceinline__ bool any_working(const KArgs &a, uint32_t me) { return state_any(a, me, false); }
+
+// A wave w != me (w < n_waves) whose bit is set in `bits`, or -1: one of this
+// wave's XCD (they share an L2) when there is one, and starting from different
+// places for different `me`, so that waves looking at the same time spread out.
+__device__ __forceinline__ int find_wave(unsigned long long *bits, uint32_t n_waves, uint32_t me) {
+  const uint32_t l = lane();
+  const uint32_t nwords = (n_waves + 63) / 64;
+  const uint64_t xcd = 0x0101010101010101ull << (me & 7);
+  int found = -1;
+  for (uint32_t base = 0; base < nwords && found < 0; base += 64) {
+    const uint32_t j = base + l;
+    uint64_t w = j < nwords ? ld_relaxed(&bits[j]) : 0;
+    if (j == (me >> 6)) w &= ~(1ull << (me & 63));
+    const uint64_t near = __ballot((w & xcd) != 0);
+    const uint64_t any = __ballot(w != 0);
+    const uint64_t pick = near ? near : any;
+    if (pick) {
+      const uint32_t start = (me >> 6) & 63;
+      const uint64_t rot = (pick >> start) | (start ? pick << (64 - start) : 0);
+      const uint32_t jl = ((uint32_t)__builtin_ctzll(rot) + start) & 63;
+      uint64_t word = readlane64(w, jl);
+      if (near) word &= xcd;
+      const uint32_t sb = (me + 1) & 63;
+      const uint64_t r2 = (word >> sb) | (sb ? word << (64 - sb) : 0);
+      const uint32_t bit = ((uint32_t)__builtin_ctzll(r2) + sb) & 63;
+      found = (int)((base + jl) * 64 + bit);
+    }
+  }
+  return found >= 0 && (uint32_t)found < n_waves ? found : -1;
+}
 
 // Inclusive prefix sum / maximum over the 64 lanes (DPP row_shr 1/2/4/8
 // inside each 16-lane row, then row_bcast 15/31 across rows).
@@ -249,7 +336,7 @@ __device__ __forceinline__ void or64_lds(lds64 *p, uint64_t v) {
 __device__ __forceinline__ uint32_t root_lists(const KArgs &a, uint64_t canon, uint32_t *Pl, uint64_t ccap, Sub &s,
                                                uint64_t &p, uint64_t &x, Acc &acc) {
   const uint32_t l = lane();
-  const uint64_t desc = a.roots[canon];
+  const uint64_t desc = bcast64(a.roots[canon]);
   const uint32_t *col = a.col;
   p = 0;
   x = 0;
@@ -258,14 +345,14 @@ __device__ __forceinline__ uint32_t root_lists(const KArgs &a, uint64_t canon, u
     s.v0 = (uint32_t)(desc >> 32);
     s.v1 = (uint32_t)desc;
     s.base_size = 2;
-    s.base_key = a.label_hash[s.v0] + a.label_hash[s.v1];
+    s.base_key = bcast64(a.label_hash[s.v0] + a.label_hash[s.v1]);
     above = s.v1;
-    const uint64_t b0 = a.rowoff[s.v0], e0 = a.rowoff[s.v0 + 1], o0 = a.outoff[s.v0];
-    const uint64_t b1 = a.rowoff[s.v1], e1 = a.rowoff[s.v1 + 1], o1 = a.outoff[s.v1];
+    const uint64_t b0 = bcast64(a.rowoff[s.v0]), e0 = bcast64(a.rowoff[s.v0 + 1]), o0 = bcast64(a.outoff[s.v0]);
+    const uint64_t b1 = bcast64(a.rowoff[s.v1]), e1 = bcast64(a.rowoff[s.v1 + 1]), o1 = bcast64(a.outoff[s.v1]);
     // P = N+(v1) & (N+(v0) above v1): iterate the shorter run, binary-search
     // the longer (BkPivotBitBalance.cuh:449-469 builds it from N(v0) & N(v1)).
     {
-      const uint64_t s0 = lower_bound(col, o0, e0, s.v1 + 1);
+      const uint64_t s0 = bcast64(lower_bound(col, o0, e0, s.v1 + 1));
       uint64_t ab = o1, ae = e1, bb = s0, be = e0;
       if (ae - ab > be - bb) {
         uint64_t t0 = ab, t1 = ae;
@@ -291,7 +378,7 @@ __device__ __forceinline__ uint32_t root_lists(const KArgs &a, uint64_t canon, u
     }
     // X = (N(v0) below v1) & N-(v1); with P empty only its emptiness matters.
     {
-      uint64_t ab = b0, ae = lower_bound(col, b0, e0, s.v1), bb = b1, be = o1;
+      uint64_t ab = b0, ae = bcast64(lower_bound(col, b0, e0, s.v1)), bb = b1, be = o1;
       if (ae - ab > be - bb) {
         uint64_t t0 = ab, t1 = ae;
         ab = bb;
@@ -319,9 +406,9 @@ __device__ __forceinline__ uint32_t root_lists(const KArgs &a, uint64_t canon, u
     s.v0 = (uint32_t)desc;
     s.v1 = 0;
     s.base_size = 1;
-    s.base_key = a.label_hash[s.v0];
+    s.base_key = bcast64(a.label_hash[s.v0]);
     above = s.v0;
-    const uint64_t b = a.rowoff[s.v0], e = a.rowoff[s.v0 + 1], o = a.outoff[s.v0];
+    const uint64_t b = bcast64(a.rowoff[s.v0]), e = bcast64(a.rowoff[s.v0 + 1]), o = bcast64(a.outoff[s.v0]);
     p = e - o;
     x = o - b;
     for (uint64_t i = l; i < p && i < ccap; i += 64) Pl[i] = col[o + i];

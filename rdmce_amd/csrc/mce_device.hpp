@@ -171,6 +171,14 @@ struct KArgs {
   // them across waves.
   uint64_t *heavy;
   unsigned long long *n_heavy;
+  // Packed search, sharing (pk_share != 0): a wave out of work sets its bit in
+  // pk_idle; a wave with work to spare clears it and writes into that wave's
+  // mail (kPackMailWords words) part of its run, or of its stack with the
+  // subproblem the records belong to.
+  int32_t pk_share;
+  uint32_t pk_nwaves;               // waves of this launch
+  unsigned long long *pk_idle;
+  uint64_t *pk_mail;
 };
 
 // Packed search variants: |P0| <= 64 NW and |X0'| <= 64 NX.
@@ -186,6 +194,13 @@ constexpr uint32_t pack_hist_words(uint32_t nw) { return 64 * nw + 3; }
 // Per-slot bookkeeping words (canon, key, p|xq, base|graph, v0|v1, nodes,
 // refs, count, hash).
 constexpr uint32_t kPackMetaWords = 9;
+// A wave's mail: header, bookkeeping and LDS words of one subproblem, the P0
+// ids (clique lists), up to 64 records.
+constexpr uint32_t kMailHdr = 16;
+constexpr uint32_t pack_mail_words(uint32_t nw, uint32_t nx) {
+  return kMailHdr + 16 + pack_slot_words(nw, nx) + kPackMaxP / 2 + 64 * pack_rec_words(nw, nx);
+}
+constexpr uint32_t kPackMailWords = pack_mail_words(2, 2);
 // LDS bytes of a wave of the packed search.
 constexpr uint64_t pack_lds_bytes(uint32_t nw, uint32_t nx, uint32_t slots, bool batch) {
   return 8ull * (kLdsHist + 32 + slots * (kPackMetaWords + pack_slot_words(nw, nx) + (batch ? pack_hist_words(nw) : 0)));

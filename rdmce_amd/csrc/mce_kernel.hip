@@ -263,29 +263,6 @@ __device__ __forceinline__ void publish_bit(const KArgs &a, uint32_t w, bool set
   else atomicAnd(&a.has_work[w >> 6], ~(1ull << (w & 63)));
 }
 
-// The numbers of working and of looking waves are kept in kStateShards
-// copies: a wave changing state updates its own copy (one atomic; updating
-// every one of 64 copies at each change cost an empty launch of 4,096 waves
-// 174 us, this 12 us), and a poll reads all of them (lane i copy i).
-constexpr unsigned long long kWorking = 1ull, kLooking = 1ull << 32;
-__device__ __forceinline__ void state_add(const KArgs &a, uint32_t me, unsigned long long d) {
-  if (lane() == 0) atomicAdd(&a.state[(uint64_t)(me % kStateShards) * kShardWords], d);
-}
-// A poll reads this wave's own copy first: a few thousand waves polling all
-// copies would saturate the lines they share with the updates.
-__device__ __forceinline__ bool state_any(const KArgs &a, uint32_t me, bool looking) {
-  const uint32_t l = lane(), own = me % kStateShards;
-  unsigned long long v = 0;
-  if (l == own) v = ld_relaxed(&a.state[(uint64_t)l * kShardWords]);
-  bool any = __ballot((looking ? v >> 32 : v & 0xFFFFFFFFull) != 0) != 0;
-  if (!any) {
-    if (l < kStateShards) v = ld_relaxed(&a.state[(uint64_t)l * kShardWords]);
-    any = __ballot((looking ? v >> 32 : v & 0xFFFFFFFFull) != 0) != 0;
-  }
-  return any;
-}
-__device__ __forceinline__ bool any_idle(const KArgs &a, uint32_t me) { return state_any(a, me, true); }
-__device__ __forceinline__ bool any_working(const KArgs &a, uint32_t me) { return state_any(a, me, false); }
 // Whether to expose a level now: at once for an eager root's top level,
 // otherwise when some wave looks for work; never while an earlier
 // publication's takers still read its levels.
@@ -1003,7 +980,7 @@ __device__ __forceinline__ uint64_t solve_root(const KArgs &a, uint8_t *slot, ui
   Sub s;
   s.canon = canon;
   s.bm_owner = me;
-  s.graph = a.root_graph ? a.root_graph[canon] : 0;
+  s.graph = a.root_graph ? bcast32(a.root_graph[canon]) : 0;
   uint64_t p = 0, x = 0;
   // every P vertex lies above `above`, every X vertex below it
   const uint32_t above = root_lists(a, canon, Pl, ccap, s, p, x, acc);
@@ -1138,35 +1115,36 @@ __device__ __forceinline__ uint64_t solve_root(const KArgs &a, uint8_t *slot, ui
                  eager);
 }
 
+// A subproblem read from another wave's record, its fields uniform.
+__device__ __forceinline__ Sub uniform_sub(const Sub &r) {
+  Sub s;
+  s.p = bcast32(r.p);
+  s.xq = bcast32(r.xq);
+  s.W = bcast32(r.W);
+  s.Wx = bcast32(r.Wx);
+  s.rows_pad = bcast32(r.rows_pad);
+  s.LS = bcast32(r.LS);
+  s.base_size = bcast32(r.base_size);
+  s.v0 = bcast32(r.v0);
+  s.v1 = bcast32(r.v1);
+  s.bm_owner = bcast32(r.bm_owner);
+  s.levels = bcast32(r.levels);
+  s.graph = bcast32(r.graph);
+  s.base_key = bcast64(r.base_key);
+  s.canon = bcast64(r.canon);
+  s.Plist = bcastp(r.Plist);
+  s.bm = bcastp(r.bm);
+  s.gP = bcastp(r.gP);
+  return s;
+}
+
 // Looks for a published task (preferring waves on this XCD, which share
 // this wave's L2) and runs it.  Returns true when a task was run.
 __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk_g, lds64 *lds, Acc &acc,
                       ldsu64 *s_hist, bool &is_idle) {
   const uint32_t l = lane();
-  const uint32_t nwords = (a.n_waves + 63) / 64;
-  const uint64_t xcd = 0x0101010101010101ull << (me & 7);
-  int victim = -1;
-  for (uint32_t base = 0; base < nwords && victim < 0; base += 64) {
-    uint32_t j = base + l;
-    uint64_t w = j < nwords ? ld_relaxed(&a.has_work[j]) : 0;
-    if (j == (me >> 6)) w &= ~(1ull << (me & 63));
-    uint64_t near = __ballot((w & xcd) != 0);
-    uint64_t any = __ballot(w != 0);
-    uint64_t pick = near ? near : any;
-    if (pick) {
-      // rotate so that thieves starting from different waves spread out
-      uint32_t start = (me >> 6) & 63;
-      uint64_t rot = (pick >> start) | (start ? pick << (64 - start) : 0);
-      uint32_t jl = ((uint32_t)__builtin_ctzll(rot) + start) & 63;
-      uint64_t word = readlane64(w, jl);
-      if (near) word &= xcd;
-      uint32_t sb = (me + 1) & 63;
-      uint64_t r2 = (word >> sb) | (sb ? word << (64 - sb) : 0);
-      uint32_t bit = ((uint32_t)__builtin_ctzll(r2) + sb) & 63;
-      victim = (int)((base + jl) * 64 + bit);
-    }
-  }
-  if (victim < 0 || (uint32_t)victim >= a.n_waves) return false;
+  const int victim = find_wave(a.has_work, a.n_waves, me);
+  if (victim < 0) return false;
   ShareRec *r = a.recs + victim;
   int idx = -1;
   bool last = false;
@@ -1178,8 +1156,8 @@ __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk
     state_add(a, me, kWorking - kLooking);
     is_idle = false;
   }
-  Sub s = r->sub;
-  const uint64_t *snap = r->snap;
+  const Sub s = uniform_sub(r->sub);
+  const uint64_t *snap = bcastp(r->snap);
   if (l == 0) atomicAdd(&a.users[s.bm_owner], 1u);
   // Tiers as for a root: bitmap, label hashes and stack in LDS; or bitmap
   // and label hashes in LDS with the stack in HBM; or all in HBM.
@@ -1269,9 +1247,9 @@ __device__ __forceinline__ void mce_main(const KArgs &a) {
             state_add(a, me, kWorking - kLooking);
             is_idle = false;
           }
-          uint64_t canon = a.perm ? a.perm[i] : (a.reverse ? n_dispatch - 1 - i : i);
+          const uint64_t canon = bcast64(a.perm ? a.perm[i] : (a.reverse ? n_dispatch - 1 - i : i));
           uint64_t t0 = clock64();
-          const bool eager = a.eager && a.eager[i];
+          const bool eager = a.eager && bcast32(a.eager[i]);
           uint64_t nodes = solve_root(a, slot, stk, lds, me, canon, acc, s_hist, published, eager);
           acc.nodes += nodes;
           if (a.root_graph) flush_graph(a, a.root_graph[canon], acc, s_hist);

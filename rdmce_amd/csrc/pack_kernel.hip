@@ -39,6 +39,20 @@
 // copy (a.pk_whandle) instead of building it again.  A derived root with
 // too many X0' rows whose top node one of them prunes (it covers P0) is
 // settled there, as one tree node, and goes nowhere.
+//
+// Sharing: a wave that runs out of roots and records asks for work (its bit in
+// pk_idle); every kPackPoll passes a working wave looks for such waves and
+// mails one of them half of its run's unbuilt roots or, when its run has none
+// to spare, about half of its pending tasks - whole records from the bottom of
+// its stack (the shallowest, so the largest subtrees) with a copy of their
+// subproblem.  The records given away stay in the stack as empty ones.  This
+// is the reference's root-down exposure (BkPivotBitBalance.cuh:87-138) with
+// the giver doing the copying: a taker reads only its own mail, so a few
+// thousand waiting waves poll a few thousand lines.
+// What it measured: R-MAT 14, edge factor 14 (108M nodes, most below a few
+// roots), one-word launch 30.2 -> 6.0 ms, two-word launch 80 -> 16.2 ms; a
+// 200k-vertex community graph 23.7 -> 16.9 and 7.0 -> 6.3 ms.  It is off where
+// no root can reach the sharing bound (|P0| is at most the largest out-degree).
 #include "mce_common.hpp"
 
 extern __shared__ uint64_t lds_dyn[];
@@ -47,6 +61,11 @@ namespace rdmce {
 namespace {
 
 constexpr uint32_t kRecRoot = 1u << 24;  // meta flag: the record's one task is its root's top node
+// Passes between looks for idle waves (a power of two; a pass takes a few us,
+// a look one round trip past the L2), and pending tasks from which on a wave
+// gives some away (a gift costs the giver a few passes).
+constexpr uint32_t kPackPoll = 16;
+constexpr uint32_t kPackSpare = 16;
 
 template <int NW, int NX>
 struct PackCfg {
@@ -55,13 +74,20 @@ struct PackCfg {
   static constexpr uint32_t HS = pack_hist_words(NW);
   // record fields (each a column of pk_cap words in the wave's stack):
   // P XP V (NW each), XX (NX), key, meta, R (NW, read and written only for
-  // clique lists).  meta = first << 32 | root flag | slot << 16 | |R|, where
-  // the record's remaining candidates are the members of V from `first` on.
+  // clique lists).  meta = end << 40 | first << 32 | root flag | slot << 16 |
+  // |R|, where the record's remaining candidates are the members of V in
+  // [first, end).
   static constexpr uint32_t oP = 0, oX = NW, oV = 2 * NW, oXX = 3 * NW, oKey = 3 * NW + NX, oMeta = 3 * NW + NX + 1,
                             oR = 3 * NW + NX + 2;
   // slot word offsets
   static constexpr uint32_t sProw = 0, sXrow = 64 * NW * NW, sXcol = sXrow + 64 * NX * NW, sG = sXcol + 64 * NW * NX;
 };
+
+// Bits [64 q, 64 q + 64) of the range [first, end) that a record's meta names.
+__device__ __forceinline__ uint64_t range_word(uint64_t meta, uint32_t q) {
+  const uint32_t first = (uint32_t)(meta >> 32) & 0xFF, end = (uint32_t)(meta >> 40) & 0xFF, lo = 64u * q;
+  return low_mask(end > lo ? end - lo : 0u) & ~low_mask(first > lo ? first - lo : 0u);
+}
 
 // Position of the k-th (0-based) set bit of w; k < popcount(w).
 __device__ __forceinline__ uint32_t select64(uint64_t w, uint32_t k) {
@@ -154,8 +180,8 @@ __device__ __forceinline__ void pk_seal(const PackWave<NW, NX> &w, uint32_t s, u
                                         uint64_t base_key, uint32_t base_size, uint32_t graph, uint32_t v0,
                                         uint32_t v1) {
   using C = PackCfg<NW, NX>;
-  const KArgs &a = w.a;
-  const uint32_t l = lane();
+  const KArgs &a = cold_args(w.a);
+  const uint32_t l = cold_lane();
   lds64 *sl = w.slot(s);
   wave_fence();
   // Columns of the X0' block: bit x of column j is bit j of row x.  Lane l
@@ -228,11 +254,11 @@ template <int NW, int NX>
 __device__ __forceinline__ uint32_t pk_build(const PackWave<NW, NX> &w, uint8_t *scratch, uint32_t s, uint64_t canon,
                                              Acc &acc, uint64_t &cnt, uint64_t &hsh) {
   using C = PackCfg<NW, NX>;
-  const KArgs &a = w.a;
-  const uint32_t l = lane();
+  const KArgs &a = cold_args(w.a);
+  const uint32_t l = cold_lane();
   Sub sub;
   sub.canon = canon;
-  sub.graph = a.root_graph ? a.root_graph[canon] : 0;
+  sub.graph = a.root_graph ? bcast32(a.root_graph[canon]) : 0;
   uint32_t *Pl = (uint32_t *)scratch;
   const uint64_t ccap = a.slot_bytes / 4;
   uint64_t p = 0, x = 0;
@@ -308,10 +334,11 @@ struct PkGroup {
 // room for `run` wide root ids after it; `claim` is an LDS word for handing
 // out rows.  Returns false when it does not fit (the caller then builds each
 // edge root on its own).
-__device__ __forceinline__ bool pk_group_build(const KArgs &a, uint8_t *scratch, uint32_t v0, uint64_t run, PkGroup &G,
+__device__ __forceinline__ bool pk_group_build(const KArgs &a0, uint8_t *scratch, uint32_t v0, uint64_t run, PkGroup &G,
                                                Acc &acc, ldsu32 *claim) {
-  const uint32_t l = lane();
-  const uint64_t b0 = a.rowoff[v0], e0 = a.rowoff[(uint64_t)v0 + 1], o0 = a.outoff[v0];
+  const KArgs &a = cold_args(a0);
+  const uint32_t l = cold_lane();
+  const uint64_t b0 = bcast64(a.rowoff[v0]), e0 = bcast64(a.rowoff[(uint64_t)v0 + 1]), o0 = bcast64(a.outoff[v0]);
   const uint64_t d0 = e0 - o0, x0 = o0 - b0;
   const uint64_t W0 = (d0 + 63) / 64;
   if (W0 == 0 || W0 > kGroupMaxW) return false;
@@ -353,7 +380,7 @@ __device__ __forceinline__ bool pk_group_build(const KArgs &a, uint8_t *scratch,
   G.xq0 = (uint32_t)xq0;
   G.rp = (uint32_t)rp;
   G.o0 = o0;
-  G.rfirst = a.rfirst[v0];
+  G.rfirst = bcast64(a.rfirst[v0]);
   G.T = T;
   G.cm = cm;
   G.wide = (uint64_t *)(scratch + wide_off);
@@ -361,7 +388,7 @@ __device__ __forceinline__ bool pk_group_build(const KArgs &a, uint8_t *scratch,
   for (uint64_t j = l; j < d0; j += 64) lh[j] = a.label_hash[a.col[o0 + j]];
   wave_fence();
   G.lh = lh;
-  G.lh0 = a.label_hash[v0];
+  G.lh0 = bcast64(a.label_hash[v0]);
   return true;
 }
 
@@ -396,12 +423,12 @@ template <int NW, int NX>
 __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const PkGroup &G, uint32_t s, uint64_t canon,
                                               Acc &acc, uint64_t &cnt, uint64_t &hsh, uint32_t &pruned) {
   using C = PackCfg<NW, NX>;
-  const KArgs &a = w.a;
-  const uint32_t l = lane();
+  const KArgs &a = cold_args(w.a);
+  const uint32_t l = cold_lane();
   const uint32_t k = (uint32_t)(canon - G.rfirst);
-  const uint32_t uk = a.list ? a.col[G.o0 + k] : 0u;  // the root's v1 (clique lists only)
-  const uint32_t graph = a.root_graph ? a.root_graph[canon] : 0;
-  const uint64_t base_key = G.lh0 + G.lh[k];
+  const uint32_t uk = a.list ? bcast32(a.col[G.o0 + k]) : 0u;  // the root's v1 (clique lists only)
+  const uint32_t graph = a.root_graph ? bcast32(a.root_graph[canon]) : 0;
+  const uint64_t base_key = G.lh0 + bcast64(G.lh[k]);
   // Row k of U, split at k: P0 above it, the U part of X0 below it (one
   // word per lane).
   const uint32_t q = l;
@@ -613,9 +640,186 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
   bool grouped = false;
   uint32_t nwide = 0;  // wide roots of the current grouped run, in G.wide
   PkGroup G{};
+  bool new_run = false;  // [gcur, gend) has been taken and its vertex bitmap is to be built
+  // Sharing: this wave's mail and its parts.
+  const bool sharing = a.pk_share != 0;
+  uint32_t tick = 0, given = 0;  // records below `given` are empty (given away)
+  constexpr uint32_t oMeta0 = kMailHdr, oSlot = kMailHdr + 16, oIds = oSlot + C::SW, oRecs = oIds + kPackMaxP / 2;
+  uint64_t *mail = a.pk_mail + (uint64_t)w.me * kPackMailWords;
+  // Gives an idle wave, if there is one, part of this wave's work.
+  auto give = [&]() {
+    const KArgs &a = cold_args(w.a);
+    const uint32_t l = cold_lane();
+    const bool range = gend - gcur >= 2;
+    uint64_t dm = 0, sel_m = 0;
+    uint32_t ci = 0, s0 = 0, cands = 0, mid = 0;
+    bool split = false, take = false;
+    if (!range) {
+      if (pending < kPackSpare) return;
+      // lane l looks at record given + l
+      const uint32_t nl = top - given < 64 ? top - given : 64;
+      uint64_t rem[NW];
+#pragma unroll
+      for (int q = 0; q < NW; ++q) rem[q] = 0;
+      if (l < nl) {
+        dm = fld(C::oMeta, given + l);
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+          rem[q] = fld(C::oV + q, given + l) & range_word(dm, q);
+          ci += (uint32_t)__popcll(rem[q]);
+        }
+      }
+      const uint64_t nz = __ballot(ci != 0);
+      if (nz == 0) {
+        given += nl;
+        return;
+      }
+      const uint32_t f = (uint32_t)__builtin_ctzll(nz);
+      s0 = __builtin_amdgcn_readlane((uint32_t)(dm >> 16) & 0xFF, f);
+      const uint32_t c = ((uint32_t)(dm >> 16) & 0xFF) == s0 ? ci : 0u;
+      const uint32_t incl = wave_scan_add_u32(c);
+      const uint32_t half = (uint32_t)((pending + 1) / 2);
+      take = c != 0 && incl - c < half;
+      sel_m = __ballot(take);
+      uint32_t last = 63 - (uint32_t)__builtin_clzll(sel_m);
+      cands = __builtin_amdgcn_readlane(incl, last);
+      if (cands == pending) {
+        if (sel_m & (sel_m - 1)) {  // everything: keep the last one
+          sel_m &= ~(1ull << last);
+          take = take && l != last;
+          cands -= __builtin_amdgcn_readlane(c, last);
+        } else {  // one record holds all tasks: its upper half
+          split = true;
+          uint32_t kk = ci / 2, base = 0;
+#pragma unroll
+          for (int q = 0; q < NW - 1; ++q) {
+            const uint32_t cq = (uint32_t)__popcll(rem[q]);
+            if (base == (uint32_t)q * 64 && kk >= cq) {
+              kk -= cq;
+              base = (uint32_t)(q + 1) * 64;
+            }
+          }
+          uint64_t rw = rem[0];
+#pragma unroll
+          for (int q = 1; q < NW; ++q)
+            if (base == (uint32_t)q * 64) rw = rem[q];
+          mid = base + (take ? select64(rw, kk) : 0u);
+          cands -= cands / 2;
+        }
+      }
+    }
+    // claim an idle wave
+    const int to = find_wave(a.pk_idle, a.pk_nwaves, w.me);
+    if (to < 0) return;
+    const uint64_t tb = 1ull << (to & 63);
+    bool mine = false;
+    if (l == 0) mine = (atomicAnd(&a.pk_idle[to >> 6], (unsigned long long)~tb) & tb) != 0;
+    if (!bcast32(mine)) return;
+    uint64_t *out = a.pk_mail + (uint64_t)to * kPackMailWords;
+    uint64_t flag;
+    if (range) {  // the upper half of the run's unbuilt roots
+      const uint64_t at = gcur + (gend - gcur + 1) / 2;
+      if (l == 0) {
+        out[1] = at;
+        out[2] = gend;
+      }
+      gend = at;
+      flag = 2;
+    } else {
+      const lds64 *sl = w.slot(s0);
+      const uint32_t n = (uint32_t)__popcll(sel_m), rk = rank_below(sel_m);
+      for (uint32_t i = l; i < C::SW; i += 64) out[oSlot + i] = sl[i];
+      if (l < kPackMetaWords) {
+        uint64_t v = w.L.meta[l * S + s0];
+        v = l == mRefs ? (uint64_t)n : (l == mNodes || l == mCount || l == mHash ? 0ull : v);
+        out[oMeta0 + l] = v;
+      }
+      if (lists) {
+        const uint32_t *pl = a.pk_plist + ((uint64_t)w.me * S + s0) * kPackMaxP;
+        uint32_t *dst = (uint32_t *)(out + oIds);
+        for (uint32_t i = l; i < kPackMaxP; i += 64) dst[i] = pl[i];
+      }
+      if (take) {
+        for (uint32_t f = 0; f < (lists ? C::RS : C::RS - NW); ++f)
+          if (f != C::oMeta) out[oRecs + f * 64 + rk] = fld(f, given + l);
+        uint64_t tm = dm & ~(0xFFull << 16);  // the taker's slot 0
+        if (split) tm = (tm & ~(0xFFull << 32)) | ((uint64_t)mid << 32);
+        out[oRecs + C::oMeta * 64 + rk] = tm;
+        fld(C::oMeta, given + l) = split ? (dm & ~(0xFFull << 40)) | ((uint64_t)mid << 40) : dm & 0xFFFFFFFFull;
+      }
+      pending -= cands;
+      const uint64_t empty = __ballot(given + l < top && (ci == 0 || (take && !split)));
+      given += ~empty ? (uint32_t)__builtin_ctzll(~empty) : 64u;
+      flag = 1 | ((uint64_t)n << 8) | ((uint64_t)cands << 32);
+    }
+    state_add(a, (uint32_t)to, kWorking - kLooking);
+    wave_fence();
+    if (l == 0) __hip_atomic_store((unsigned long long *)out, (unsigned long long)flag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  // Waits for work from another wave; false when there is none to come.
+  auto wait_mail = [&]() -> bool {
+    const KArgs &a = cold_args(w.a);
+    const uint32_t l = cold_lane();
+    const uint64_t bit = 1ull << (w.me & 63);
+    if (l == 0) {
+      __hip_atomic_store((unsigned long long *)mail, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_fetch_or(&a.pk_idle[w.me >> 6], (unsigned long long)bit, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    state_add(a, w.me, kLooking - kWorking);
+    uint64_t flag = 0;
+    bool asked = true;
+    for (uint32_t n = 1, k = 0;; n = n < 8 ? n * 2 : 8, ++k) {
+      unsigned long long v = 0;
+      if (l == 0) v = ld_relaxed((unsigned long long *)mail);
+      flag = bcast64(v);
+      if (flag) break;
+      if (asked && (k & 3) == 0 && !any_working(a, w.me)) {
+        // withdraw; a wave that has cleared the bit already will send
+        bool had = false;
+        if (l == 0) had = (atomicAnd(&a.pk_idle[w.me >> 6], (unsigned long long)~bit) & bit) != 0;
+        if (bcast32(had)) return false;
+        asked = false;
+      }
+      if (l == 0) nap(n);
+    }
+    if (l == 0) {
+      unsigned long long v = __hip_atomic_load((unsigned long long *)mail, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+      (void)v;
+    }
+    wave_fence();
+    ++acc.shared;
+    if ((flag & 0xFF) == 2) {
+      gcur = bcast64(mail[1]);
+      gend = bcast64(mail[2]);
+      new_run = true;
+      return true;
+    }
+    const uint32_t n = (uint32_t)(flag >> 8) & 0xFF;
+    lds64 *sl = w.slot(0);
+    for (uint32_t i = l; i < C::SW; i += 64) sl[i] = mail[oSlot + i];
+    if (l < kPackMetaWords) w.L.meta[l * S] = mail[oMeta0 + l];
+    if (a.root_graph)
+      for (uint32_t i = l; i < C::HS; i += 64) w.L.bhist[i] = 0;
+    if (lists) {
+      uint32_t *pl = a.pk_plist + (uint64_t)w.me * S * kPackMaxP;
+      const uint32_t *src = (const uint32_t *)(mail + oIds);
+      for (uint32_t i = l; i < kPackMaxP; i += 64) pl[i] = src[i];
+    }
+    if (l < n)
+      for (uint32_t f = 0; f < (lists ? C::RS : C::RS - NW); ++f) fld(f, l) = mail[oRecs + f * 64 + l];
+    wave_fence();
+    top = n;
+    given = 0;
+    pending = flag >> 32;
+    busy = 1;
+    return true;
+  };
+  if (sharing) state_add(a, w.me, kWorking);
   for (;;) {
+    const KArgs &a = cold_args(w.a);
+    const uint32_t l = cold_lane();
     // Refill: build roots into free slots while fewer than 64 tasks wait.
-    while (roots_left && pending < 64 && busy != full) {
+    while ((roots_left || gcur != gend || nwide) && pending < 64 && busy != full) {
       if (gcur == gend) {
         if (nwide) {  // the finished run's wide roots go out with a copy of its vertex bitmap
           wave_fence();
@@ -648,6 +852,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
           }
           nwide = 0;
         }
+        if (!roots_left) break;
         uint64_t gi = 0;
         const Claim claim = next_entry(a, a.pk_gstart ? a.pk_ngroups : n_dispatch, shard, gi);
         if (claim == kHop) continue;
@@ -655,34 +860,39 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
           roots_left = false;
           break;
         }
-        gcur = a.pk_gstart ? a.pk_gstart[gi] : gi;
-        gend = a.pk_gstart ? a.pk_gstart[gi + 1] : gi + 1;
+        gcur = a.pk_gstart ? bcast64(a.pk_gstart[gi]) : gi;
+        gend = a.pk_gstart ? bcast64(a.pk_gstart[gi + 1]) : gi + 1;
+        new_run = true;
+      }
+      if (new_run) {
+        new_run = false;
         grouped = false;
         if (gend - gcur >= 2 && a.root_mode == 2) {
-          const uint64_t c0 = a.perm ? a.perm[gcur] : (a.reverse ? n_dispatch - 1 - gcur : gcur);
-          grouped = pk_group_build(a, scratch, (uint32_t)(a.roots[c0] >> 32), a.wide_h ? gend - gcur : 0, G, acc,
+          const uint64_t c0 = bcast64(a.perm ? a.perm[gcur] : (a.reverse ? n_dispatch - 1 - gcur : gcur));
+          grouped = pk_group_build(a, scratch, bcast32((uint32_t)(a.roots[c0] >> 32)), a.wide_h ? gend - gcur : 0, G, acc,
                                    map32);
         }
       }
       const uint64_t i = gcur++;
-      const uint64_t canon = a.perm ? a.perm[i] : (a.reverse ? n_dispatch - 1 - i : i);
-      if (a.eager && a.eager[i]) {  // split before launch: to the one-root-per-wave kernel
+      const uint64_t canon = bcast64(a.perm ? a.perm[i] : (a.reverse ? n_dispatch - 1 - i : i));
+      if (a.eager && bcast32(a.eager[i])) {  // split before launch: to the one-root-per-wave kernel
         if (l == 0) a.heavy[atomicAdd(a.n_heavy, 1ull)] = canon;
         continue;
       }
       const uint32_t s = (uint32_t)__builtin_ctzll((uint64_t)(~busy & full));
       bool derive = grouped;
-      const uint64_t hk = a.pk_whandle ? a.pk_whandle[i] : ~0ull;
+      const uint64_t hk = a.pk_whandle ? bcast64(a.pk_whandle[i]) : ~0ull;
       if (hk != ~0ull) {  // the vertex bitmap an earlier launch kept for this root
         const uint64_t *hdr = a.pk_pool + hk;
-        G.v0 = (uint32_t)hdr[0];
-        G.d0 = (uint32_t)hdr[1];
-        G.W0 = (uint32_t)hdr[2];
-        G.xq0 = (uint32_t)hdr[3];
-        G.rp = (uint32_t)hdr[4];
-        G.o0 = hdr[5];
-        G.rfirst = hdr[6];
-        G.lh0 = hdr[7];
+        const uint64_t hv = hdr[l & (kPoolHdr - 1)];
+        G.v0 = __builtin_amdgcn_readlane((uint32_t)hv, 0);
+        G.d0 = __builtin_amdgcn_readlane((uint32_t)hv, 1);
+        G.W0 = __builtin_amdgcn_readlane((uint32_t)hv, 2);
+        G.xq0 = __builtin_amdgcn_readlane((uint32_t)hv, 3);
+        G.rp = __builtin_amdgcn_readlane((uint32_t)hv, 4);
+        G.o0 = readlane64(hv, 5);
+        G.rfirst = readlane64(hv, 6);
+        G.lh0 = readlane64(hv, 7);
         G.T = hdr + kPoolHdr;
         G.cm = G.T + (uint64_t)G.W0 * G.rp;
         G.lh = G.cm + G.W0;
@@ -710,7 +920,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
         if (l == 0) {  // one task (V = {0}): the root's top node
           for (uint32_t f = 0; f < C::RS; ++f) fld(f, top) = 0;
           fld(C::oV, top) = 1;
-          fld(C::oMeta, top) = ((uint64_t)s << 16) | kRecRoot;
+          fld(C::oMeta, top) = (1ull << 40) | ((uint64_t)s << 16) | kRecRoot;
         }
         wave_fence();
         ++top;
@@ -718,7 +928,10 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
         busy |= 1u << s;
       }
     }
-    if (top == 0) break;  // no records and no roots left (see the refill condition)
+    if (__builtin_expect_with_probability(top == 0, 0, 0.999)) {  // no records and no roots left (see the refill condition)
+      if (!sharing || !wait_mail()) break;
+      continue;
+    }
 
     // Dispatch up to 64 tasks from the top of the stack: look-lane i sees
     // record top-1-i; task lane l takes candidate k of look-record ri.
@@ -730,12 +943,9 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     if (l < nlook) {
       const uint32_t r = top - 1 - l;
       lmeta = fld(C::oMeta, r);
-      const uint32_t first = (uint32_t)(lmeta >> 32);
 #pragma unroll
       for (int q = 0; q < NW; ++q) {
-        const uint32_t lo = 64u * q;
-        const uint64_t keep = first <= lo ? ~0ull : (first >= lo + 64 ? 0ull : ~0ull << (first - lo));
-        lrem[q] = fld(C::oV + q, r) & keep;
+        lrem[q] = fld(C::oV + q, r) & range_word(lmeta, q);
         ci += (uint32_t)__popcll(lrem[q]);
       }
     }
@@ -752,7 +962,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     const uint32_t nfull = (uint32_t)__popcll(__ballot(lfull));
     map32[l] = 0;
     wave_fence();
-    if (l < nlook && excl < T) map32[excl] = ((l + 1) << 8) | excl;
+    if (l < nlook && ci && excl < T) map32[excl] = ((l + 1) << 8) | excl;
     wave_fence();
     const uint32_t mv = wave_scan_max_u32(l < T ? map32[l] : 0u);
     const bool act = l < T;
@@ -768,7 +978,6 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     if (act) {
       const uint32_t r = top - 1 - ri;
       const uint64_t m64 = fld(C::oMeta, r);
-      const uint32_t first = (uint32_t)(m64 >> 32);
       uint64_t rem[NW];
 #pragma unroll
       for (int q = 0; q < NW; ++q) {
@@ -776,8 +985,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
         P[q] = fld(C::oP + q, r);
         XP[q] = fld(C::oX + q, r);
         V[q] = fld(C::oV + q, r);
-        const uint32_t lo = 64u * q;
-        rem[q] = V[q] & (first <= lo ? ~0ull : (first >= lo + 64 ? 0ull : ~0ull << (first - lo)));
+        rem[q] = V[q] & range_word(m64, q);
       }
 #pragma unroll
       for (int j = 0; j < NX; ++j) XX[j] = fld(C::oXX + j, r);
@@ -819,10 +1027,11 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
       for (int q = 1; q < NW; ++q)
         if (base == (uint32_t)q * 64) rw = lrem[q];
       const uint32_t first = base + select64(rw, kk);
-      fld(C::oMeta, top - 1 - l) = (lmeta & 0xFFFFFFFFull) | ((uint64_t)first << 32);
+      fld(C::oMeta, top - 1 - l) = (lmeta & ~(0xFFull << 32)) | ((uint64_t)first << 32);
     }
     if (lfull) __hip_atomic_fetch_sub(w.m(mRefs, lslot), (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     top -= nfull;
+    given = given < top ? given : top;
 
     // The task: one tree node per lane.
     const uint32_t s = (meta >> 16) & 0xFF;
@@ -1032,7 +1241,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
 #pragma unroll
       for (int j = 0; j < NX; ++j) fld(C::oXX + j, r) = XX[j];
       fld(C::oKey, r) = key;
-      fld(C::oMeta, r) = meta;  // first = 0: every candidate remains
+      fld(C::oMeta, r) = (uint64_t)meta | ((uint64_t)(64 * NW) << 40);  // every candidate remains
       __hip_atomic_fetch_add(w.m(mRefs, s), (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     const uint32_t vsum = __builtin_amdgcn_readlane(wave_scan_add_u32(vc), 63);
@@ -1044,6 +1253,9 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     const uint64_t dm = __ballot(done);
     if (done) pk_finish<NW, NX>(w, l);
     busy &= ~(uint32_t)dm;
+    if (sharing && __builtin_expect((++tick & (kPackPoll - 1)) == 0, 0) &&
+        __builtin_expect_with_probability(any_idle(a, w.me), 0, 0.999))
+      give();
   }
 
   // Exit: the wave's sums.
