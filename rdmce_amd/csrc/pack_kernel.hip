@@ -173,19 +173,15 @@ __device__ __forceinline__ void pk_emit(const PackWave<NW, NX> &w, uint32_t s, u
   }
 }
 
-// Completes slot s once its P0 rows, X0' rows, label hashes (and clique-list
-// ids) are in place: the columns of the X0' block and the bookkeeping.
+// The columns of slot s's X0' block from its rows (in place): bit x of column
+// j is bit j of row x.  Lane l holds row 64 b + l of block b; one ballot per
+// P0 vertex and block.
 template <int NW, int NX>
-__device__ __forceinline__ void pk_seal(const PackWave<NW, NX> &w, uint32_t s, uint64_t p, uint64_t xq, uint64_t canon,
-                                        uint64_t base_key, uint32_t base_size, uint32_t graph, uint32_t v0,
-                                        uint32_t v1) {
+__device__ __forceinline__ void pk_columns(const PackWave<NW, NX> &w, uint32_t s, uint32_t p, uint32_t xq) {
   using C = PackCfg<NW, NX>;
-  const KArgs &a = cold_args(w.a);
   const uint32_t l = cold_lane();
   lds64 *sl = w.slot(s);
   wave_fence();
-  // Columns of the X0' block: bit x of column j is bit j of row x.  Lane l
-  // holds row 64 b + l of block b; one ballot per P0 vertex and block.
 #pragma unroll
   for (int b = 0; b < NX; ++b) {
     uint64_t row[NW];
@@ -194,13 +190,25 @@ __device__ __forceinline__ void pk_seal(const PackWave<NW, NX> &w, uint32_t s, u
 #pragma unroll
     for (int q = 0; q < NW; ++q) {
       uint64_t mine = 0;
-      for (uint32_t j = 0; j < 64; ++j) {
+      const uint32_t n = p > 64u * q ? (p - 64u * q < 64 ? p - 64u * q : 64u) : 0u;
+      for (uint32_t j = 0; j < n; ++j) {
         const uint64_t col = __ballot((row[q] >> j) & 1);
         if (l == j) mine = col;
       }
       if (64u * q + l < p) sl[C::sXcol + (64u * q + l) * NX + b] = mine;
     }
   }
+}
+
+// Bookkeeping of slot s once its rows, columns, label hashes (and clique-list
+// ids) are in place.
+template <int NW, int NX>
+__device__ __forceinline__ void pk_seal(const PackWave<NW, NX> &w, uint32_t s, uint64_t p, uint64_t xq, uint64_t canon,
+                                        uint64_t base_key, uint32_t base_size, uint32_t graph, uint32_t v0,
+                                        uint32_t v1) {
+  using C = PackCfg<NW, NX>;
+  const KArgs &a = cold_args(w.a);
+  const uint32_t l = cold_lane();
   if (l == 0) {
     *w.m(mCanon, s) = canon;
     *w.m(mKey, s) = base_key;
@@ -296,7 +304,7 @@ __device__ __forceinline__ uint32_t pk_build(const PackWave<NW, NX> &w, uint8_t 
         or64_lds(sl + C::sProw + (uint64_t)j * NW + (i >> 6), 1ull << (i & 63));
       },
       [&](uint64_t i, uint32_t wd, uint64_t bits) { or64_lds(sl + C::sXrow + (i - p) * NW + wd, bits); });
-  wave_fence();
+  pk_columns<NW, NX>(w, s, (uint32_t)p, (uint32_t)xq);
   pk_seal<NW, NX>(w, s, p, xq, canon, sub.base_key, sub.base_size, sub.graph, sub.v0, sub.v1);
   return 1;
 }
@@ -392,30 +400,6 @@ __device__ __forceinline__ bool pk_group_build(const KArgs &a0, uint8_t *scratch
   return true;
 }
 
-// Bits of `row` at the set positions of the mask (held one word per lane,
-// lanes < W0), compressed in order into NW words.  The mask is uniform, so
-// every lane runs the same loop.
-template <int NW>
-__device__ __forceinline__ void pext_row(const PkGroup &G, uint64_t mk, uint32_t row, bool act, uint64_t (&out)[NW]) {
-#pragma unroll
-  for (int q = 0; q < NW; ++q) out[q] = 0;
-  uint32_t c = 0;
-  for (uint32_t q = 0; q < G.W0; ++q) {
-    uint64_t m = readlane64(mk, q);
-    if (m == 0) continue;
-    const uint64_t rw = act ? G.T[(uint64_t)q * G.rp + row] : 0ull;
-    for (; m; m &= m - 1, ++c) {
-      const uint64_t bit = (rw >> __builtin_ctzll(m)) & 1;
-      if constexpr (NW == 1) {
-        out[0] |= bit << c;
-      } else {
-        if (c < 64) out[0] |= bit << c;
-        else out[1] |= bit << (c - 64);
-      }
-    }
-  }
-}
-
 // Derives edge root `canon` = (v0, u_k) of group G into slot s (the whole
 // wave).  Returns as pk_build does, or 3 when the root's top node is pruned
 // by an X0' row covering P0 (its search words in `pruned`).
@@ -448,76 +432,53 @@ __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const P
   if (p > 64u * NW) {
     return 2;
   }
-  // X0' rows, in vertex order: rows x of X0v' adjacent to u_k, then U rows
-  // j < k adjacent to u_k, each kept when it has a neighbour in P0.  Their
-  // row numbers go to a list in the slot's column area (rewritten below).
+  // Candidate X0 rows, 64 a block: the rows x of X0v' adjacent to u_k (blocks
+  // [0, nbx)), then the U rows j < k adjacent to u_k (a block per word of xu) -
+  // ascending vertex order.
+  const uint32_t nbx = (G.xq0 + 63) / 64, nb = nbx + kq + 1;
+  auto candidate = [&](uint32_t b, uint32_t &row) -> bool {
+    if (b < nbx) {
+      row = G.d0 + 64 * b + l;
+      return 64 * b + l < G.xq0 && ((G.T[(uint64_t)kq * G.rp + row] >> kb) & 1);
+    }
+    row = 64 * (b - nbx) + l;
+    return (readlane64(xu, b - nbx) >> l) & 1;
+  };
+  // X0' keeps the rows with a neighbour in P0.  Row numbers go to lists in the
+  // slot's column area (rewritten below): X0' rows, then P0 rows.
   lds64 *sl = w.slot(s);
-  ldsu32 *xl = (ldsu32 *)(sl + C::sXcol);
+  ldsu32 *xl = (ldsu32 *)(sl + C::sXcol), *pl = xl + 64 * NX;
   uint32_t xq = 0;
-  for (uint32_t base = 0; base < G.xq0; base += 64) {
-    const uint32_t x = base + l;
-    const bool cand = x < G.xq0 && ((G.T[(uint64_t)kq * G.rp + G.d0 + x] >> kb) & 1);
-    bool keep = false;
-    for (uint32_t z = 0; z < G.W0; ++z) {  // uniform loop: the mask word is a readlane
+  for (uint32_t b = 0; b < nb; ++b) {
+    uint32_t row;
+    const bool cand = candidate(b, row);
+    if (__ballot(cand) == 0) continue;
+    uint64_t hit = 0;
+    for (uint32_t z = kq; z < G.W0; ++z) {  // (P0 lies above u_k)
       const uint64_t mz = readlane64(pk, z);
-      if (cand && !keep) keep = (G.T[(uint64_t)z * G.rp + G.d0 + x] & mz) != 0;
+      if (mz && cand) hit |= G.T[(uint64_t)z * G.rp + row] & mz;
     }
-    const uint64_t m = __ballot(keep);
-    if (keep && xq + rank_below(m) < 64u * NX) xl[xq + rank_below(m)] = G.d0 + x;
+    const uint64_t m = __ballot(hit != 0);
+    const uint32_t at = xq + rank_below(m);
+    if (hit != 0 && at < 64u * NX) xl[at] = row;
     xq += (uint32_t)__popcll(m);
   }
-  words_read += (G.xq0 + 63) / 64 * 64;
   const uint32_t nxu = __builtin_amdgcn_readlane(wave_scan_add_u32((uint32_t)__popcll(xu)), 63);
-  for (uint32_t base = 0; base < nxu; base += 64) {
-    // lane l takes the (base + l)-th U row below k adjacent to u_k
-    const uint32_t t = base + l;
-    uint32_t j = 0, before = 0;
-    for (uint32_t z = 0; z <= kq; ++z) {
-      const uint64_t wz = readlane64(xu, z);
-      const uint32_t cz = (uint32_t)__popcll(wz);
-      if (t >= before && t < before + cz) j = 64 * z + select64(wz, t - before);
-      before += cz;
-    }
-    bool keep = false;
-    for (uint32_t z = 0; z < G.W0; ++z) {
-      const uint64_t mz = readlane64(pk, z);
-      if (t < nxu && !keep) keep = (G.T[(uint64_t)z * G.rp + j] & mz) != 0;
-    }
-    const uint64_t m = __ballot(keep);
-    if (keep && xq + rank_below(m) < 64u * NX) xl[xq + rank_below(m)] = j;
-    xq += (uint32_t)__popcll(m);
-  }
-  words_read += (uint64_t)nxu * G.W0;
+  words_read += (uint64_t)nbx * 64 + (uint64_t)nxu * G.W0;
   if (xq > 64u * NX) {
     // Too many X0' rows for this variant.  When one of them covers P0, the
     // root's top node is pruned (no maximal clique below it): one node, no
     // slot.  Otherwise the root goes to the next launch.
     bool cov = false;
-    for (uint32_t base = 0; base < G.xq0; base += 64) {
-      const uint32_t x = base + l;
-      const bool cand = x < G.xq0 && ((G.T[(uint64_t)kq * G.rp + G.d0 + x] >> kb) & 1);
-      uint32_t c = 0;
-      for (uint32_t z = 0; z < G.W0; ++z) {
+    for (uint32_t b = 0; b < nb; ++b) {
+      uint32_t row;
+      const bool cand = candidate(b, row);
+      uint64_t miss = 0;
+      for (uint32_t z = kq; z < G.W0; ++z) {
         const uint64_t mz = readlane64(pk, z);
-        if (cand) c += (uint32_t)__popcll(G.T[(uint64_t)z * G.rp + G.d0 + x] & mz);
+        if (mz && cand) miss |= mz & ~G.T[(uint64_t)z * G.rp + row];
       }
-      cov |= cand && c == p;
-    }
-    for (uint32_t base = 0; base < nxu; base += 64) {
-      const uint32_t t = base + l;
-      uint32_t j = 0, before = 0;
-      for (uint32_t z = 0; z <= kq; ++z) {
-        const uint64_t wz = readlane64(xu, z);
-        const uint32_t cz = (uint32_t)__popcll(wz);
-        if (t >= before && t < before + cz) j = 64 * z + select64(wz, t - before);
-        before += cz;
-      }
-      uint32_t c = 0;
-      for (uint32_t z = 0; z < G.W0; ++z) {
-        const uint64_t mz = readlane64(pk, z);
-        if (t < nxu) c += (uint32_t)__popcll(G.T[(uint64_t)z * G.rp + j] & mz);
-      }
-      cov |= t < nxu && c == p;
+      cov |= cand && miss == 0;
     }
     if (__ballot(cov) == 0) return 2;
     words_read += (uint64_t)(G.xq0 + nxu) * G.W0;
@@ -525,54 +486,94 @@ __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const P
     pruned = (p + xq) * ((p + 63) / 64);  // the search words of evaluating the top node
     return 3;
   }
+  for (uint32_t z = kq, before = 0; z < G.W0; ++z) {
+    const uint64_t mz = readlane64(pk, z);
+    if ((mz >> l) & 1) pl[before + rank_below(mz)] = 64 * z + l;
+    before += (uint32_t)__popcll(mz);
+  }
   wave_fence();
-  // Row numbers (in G) of the edge root's rows: P0 (the set bits of pk in
-  // order) and X0' (the list).
-  uint32_t prow_id[NW], xrow_id[NX];
+  uint32_t prow[NW], xrow[NX];
 #pragma unroll
-  for (int r = 0; r < NW; ++r) {
-    const uint32_t t = 64u * r + l;
-    uint32_t j = 0, before = 0;
-    for (uint32_t z = 0; z < G.W0; ++z) {
-      const uint64_t wz = readlane64(pk, z);
-      const uint32_t cz = (uint32_t)__popcll(wz);
-      if (t >= before && t < before + cz) j = 64 * z + select64(wz, t - before);
-      before += cz;
+  for (int r = 0; r < NW; ++r) prow[r] = 64u * r + l < p ? (uint32_t)pl[64 * r + l] : 0u;
+#pragma unroll
+  for (int r = 0; r < NX; ++r) xrow[r] = 64u * r + l < xq ? (uint32_t)xl[64 * r + l] : 0u;
+  wave_fence();  // the lists are read before the column area is rewritten
+  // Every row restricted to P0's columns and compressed to P0's indices: the
+  // columns in order, one at a time, the same for every lane; a column's bit
+  // is shifted into the top of a 32-bit word (2 instructions per row block
+  // and column), and its ballot over the X0' rows is that column of the X0'
+  // block.  (Compressing each row on its own and transposing the block after
+  // took 16 instructions per column and 5 per column of all 64 NW.)
+  uint32_t pc[NW] = {}, xc[NX] = {};       // words being filled
+  uint32_t po[NW][2 * NW] = {}, xo[NX][2 * NW] = {};
+  uint64_t col[NW][NX] = {};               // lane l: column 64 q + l
+  uint32_t c = 0;
+  auto put = [&](uint32_t done) {          // word done / 32 - 1 is full, or the last one
+#pragma unroll
+    for (int o = 0; o < 2 * NW; ++o)
+      if ((done - 1) / 32 == (uint32_t)o) {
+        const uint32_t sh = (32 - (done & 31)) & 31;
+#pragma unroll
+        for (int r = 0; r < NW; ++r) po[r][o] = pc[r] >> sh;
+#pragma unroll
+        for (int r = 0; r < NX; ++r) xo[r][o] = xc[r] >> sh;
+      }
+  };
+  for (uint32_t z = kq; z < G.W0; ++z) {
+    const uint64_t mz = readlane64(pk, z);
+    if (mz == 0) continue;
+    uint64_t pw[NW], xw[NX];
+#pragma unroll
+    for (int r = 0; r < NW; ++r) pw[r] = 64u * r + l < p ? G.T[(uint64_t)z * G.rp + prow[r]] : 0ull;
+#pragma unroll
+    for (int r = 0; r < NX; ++r) xw[r] = 64u * r + l < xq ? G.T[(uint64_t)z * G.rp + xrow[r]] : 0ull;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      uint32_t ph[NW], xh[NX];
+#pragma unroll
+      for (int r = 0; r < NW; ++r) ph[r] = (uint32_t)(pw[r] >> (32 * h));
+#pragma unroll
+      for (int r = 0; r < NX; ++r) xh[r] = (uint32_t)(xw[r] >> (32 * h));
+      for (uint32_t m = (uint32_t)(mz >> (32 * h)); m; m &= m - 1) {
+        const uint32_t b = (uint32_t)__builtin_ctzll((uint64_t)m);
+#pragma unroll
+        for (int r = 0; r < NW; ++r) pc[r] = ((ph[r] >> b) << 31) | (pc[r] >> 1);
+#pragma unroll
+        for (int r = 0; r < NX; ++r) {
+          const uint32_t t = xh[r] >> b;
+          xc[r] = (t << 31) | (xc[r] >> 1);
+          const uint64_t cb = __ballot(t & 1);
+#pragma unroll
+          for (int q = 0; q < NW; ++q)
+            if (c == 64u * q + l) col[q][r] = cb;
+        }
+        if ((++c & 31) == 0) put(c);
+      }
     }
-    prow_id[r] = j;
   }
-#pragma unroll
-  for (int r = 0; r < NX; ++r) {
-    const uint32_t t = 64u * r + l;
-    xrow_id[r] = t < xq ? (uint32_t)xl[t] : 0u;
-  }
-  wave_fence();  // the list is read before the column area is rewritten
-  for (uint32_t i = l; i < C::sXcol; i += 64) sl[i] = 0;
+  if (c & 31) put(c);
 #pragma unroll
   for (int r = 0; r < NW; ++r) {
     const uint32_t t = 64u * r + l;
-    uint64_t o[NW];
-    pext_row<NW>(G, pk, prow_id[r], t < p, o);
     if (t < p) {
 #pragma unroll
-      for (int z = 0; z < NW; ++z) sl[C::sProw + t * NW + z] = o[z];
-      sl[C::sG + t] = G.lh[prow_id[r]];
-      if (a.list) a.pk_plist[((uint64_t)w.me * w.S + s) * kPackMaxP + t] = a.col[G.o0 + prow_id[r]];
+      for (int o = 0; o < NW; ++o) sl[C::sProw + t * NW + o] = (uint64_t)po[r][2 * o] | ((uint64_t)po[r][2 * o + 1] << 32);
+#pragma unroll
+      for (int b = 0; b < NX; ++b) sl[C::sXcol + t * NX + b] = col[r][b];
+      sl[C::sG + t] = G.lh[prow[r]];
+      if (a.list) a.pk_plist[((uint64_t)w.me * w.S + s) * kPackMaxP + t] = a.col[G.o0 + prow[r]];
     }
   }
 #pragma unroll
   for (int r = 0; r < NX; ++r) {
     const uint32_t t = 64u * r + l;
-    uint64_t o[NW];
-    pext_row<NW>(G, pk, xrow_id[r], t < xq, o);
     if (t < xq) {
 #pragma unroll
-      for (int z = 0; z < NW; ++z) sl[C::sXrow + t * NW + z] = o[z];
+      for (int o = 0; o < NW; ++o) sl[C::sXrow + t * NW + o] = (uint64_t)xo[r][2 * o] | ((uint64_t)xo[r][2 * o + 1] << 32);
     }
   }
   words_read += (uint64_t)(p + xq) * G.W0;
   acc.build += 8 * words_read + 8ull * NW * (p + xq);
-  wave_fence();
   pk_seal<NW, NX>(w, s, p, xq, canon, base_key, 2, graph, G.v0, uk);
   return 1;
 }
