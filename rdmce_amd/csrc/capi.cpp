@@ -418,6 +418,7 @@ struct mce_plan {
   // packed search (pack_kernel.hip): settings and arenas, allocated at its
   // first run
   uint64_t max_out = 0;              // largest out-degree: bounds |P0| and the search depth
+  uint64_t max_deg = 0;              // largest degree: bounds |X0'|
   int pack = 0;
   uint32_t pack_slots = 4;
   int pack_wpc = 16;
@@ -425,10 +426,10 @@ struct mce_plan {
   uint64_t pk_stack_words = 0;       // record stack words per wave
   uint64_t *d_pk_stack = nullptr;
   uint32_t *d_pk_plist = nullptr;
-  uint64_t *d_wide[2] = {nullptr, nullptr};
+  uint64_t *d_wide[kPackVariants] = {};  // roots too wide for variant v, in the order met
   uint64_t *d_mail = nullptr;       // packed search: per-wave mail (work handed to idle waves)
   unsigned long long *d_pk_idle = nullptr;
-  uint64_t *d_wide_h = nullptr;     // per entry of the first list: its kept vertex bitmap in d_pool
+  uint64_t *d_wide_h[2] = {};       // per entry of list v (in turn): its kept vertex bitmap in d_pool
   uint64_t *d_pool = nullptr;
   uint64_t pool_words = 0;
   uint64_t pool_bound = 0;           // words that every vertex's bitmap would take
@@ -451,12 +452,13 @@ namespace {
 // Words of d_ctr: the collected sums (Sum), then the others.
 enum Ctr { kCount = sCount, kHash = sHash, kNodes = sNodes, kWords = sWords, kBuild = sBuild, kShared = sShared,
            kPublished = sPublished, kOwnerTasks = sOwner, kListCursor = kNumSums, kNDeferred, kDeferNeed,
-           kDeferStackNeed, kErr, kNWide1, kNWide2, kPoolUsed, kNumCtr };
+           kDeferStackNeed, kErr, kNWide0, kPoolUsed = kNWide0 + kPackVariants, kNumCtr };
 // Words of d_work, the per-run counters kept in copies: dispatch counters and
-// work state of up to three launches, the sums and the clique sizes.
+// work state of each launch of a run, the sums and the clique sizes.
+constexpr uint64_t kLaunches = kPackVariants + 1;
 constexpr uint64_t kNextWords = (uint64_t)kShards * kShardWords;
 constexpr uint64_t kStateWords = (uint64_t)kStateShards * kShardWords;
-constexpr uint64_t kStateAt = 3 * kNextWords, kSumsAt = kStateAt + 3 * kStateWords,
+constexpr uint64_t kStateAt = kLaunches * kNextWords, kSumsAt = kStateAt + kLaunches * kStateWords,
                    kHistAt = kSumsAt + (uint64_t)kShards * kShardWords,
                    kWorkWords = kHistAt + (uint64_t)kShards * kLdsHist;
 
@@ -481,9 +483,10 @@ void plan_release(mce_plan *p) {
                   p->d_root_nodes, p->d_root_cycles, p->d_list,     p->d_deferred,    p->d_deferred2,
                   p->d_slots2,   p->d_stacks,      p->d_stacks2,    p->d_recs,        p->d_users,
                   p->d_has_work, p->d_root_graph,  p->d_gcount,     p->d_ghash,       p->d_ghist,
-                  p->d_work,     p->d_pk_stack,    p->d_pk_plist,   p->d_wide[0],     p->d_wide[1],
-                  p->d_wide_h,   p->d_mail,    p->d_pk_idle,  p->d_pool,        p->d_rfirst,     p->d_gstart};
+                  p->d_work,     p->d_pk_stack,    p->d_pk_plist,   p->d_wide_h[0], p->d_wide_h[1],   p->d_mail,    p->d_pk_idle,  p->d_pool,        p->d_rfirst,     p->d_gstart};
   for (void *q : ptrs)
+    if (q) (void)hipFree(q);
+  for (void *q : p->d_wide)
     if (q) (void)hipFree(q);
   for (auto &e : p->ev)
     if (e) (void)hipEventDestroy(e);
@@ -612,6 +615,7 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
     // (the packed search's pool bound)
     for (uint64_t v = 0; v < g.n; ++v) {
       const uint64_t d = g.rowoff[v + 1] - outoff[v], x = outoff[v] - g.rowoff[v];
+      p->max_deg = std::max(p->max_deg, d + x);
       if (d >= 2 && d <= 1024) p->pool_bound += 8 + (d + 63) / 64 * (align_up(d + x, 64) + 1) + d;
     }
     PTRY(dalloc(&p->d_outoff, g.n + 1));
@@ -803,16 +807,16 @@ uint64_t pack_need_records(const mce_plan *p, uint32_t nw) {
 mce_status ensure_pack(mce_plan *p) {
   if (p->d_pk_stack && (!p->opt.want_list || p->d_pk_plist)) return MCE_OK;
   const uint32_t waves = (uint32_t)std::min<uint64_t>(p->max_waves, (uint64_t)p->cus * 32);
-  const uint64_t words = std::max(pack_need_records(p, 1) * pack_rec_words(1, 1),
-                                  pack_need_records(p, 2) * pack_rec_words(2, 2));
+  uint64_t words = 0;
+  for (int v = 0; v < kPackVariants; ++v)
+    words = std::max(words, pack_need_records(p, kPackNW[v]) * pack_rec_words(kPackNW[v], kPackNX[v]));
   if (!p->d_pk_stack) {
     HIP_TRY(dalloc(&p->d_pk_stack, words * waves));
     p->pk_stack_words = words;
     p->pack_waves_alloc = waves;
     p->wide_cap = std::max<uint64_t>(p->n_dispatch, 1);
-    HIP_TRY(dalloc(&p->d_wide[0], p->wide_cap));
-    HIP_TRY(dalloc(&p->d_wide[1], p->wide_cap));
-    HIP_TRY(dalloc(&p->d_wide_h, p->wide_cap));
+    for (auto &q : p->d_wide) HIP_TRY(dalloc(&q, p->wide_cap));
+    for (auto &q : p->d_wide_h) HIP_TRY(dalloc(&q, p->wide_cap));
     HIP_TRY(dalloc(&p->d_mail, (uint64_t)kPackMailWords * waves));
     HIP_TRY(dalloc(&p->d_pk_idle, (waves + 63) / 64));
     // Kept vertex bitmaps: at most one per vertex with two or more edge
@@ -868,10 +872,10 @@ uint32_t mce_waves(const mce_plan *p, KArgs &a) {
 
 // Resets every counter, result and sharing word of a run with one fill kernel
 // (graph-capturable; one launch per buffer took 11 launches, 2 us each) and
-// launches the enumeration kernels: with the packed
-// search on, pack<1,1> over the dispatch list, pack<2,2> over the roots it
-// found too wide (derived from the vertex bitmaps pack<1,1> kept for them),
-// and the one-root-per-wave kernel over the rest (each
+// launches the enumeration kernels: with the packed search on, its variants
+// in turn, the first over the dispatch list, each next one over the roots the
+// one before found too wide (derived from the vertex bitmaps the first one
+// kept for them), and the one-root-per-wave kernel over the rest (each
 // later launch reads its list length from the counter the earlier one
 // filled, so the sequence needs no host round trip).
 hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
@@ -891,8 +895,9 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
   }
   const uint64_t units = a.pk_gstart ? a.pk_ngroups : a.n_dispatch;
   const bool share = can_share(p, a);
-  for (int v = 0; v < 2 && e == hipSuccess; ++v) {
-    const uint32_t nw = v == 0 ? 1 : 2, nx = nw;
+  const bool batch = a.root_graph != nullptr;
+  for (int v = 0; v < kPackVariants && e == hipSuccess; ++v) {
+    const uint32_t nw = kPackNW[v], nx = kPackNX[v];
     KArgs b = a;
     b.pk_stack = p->d_pk_stack;
     b.pk_cap = p->pk_stack_words / pack_rec_words(nw, nx);
@@ -900,37 +905,38 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
 #ifdef RDMCE_PACK_THR_MAX  // test builds: reach the depth-first expansion on small graphs
     b.pk_thr = std::min<uint32_t>(b.pk_thr, RDMCE_PACK_THR_MAX);
 #endif
-    // the two-word variant's slots are 3.5x larger: half as many; and no more
-    // than let the requested waves per CU all be resident in its LDS (a wave
-    // that waits for LDS starts late and finds little work left)
-    const bool batch = a.root_graph != nullptr;
-    uint32_t slots = v == 0 ? p->pack_slots : std::max<uint32_t>(1, p->pack_slots / 2);
+    // the wider variants' slots are 3.5 and 5.3 times larger: half and a
+    // quarter as many; and no more than let the requested waves per CU all be
+    // resident in its LDS (a wave that waited for LDS started late)
+    uint32_t slots = std::max<uint32_t>(1, p->pack_slots >> v);
     while (slots > 1 && (pack_lds_bytes(nw, nx, slots, batch) > p->lds_per_block_max ||
                          pack_lds_bytes(nw, nx, slots, batch) * (uint64_t)p->pack_wpc > p->lds_per_cu))
       --slots;
     b.pk_slots = slots;
     b.pk_plist = p->d_pk_plist;
     b.wide = p->d_wide[v];
-    b.n_wide = p->d_ctr + (v == 0 ? kNWide1 : kNWide2);
-    b.heavy = p->d_wide[1];
-    b.n_heavy = p->d_ctr + kNWide2;
+    b.n_wide = p->d_ctr + kNWide0 + v;
+    b.heavy = p->d_wide[kPackVariants - 1];
+    b.n_heavy = p->d_ctr + kNWide0 + kPackVariants - 1;
     b.pk_pool = p->d_pool;
     b.pk_pool_words = p->pool_words;
     b.pk_pool_used = p->d_ctr + kPoolUsed;
-    if (v == 0) {  // wide roots leave with a copy of their vertex bitmap ...
-      b.wide_h = p->d_wide_h;
-    } else {       // ... from which the next launch derives them
+    // wide roots leave with a copy of their vertex bitmap, from which the
+    // next launches derive them
+    b.wide_h = v + 1 < kPackVariants ? p->d_wide_h[v & 1] : nullptr;
+    if (v) {
       b.eager = nullptr;
       b.pk_gstart = nullptr;
-      b.pk_whandle = p->d_wide_h;
-      b.perm = p->d_wide[0];
+      b.pk_whandle = p->d_wide_h[(v - 1) & 1];
+      b.perm = p->d_wide[v - 1];
       b.reverse = 0;
-      b.n_dispatch_dev = p->d_ctr + kNWide1;
-      b.next_root = p->d_work + kNextWords;
+      b.n_dispatch_dev = p->d_ctr + kNWide0 + v - 1;
+      b.next_root = p->d_work + v * kNextWords;
     }
-    // Without sharing, waves beyond the runs the first launch hands out have
-    // nothing to do (the second one's list length is not known here).
-    uint32_t pw = pack_waves(p);
+    // Waves: those that fit a CU's LDS; without sharing, no more than the runs
+    // the first launch hands out (the others' list lengths are not known here).
+    const uint64_t fit = std::max<uint64_t>(1, p->lds_per_cu / pack_lds_bytes(nw, nx, slots, batch));
+    uint32_t pw = (uint32_t)std::min<uint64_t>(pack_waves(p), fit * p->cus);
     if (v == 0 && !share) pw = (uint32_t)std::min<uint64_t>(pw, std::max<uint64_t>(units, 1));
     b.state = p->d_work + kStateAt + v * kStateWords;
     b.pk_share = share;
@@ -938,15 +944,18 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
     b.pk_idle = p->d_pk_idle;
     b.pk_mail = p->d_mail;
     e = launch_pack(b, v, pw, (uint32_t)p->pack_wpc, s);
+    // No root of this graph is too wide for this variant: |P0| is at most the
+    // largest out-degree, |X0'| the largest degree.
+    if (p->max_out <= 64 * nw && p->max_deg <= 64 * nx && !a.eager) return e == hipSuccess ? collect(p, s) : e;
   }
   if (e != hipSuccess) return e;
   KArgs c = a;
-  c.perm = p->d_wide[1];
+  c.perm = p->d_wide[kPackVariants - 1];
   c.reverse = 0;
   c.eager = nullptr;
-  c.n_dispatch_dev = p->d_ctr + kNWide2;
-  c.next_root = p->d_work + 2 * kNextWords;
-  c.state = p->d_work + kStateAt + 2 * kStateWords;
+  c.n_dispatch_dev = p->d_ctr + kNWide0 + kPackVariants - 1;
+  c.next_root = p->d_work + kPackVariants * kNextWords;
+  c.state = p->d_work + kStateAt + kPackVariants * kStateWords;
   if (!can_share(p, c)) c.share_bound = -1;
   e = launch_mce(c, p->waves, (uint32_t)p->waves_per_cu, s);
   return e == hipSuccess ? collect(p, s) : e;

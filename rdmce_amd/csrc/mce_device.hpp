@@ -181,7 +181,13 @@ struct KArgs {
   uint64_t *pk_mail;
 };
 
-// Packed search variants: |P0| <= 64 NW and |X0'| <= 64 NX.
+// Packed search variants: |P0| <= 64 NW and |X0'| <= 64 NX.  The third one is
+// for skewed graphs, whose roots often have twice as many excluded rows as
+// candidates: on R-MAT 14, edge factor 14, roots with |P0| <= 128 and 128 <
+// |X0'| <= 192 hold 58% of the tree nodes.
+constexpr int kPackVariants = 3;
+constexpr uint32_t kPackNW[kPackVariants] = {1, 2, 2};
+constexpr uint32_t kPackNX[kPackVariants] = {1, 2, 4};
 constexpr uint32_t kPackMaxP = 128;
 constexpr uint32_t kPackMaxSlots = 8;
 // Record words of variant (nw, nx): P XP V R (nw each), XX (nx), key, meta.
@@ -200,7 +206,7 @@ constexpr uint32_t kMailHdr = 16;
 constexpr uint32_t pack_mail_words(uint32_t nw, uint32_t nx) {
   return kMailHdr + 16 + pack_slot_words(nw, nx) + kPackMaxP / 2 + 64 * pack_rec_words(nw, nx);
 }
-constexpr uint32_t kPackMailWords = pack_mail_words(2, 2);
+constexpr uint32_t kPackMailWords = pack_mail_words(2, 4);
 // LDS bytes of a wave of the packed search.
 constexpr uint64_t pack_lds_bytes(uint32_t nw, uint32_t nx, uint32_t slots, bool batch) {
   return 8ull * (kLdsHist + 32 + slots * (kPackMetaWords + pack_slot_words(nw, nx) + (batch ? pack_hist_words(nw) : 0)));
@@ -209,9 +215,10 @@ constexpr uint64_t pack_lds_bytes(uint32_t nw, uint32_t nx, uint32_t slots, bool
 // waves_per_cu selects the kernel variant compiled for that occupancy
 // (<= 16: 4 waves per SIMD, <= 20: 5, <= 24: 6, else 8).
 hipError_t launch_mce(const KArgs &a, uint32_t waves, uint32_t waves_per_cu, hipStream_t stream);
-// Packed search: variant 0 = (NW, NX) = (1, 1), 1 = (2, 2); waves_per_cu
-// selects the kernel compiled for that occupancy (<= 16: 4 waves per SIMD,
-// <= 20: 5, <= 24: 6, else 8).
+// Packed search: variant v = (kPackNW[v], kPackNX[v]); waves_per_cu selects
+// the kernel compiled for that occupancy (<= 16: 4 waves per SIMD, <= 20: 5,
+// <= 24: 6, else 8), except for the last variant, of which LDS lets 13 waves
+// share a CU.
 hipError_t launch_pack(const KArgs &a, int variant, uint32_t waves, uint32_t waves_per_cu, hipStream_t stream);
 hipError_t launch_copy_probe(const void *src, void *dst, uint64_t bytes, hipStream_t stream);
 // Zero-fills n 64-bit words with a kernel (safe inside captured hipGraphs,

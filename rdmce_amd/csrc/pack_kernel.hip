@@ -914,7 +914,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
         } else if (l == 0) {
           const unsigned long long at = atomicAdd(a.n_wide, 1ull);
           a.wide[at] = canon;
-          if (a.wide_h) a.wide_h[at] = ~0ull;
+          if (a.wide_h) a.wide_h[at] = hk;
         }
       }
       if (built == 1) {
@@ -1298,7 +1298,14 @@ hipError_t launch_variant(const KArgs &a, uint32_t waves, uint32_t wpc, size_t l
 hipError_t launch_pack(const KArgs &a, int variant, uint32_t waves, uint32_t waves_per_cu, hipStream_t stream) {
   const bool batch = a.root_graph != nullptr;
   if (variant == 0) return launch_variant<1, 1>(a, waves, waves_per_cu, pack_lds_bytes(1, 1, a.pk_slots, batch), stream);
-  return launch_variant<2, 2>(a, waves, waves_per_cu, pack_lds_bytes(2, 2, a.pk_slots, batch), stream);
+  if (variant == 1)
+    return launch_variant<2, 2>(a, waves, waves_per_cu, pack_lds_bytes(2, 2, a.pk_slots, batch), stream);
+  const size_t lds = pack_lds_bytes(2, 4, a.pk_slots, batch);
+  if (a.list)
+    hipLaunchKernelGGL((pack_kernel<2, 4, 4, true>), dim3(waves), dim3(64), lds, stream, a);
+  else
+    hipLaunchKernelGGL((pack_kernel<2, 4, 4, false>), dim3(waves), dim3(64), lds, stream, a);
+  return hipGetLastError();
 }
 
 }  // namespace rdmce
