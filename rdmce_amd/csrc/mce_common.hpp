@@ -237,6 +237,11 @@ __device__ __forceinline__ bool state_any(const KArgs &a, uint32_t me, bool look
   }
   return any;
 }
+// Every copy at once, one per lane (the others 0).
+__device__ __forceinline__ unsigned long long state_poll(const KArgs &a) {
+  const uint32_t l = lane();
+  return l < kStateShards ? ld_relaxed(&a.state[(uint64_t)l * kShardWords]) : 0ull;
+}
 __device__ __forceinline__ bool any_idle(const KArgs &a, uint32_t me) { return state_any(a, me, true); }
 __device__ __forceinline__ bool any_working(const KArgs &a, uint32_t me) { return state_any(a, me, false); }
 

@@ -43,16 +43,18 @@
 // Sharing: a wave that runs out of roots and records asks for work (its bit in
 // pk_idle); every kPackPoll passes a working wave looks for such waves and
 // mails one of them half of its run's unbuilt roots or, when its run has none
-// to spare, about half of its pending tasks - whole records from the bottom of
-// its stack (the shallowest, so the largest subtrees) with a copy of their
-// subproblem.  The records given away stay in the stack as empty ones.  This
-// is the reference's root-down exposure (BkPivotBitBalance.cuh:87-138) with
-// the giver doing the copying: a taker reads only its own mail, so a few
-// thousand waiting waves poll a few thousand lines.
-// What it measured: R-MAT 14, edge factor 14 (108M nodes, most below a few
-// roots), one-word launch 30.2 -> 6.0 ms, two-word launch 80 -> 16.2 ms; a
-// 200k-vertex community graph 23.7 -> 16.9 and 7.0 -> 6.3 ms.  It is off where
-// no root can reach the sharing bound (|P0| is at most the largest out-degree).
+// to spare, every other record among the lowest of its stack (the shallowest,
+// so the largest subtrees) with a copy of their subproblem - or the upper half
+// of a single record's candidates.  The records given away stay in the stack
+// as empty ones.  This is the reference's root-down exposure
+// (BkPivotBitBalance.cuh:87-138) with the giver doing the copying: a taker
+// reads only its own mail, so a few thousand waiting waves poll a few thousand
+// lines.  What it measured, all launches: R-MAT 14, edge factor 14 (108M
+// nodes, most below a few roots) 110 ms without sharing, 49 ms giving the lower
+// half of the stack (the giver was left with little and asked next), 12.5 ms
+// giving every other record; a 200k-vertex community graph 31, 28 and 24 ms.
+// It is off where no root can reach the sharing bound (|P0| is at most the
+// largest out-degree).
 #include "mce_common.hpp"
 
 extern __shared__ uint64_t lds_dyn[];
@@ -61,11 +63,13 @@ namespace rdmce {
 namespace {
 
 constexpr uint32_t kRecRoot = 1u << 24;  // meta flag: the record's one task is its root's top node
-// Passes between looks for idle waves (a power of two; a pass takes a few us,
-// a look one round trip past the L2), and pending tasks from which on a wave
-// gives some away (a gift costs the giver a few passes).
-constexpr uint32_t kPackPoll = 16;
-constexpr uint32_t kPackSpare = 16;
+// Passes between looks for idle waves (a power of two; a pass takes 10 - 20
+// us), and pending tasks from which on a wave gives some away.  R-MAT 14 /
+// community graph, ms: looks every 4 passes 12.7 / 27.1, 8 12.5 / 24.0, 16
+// 13.7 / 23.8 (each gift copies a subproblem, and the taker starts with part
+// of a pass).
+constexpr uint32_t kPackPoll = 8;
+constexpr uint32_t kPackSpare = 32;
 
 template <int NW, int NX>
 struct PackCfg {
@@ -104,6 +108,25 @@ __device__ __forceinline__ uint32_t select64(uint64_t w, uint32_t k) {
   if (k >= c) { k -= c; w >>= 2; pos += 2; }
   if (k >= (uint32_t)(w & 1)) pos += 1;
   return pos;
+}
+
+// Mail words are written and read at the coherence point of the XCDs' L2s
+// (relaxed device-scope accesses).  Plain accesses with a release by the giver
+// and an acquire by the taker write back and invalidate a whole L2 for each
+// gift: R-MAT 14 spent three quarters of its wave time waiting, with more
+// gifts making it slower.
+__device__ __forceinline__ void st_mail(uint64_t *p, uint64_t v) {
+  __hip_atomic_store((unsigned long long *)p, (unsigned long long)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t ld_mail(const uint64_t *p) { return ld_relaxed((unsigned long long *)p); }
+// Waits until this wave's mail stores have reached that point.  (A fence of
+// workgroup scope does not wait for global stores, one of device scope writes
+// back the L2.)
+__device__ __forceinline__ void mail_stored() {
+#ifdef __AMDGCN__
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+  wave_fence();
 }
 
 // The per-wave LDS areas (word offsets from lds_dyn).
@@ -509,15 +532,14 @@ __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const P
   uint64_t col[NW][NX] = {};               // lane l: column 64 q + l
   uint32_t c = 0;
   auto put = [&](uint32_t done) {          // word done / 32 - 1 is full, or the last one
+    const uint32_t sh = (32 - (done & 31)) & 31, w = (done - 1) / 32;
 #pragma unroll
-    for (int o = 0; o < 2 * NW; ++o)
-      if ((done - 1) / 32 == (uint32_t)o) {
-        const uint32_t sh = (32 - (done & 31)) & 31;
+    for (uint32_t o = 0; o < 2 * NW; ++o) {  // (selects: an indexed array would go to scratch)
 #pragma unroll
-        for (int r = 0; r < NW; ++r) po[r][o] = pc[r] >> sh;
+      for (int r = 0; r < NW; ++r) po[r][o] = o == w ? pc[r] >> sh : po[r][o];
 #pragma unroll
-        for (int r = 0; r < NX; ++r) xo[r][o] = xc[r] >> sh;
-      }
+      for (int r = 0; r < NX; ++r) xo[r][o] = o == w ? xc[r] >> sh : xo[r][o];
+    }
   };
   for (uint32_t z = kq; z < G.W0; ++z) {
     const uint64_t mz = readlane64(pk, z);
@@ -677,37 +699,31 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
       }
       const uint32_t f = (uint32_t)__builtin_ctzll(nz);
       s0 = __builtin_amdgcn_readlane((uint32_t)(dm >> 16) & 0xFF, f);
-      const uint32_t c = ((uint32_t)(dm >> 16) & 0xFF) == s0 ? ci : 0u;
-      const uint32_t incl = wave_scan_add_u32(c);
-      const uint32_t half = (uint32_t)((pending + 1) / 2);
-      take = c != 0 && incl - c < half;
-      sel_m = __ballot(take);
-      uint32_t last = 63 - (uint32_t)__builtin_clzll(sel_m);
-      cands = __builtin_amdgcn_readlane(incl, last);
-      if (cands == pending) {
-        if (sel_m & (sel_m - 1)) {  // everything: keep the last one
-          sel_m &= ~(1ull << last);
-          take = take && l != last;
-          cands -= __builtin_amdgcn_readlane(c, last);
-        } else {  // one record holds all tasks: its upper half
-          split = true;
-          uint32_t kk = ci / 2, base = 0;
+      const uint64_t same = __ballot(ci != 0 && ((uint32_t)(dm >> 16) & 0xFF) == s0);
+      const uint32_t cf = __builtin_amdgcn_readlane(ci, f);
+      if (same & (same - 1)) {  // every other record
+        take = ((same >> l) & 1) && (rank_below(same) & 1);
+      } else {                  // a single record: the upper half of its candidates
+        take = l == f;
+        split = cf > 1;
+        uint32_t kk = ci / 2, base = 0;
 #pragma unroll
-          for (int q = 0; q < NW - 1; ++q) {
-            const uint32_t cq = (uint32_t)__popcll(rem[q]);
-            if (base == (uint32_t)q * 64 && kk >= cq) {
-              kk -= cq;
-              base = (uint32_t)(q + 1) * 64;
-            }
+        for (int q = 0; q < NW - 1; ++q) {
+          const uint32_t cq = (uint32_t)__popcll(rem[q]);
+          if (base == (uint32_t)q * 64 && kk >= cq) {
+            kk -= cq;
+            base = (uint32_t)(q + 1) * 64;
           }
-          uint64_t rw = rem[0];
-#pragma unroll
-          for (int q = 1; q < NW; ++q)
-            if (base == (uint32_t)q * 64) rw = rem[q];
-          mid = base + (take ? select64(rw, kk) : 0u);
-          cands -= cands / 2;
         }
+        uint64_t rw = rem[0];
+#pragma unroll
+        for (int q = 1; q < NW; ++q)
+          if (base == (uint32_t)q * 64) rw = rem[q];
+        mid = base + (split && take ? select64(rw, kk) : 0u);
       }
+      sel_m = __ballot(take);
+      cands = split ? cf - cf / 2
+                    : __builtin_amdgcn_readlane(wave_scan_add_u32(take ? ci : 0u), 63);
     }
     // claim an idle wave
     const int to = find_wave(a.pk_idle, a.pk_nwaves, w.me);
@@ -721,31 +737,30 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     if (range) {  // the upper half of the run's unbuilt roots
       const uint64_t at = gcur + (gend - gcur + 1) / 2;
       if (l == 0) {
-        out[1] = at;
-        out[2] = gend;
+        st_mail(out + 1, at);
+        st_mail(out + 2, gend);
       }
       gend = at;
       flag = 2;
     } else {
       const lds64 *sl = w.slot(s0);
       const uint32_t n = (uint32_t)__popcll(sel_m), rk = rank_below(sel_m);
-      for (uint32_t i = l; i < C::SW; i += 64) out[oSlot + i] = sl[i];
+      for (uint32_t i = l; i < C::SW; i += 64) st_mail(out + oSlot + i, sl[i]);
       if (l < kPackMetaWords) {
         uint64_t v = w.L.meta[l * S + s0];
         v = l == mRefs ? (uint64_t)n : (l == mNodes || l == mCount || l == mHash ? 0ull : v);
-        out[oMeta0 + l] = v;
+        st_mail(out + oMeta0 + l, v);
       }
       if (lists) {
-        const uint32_t *pl = a.pk_plist + ((uint64_t)w.me * S + s0) * kPackMaxP;
-        uint32_t *dst = (uint32_t *)(out + oIds);
-        for (uint32_t i = l; i < kPackMaxP; i += 64) dst[i] = pl[i];
+        const uint64_t *ids = (const uint64_t *)(a.pk_plist + ((uint64_t)w.me * S + s0) * kPackMaxP);
+        for (uint32_t i = l; i < kPackMaxP / 2; i += 64) st_mail(out + oIds + i, ids[i]);
       }
       if (take) {
         for (uint32_t f = 0; f < (lists ? C::RS : C::RS - NW); ++f)
-          if (f != C::oMeta) out[oRecs + f * 64 + rk] = fld(f, given + l);
+          if (f != C::oMeta) st_mail(out + oRecs + f * 64 + rk, fld(f, given + l));
         uint64_t tm = dm & ~(0xFFull << 16);  // the taker's slot 0
         if (split) tm = (tm & ~(0xFFull << 32)) | ((uint64_t)mid << 32);
-        out[oRecs + C::oMeta * 64 + rk] = tm;
+        st_mail(out + oRecs + C::oMeta * 64 + rk, tm);
         fld(C::oMeta, given + l) = split ? (dm & ~(0xFFull << 40)) | ((uint64_t)mid << 40) : dm & 0xFFFFFFFFull;
       }
       pending -= cands;
@@ -754,24 +769,23 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
       flag = 1 | ((uint64_t)n << 8) | ((uint64_t)cands << 32);
     }
     state_add(a, (uint32_t)to, kWorking - kLooking);
-    wave_fence();
-    if (l == 0) __hip_atomic_store((unsigned long long *)out, (unsigned long long)flag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    mail_stored();  // the mail is there before its flag
+    if (l == 0) st_mail(out, flag);
   };
   // Waits for work from another wave; false when there is none to come.
   auto wait_mail = [&]() -> bool {
     const KArgs &a = cold_args(w.a);
     const uint32_t l = cold_lane();
     const uint64_t bit = 1ull << (w.me & 63);
-    if (l == 0) {
-      __hip_atomic_store((unsigned long long *)mail, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_fetch_or(&a.pk_idle[w.me >> 6], (unsigned long long)bit, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (l == 0) st_mail(mail, 0);
+    mail_stored();
+    if (l == 0) atomicOr(&a.pk_idle[w.me >> 6], (unsigned long long)bit);
     state_add(a, w.me, kLooking - kWorking);
     uint64_t flag = 0;
     bool asked = true;
     for (uint32_t n = 1, k = 0;; n = n < 8 ? n * 2 : 8, ++k) {
       unsigned long long v = 0;
-      if (l == 0) v = ld_relaxed((unsigned long long *)mail);
+      if (l == 0) v = ld_mail(mail);
       flag = bcast64(v);
       if (flag) break;
       if (asked && (k & 3) == 0 && !any_working(a, w.me)) {
@@ -783,31 +797,26 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
       }
       if (l == 0) nap(n);
     }
-    if (l == 0) {
-      unsigned long long v = __hip_atomic_load((unsigned long long *)mail, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-      (void)v;
-    }
     wave_fence();
     ++acc.shared;
     if ((flag & 0xFF) == 2) {
-      gcur = bcast64(mail[1]);
-      gend = bcast64(mail[2]);
+      gcur = bcast64(ld_mail(mail + 1));
+      gend = bcast64(ld_mail(mail + 2));
       new_run = true;
       return true;
     }
     const uint32_t n = (uint32_t)(flag >> 8) & 0xFF;
     lds64 *sl = w.slot(0);
-    for (uint32_t i = l; i < C::SW; i += 64) sl[i] = mail[oSlot + i];
-    if (l < kPackMetaWords) w.L.meta[l * S] = mail[oMeta0 + l];
+    for (uint32_t i = l; i < C::SW; i += 64) sl[i] = ld_mail(mail + oSlot + i);
+    if (l < kPackMetaWords) w.L.meta[l * S] = ld_mail(mail + oMeta0 + l);
     if (a.root_graph)
       for (uint32_t i = l; i < C::HS; i += 64) w.L.bhist[i] = 0;
     if (lists) {
-      uint32_t *pl = a.pk_plist + (uint64_t)w.me * S * kPackMaxP;
-      const uint32_t *src = (const uint32_t *)(mail + oIds);
-      for (uint32_t i = l; i < kPackMaxP; i += 64) pl[i] = src[i];
+      uint64_t *ids = (uint64_t *)(a.pk_plist + (uint64_t)w.me * S * kPackMaxP);
+      for (uint32_t i = l; i < kPackMaxP / 2; i += 64) ids[i] = ld_mail(mail + oIds + i);
     }
     if (l < n)
-      for (uint32_t f = 0; f < (lists ? C::RS : C::RS - NW); ++f) fld(f, l) = mail[oRecs + f * 64 + l];
+      for (uint32_t f = 0; f < (lists ? C::RS : C::RS - NW); ++f) fld(f, l) = ld_mail(mail + oRecs + f * 64 + l);
     wave_fence();
     top = n;
     given = 0;
@@ -933,6 +942,9 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
       if (!sharing || !wait_mail()) break;
       continue;
     }
+
+    // A look for idle waves, used at the end of the pass.
+    const unsigned long long seen = sharing && (++tick & (kPackPoll - 1)) == 0 ? state_poll(a) : 0ull;
 
     // Dispatch up to 64 tasks from the top of the stack: look-lane i sees
     // record top-1-i; task lane l takes candidate k of look-record ri.
@@ -1254,9 +1266,14 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     const uint64_t dm = __ballot(done);
     if (done) pk_finish<NW, NX>(w, l);
     busy &= ~(uint32_t)dm;
-    if (sharing && __builtin_expect((++tick & (kPackPoll - 1)) == 0, 0) &&
-        __builtin_expect_with_probability(any_idle(a, w.me), 0, 0.999))
-      give();
+    if (__builtin_expect_with_probability(__ballot((seen >> 32) != 0) != 0, 0, 0.999)) {
+      // Of the working waves about one per idle one tries: when all tried,
+      // they queued on the few idle waves' words.
+      const uint32_t looking = __builtin_amdgcn_readlane(wave_scan_add_u32((uint32_t)(seen >> 32)), 63);
+      const uint32_t working = __builtin_amdgcn_readlane(wave_scan_add_u32((uint32_t)seen), 63);
+      const uint32_t h = (uint32_t)splitmix64_mix(((uint64_t)w.me << 32) | tick);
+      if ((uint32_t)(((uint64_t)h * working) >> 32) < looking) give();
+    }
   }
 
   // Exit: the wave's sums.
@@ -1302,9 +1319,9 @@ hipError_t launch_pack(const KArgs &a, int variant, uint32_t waves, uint32_t wav
     return launch_variant<2, 2>(a, waves, waves_per_cu, pack_lds_bytes(2, 2, a.pk_slots, batch), stream);
   const size_t lds = pack_lds_bytes(2, 4, a.pk_slots, batch);
   if (a.list)
-    hipLaunchKernelGGL((pack_kernel<2, 4, 4, true>), dim3(waves), dim3(64), lds, stream, a);
+    hipLaunchKernelGGL((pack_kernel<2, 4, 3, true>), dim3(waves), dim3(64), lds, stream, a);
   else
-    hipLaunchKernelGGL((pack_kernel<2, 4, 4, false>), dim3(waves), dim3(64), lds, stream, a);
+    hipLaunchKernelGGL((pack_kernel<2, 4, 3, false>), dim3(waves), dim3(64), lds, stream, a);
   return hipGetLastError();
 }
 
