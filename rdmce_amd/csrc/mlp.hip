@@ -114,116 +114,204 @@ __global__ __launch_bounds__(256) void forward_kernel(const float *params, const
   out[r] = forward_one(q, X + r * kFeat, xn, h1, h2);
 }
 
-// Partial gradient of the mean squared error over samples idx[0 .. count)
-// (scaled by 1/count): block b takes samples [b*kRows, (b+1)*kRows), one per
-// thread; the activations and back-propagated errors of its samples are
-// staged in LDS and every gradient entry is then a dot product over the
-// block's samples, summed in sample order (deterministic, no atomics).
+// One training step's gradient, and before it, when `apply` names one, the
+// reduction and Adam update of the previous step.
+//
+// Gradient of the mean squared error over samples idx[0 .. count) (scaled by
+// 1/count): block b takes samples [b*kRows, (b+1)*kRows).  Wave w computes
+// hidden units 2w and 2w+1 of every sample (lane = sample, weights broadcast),
+// the activations and back-propagated errors are staged in LDS, and each
+// gradient entry is a dot product over the block's samples by one thread,
+// summed in sample order; the blocks' partial gradients are summed in block
+// order (deterministic, no atomics).  Every sum runs in the order it had when
+// one thread computed a whole sample, so the results are the same bits.
+//
+// Update: each block sums the previous step's partials and updates its own
+// copy of the weights in LDS (the same arithmetic in each), block 0 stores
+// them; read and written state alternate between two buffers.  That leaves
+// one launch a step instead of three.
+//
+// What bounds it: latency - a step of 1,024 samples is 8 MFLOP in 16 blocks.
+// One wave per block (64 threads, a sample each, then 21 entries of 64 terms
+// each) took 55 us + 5.6 us reduction + 5.1 us Adam a step; see kFusedBlocks
+// for the times of this form.
 constexpr int kRows = 64;
+constexpr int kStep = 1024;            // threads: 16 waves, two hidden units each
+constexpr int kPad = kRows + 4;        // LDS row of one unit over the samples: 16-byte reads without bank conflicts
+static_assert(kH1 == 32 && kH2 == 32 && kFeat == 8, "the thread mapping below");
+constexpr int oW1 = 0, ob1 = oW1 + kFeat * kH1, oW2 = ob1 + kH1, ob2 = oW2 + kH1 * kH2, oW3 = ob2 + kH2, ob3 = oW3 + kH2;
 
-__global__ __launch_bounds__(kRows) void backward_partial_kernel(const float *params, const float *X, const float *Y,
-                                                                 const uint32_t *idx, uint64_t count, float scale,
-                                                                 float *partial, float *loss_partial) {
-  __shared__ float sp[kParamFloats];
-  __shared__ float s_xn[kRows * kFeat], s_h1[kRows * kH1], s_h2[kRows * kH2];
-  __shared__ float s_d1[kRows * kH1], s_d2[kRows * kH2], s_dy[kRows], s_loss[kRows];
-  for (int i = threadIdx.x; i < kParamFloats; i += blockDim.x) sp[i] = params[i];
-  __syncthreads();
-  const Params q = params_at(sp);
-  const int t = threadIdx.x;
-  const uint64_t si = (uint64_t)blockIdx.x * kRows + t;
-  float xn[kFeat], h1[kH1], h2[kH2], d1[kH1], d2[kH2];
-  float dy = 0.f, lossv = 0.f;
-  for (int i = 0; i < kFeat; ++i) xn[i] = 0.f;
-  for (int i = 0; i < kH1; ++i) h1[i] = d1[i] = 0.f;
-  for (int i = 0; i < kH2; ++i) h2[i] = d2[i] = 0.f;
-  if (si < count) {
-    const uint64_t r = idx ? idx[si] : si;
-    float y = forward_one(q, X + r * kFeat, xn, h1, h2);
-    float d = y - Y[r];
-    lossv = d * d;
-    dy = 2.f * d * scale;
-#pragma unroll
-    for (int j = 0; j < kH2; ++j) d2[j] = h2[j] > 0.f ? dy * q.W3[j] : 0.f;
-#pragma unroll
-    for (int i = 0; i < kH1; ++i) {
-      float acc = 0.f;
-#pragma unroll
-      for (int j = 0; j < kH2; ++j) acc = fmaf(q.W2[i * kH2 + j], d2[j], acc);
-      d1[i] = h1[i] > 0.f ? acc : 0.f;
-    }
-  }
-  for (int i = 0; i < kFeat; ++i) s_xn[t * kFeat + i] = xn[i];
-  for (int i = 0; i < kH1; ++i) {
-    s_h1[t * kH1 + i] = h1[i];
-    s_d1[t * kH1 + i] = d1[i];
-  }
-  for (int i = 0; i < kH2; ++i) {
-    s_h2[t * kH2 + i] = h2[i];
-    s_d2[t * kH2 + i] = d2[i];
-  }
-  s_dy[t] = dy;
-  s_loss[t] = lossv;
-  __syncthreads();
-  float *out = partial + (uint64_t)blockIdx.x * kTrainFloats;
-  constexpr int oW1 = 0, ob1 = oW1 + kFeat * kH1, oW2 = ob1 + kH1, ob2 = oW2 + kH1 * kH2, oW3 = ob2 + kH2,
-                ob3 = oW3 + kH2;
-  for (int e = t; e < kTrainFloats; e += kRows) {
-    float acc = 0.f;
-    if (e < ob1) {
-      const int i = (e - oW1) / kH1, j = (e - oW1) % kH1;
-      for (int s = 0; s < kRows; ++s) acc = fmaf(s_xn[s * kFeat + i], s_d1[s * kH1 + j], acc);
-    } else if (e < oW2) {
-      const int j = e - ob1;
-      for (int s = 0; s < kRows; ++s) acc += s_d1[s * kH1 + j];
-    } else if (e < ob2) {
-      const int i = (e - oW2) / kH2, j = (e - oW2) % kH2;
-      for (int s = 0; s < kRows; ++s) acc = fmaf(s_h1[s * kH1 + i], s_d2[s * kH2 + j], acc);
-    } else if (e < oW3) {
-      const int j = e - ob2;
-      for (int s = 0; s < kRows; ++s) acc += s_d2[s * kH2 + j];
-    } else if (e < ob3) {
-      const int i = e - oW3;
-      for (int s = 0; s < kRows; ++s) acc = fmaf(s_dy[s], s_h2[s * kH2 + i], acc);
-    } else {
-      for (int s = 0; s < kRows; ++s) acc += s_dy[s];
-    }
-    out[e] = acc;
-  }
-  if (t == 0) {
-    float sum = 0.f;
-    for (int s = 0; s < kRows; ++s) sum += s_loss[s];
-    loss_partial[blockIdx.x] = sum;
-  }
+// Adam (Kingma & Ba 2015) for one parameter.
+__device__ __forceinline__ void adam_one(float &p, float g, float &m, float &v, const AdamStep &a) {
+  m = a.b1 * m + (1.f - a.b1) * g;
+  v = a.b2 * v + (1.f - a.b2) * g * g;
+  p -= a.lr * (m / a.bc1) / (sqrtf(v / a.bc2) + a.eps);
 }
 
+// Sum over s of x[s] * y[s], s ascending.
+__device__ __forceinline__ float dot_rows(const float *x, const float *y) {
+  float acc = 0.f;
+#pragma unroll
+  for (int s = 0; s < kRows; s += 4) {
+    const float4 a = *(const float4 *)(x + s), b = *(const float4 *)(y + s);
+    acc = fmaf(a.x, b.x, acc);
+    acc = fmaf(a.y, b.y, acc);
+    acc = fmaf(a.z, b.z, acc);
+    acc = fmaf(a.w, b.w, acc);
+  }
+  return acc;
+}
+__device__ __forceinline__ float sum_rows(const float *x) {
+  float acc = 0.f;
+#pragma unroll
+  for (int s = 0; s < kRows; s += 4) {
+    const float4 a = *(const float4 *)(x + s);
+    acc += a.x;
+    acc += a.y;
+    acc += a.z;
+    acc += a.w;
+  }
+  return acc;
+}
+
+__global__ __launch_bounds__(kStep) void step_kernel(const float *params, const float *X, const float *Y,
+                                                     const uint32_t *idx, uint64_t count, float scale, float *partial,
+                                                     float *loss_partial, AdamStep ap) {
+  __shared__ float sp[kParamFloats];
+  __shared__ __align__(16) float s_xn[kFeat * kPad], s_h1[kH1 * kPad], s_h2[kH2 * kPad], s_d1[kH1 * kPad],
+      s_d2[kH2 * kPad], s_dy[kPad], s_loss[kPad];
+  const int t = threadIdx.x, l = t & 63, wv = t >> 6;
+  for (int i = t; i < kParamFloats; i += kStep) {
+    float p = params[i];
+    if (ap.blocks && i < kTrainFloats) {
+      float g = 0.f;
+#pragma unroll 8
+      for (uint32_t b = 0; b < ap.blocks; ++b) g += ap.partial[(uint64_t)b * kTrainFloats + i];
+      float m = ap.m_in[i], v = ap.v_in[i];
+      adam_one(p, g, m, v, ap);
+      if (blockIdx.x == 0) {
+        ap.m_out[i] = m;
+        ap.v_out[i] = v;
+      }
+    }
+    sp[i] = p;
+    if (ap.blocks && blockIdx.x == 0) ap.p_out[i] = p;
+  }
+  if (ap.blocks && blockIdx.x == 0 && t == kStep - 1) {
+    float sum = 0.f;
+    for (uint32_t b = 0; b < ap.blocks; ++b) sum += ap.loss_partial[b];
+    *ap.loss = sum;
+  }
+  const uint64_t si = (uint64_t)blockIdx.x * kRows + l;
+  const bool live = si < count;
+  const uint64_t r = live ? (idx ? idx[si] : si) : 0;
+  const float target = live ? Y[r] : 0.f;
+  __syncthreads();
+  const Params q = params_at(sp);
+  if (wv < kFeat) s_xn[wv * kPad + l] = live ? (X[r * kFeat + wv] - q.mean[wv]) * q.istd[wv] : 0.f;
+  __syncthreads();
+  const int u0 = 2 * wv, u1 = u0 + 1;
+  {
+    float a0 = q.b1[u0], a1 = q.b1[u1];
+#pragma unroll
+    for (int i = 0; i < kFeat; ++i) {
+      const float x = s_xn[i * kPad + l];
+      a0 = fmaf(x, q.W1[i * kH1 + u0], a0);
+      a1 = fmaf(x, q.W1[i * kH1 + u1], a1);
+    }
+    s_h1[u0 * kPad + l] = live && a0 > 0.f ? a0 : 0.f;
+    s_h1[u1 * kPad + l] = live && a1 > 0.f ? a1 : 0.f;
+  }
+  __syncthreads();
+  {
+    float a0 = q.b2[u0], a1 = q.b2[u1];
+#pragma unroll
+    for (int i = 0; i < kH1; ++i) {
+      const float x = s_h1[i * kPad + l];
+      a0 = fmaf(x, q.W2[i * kH2 + u0], a0);
+      a1 = fmaf(x, q.W2[i * kH2 + u1], a1);
+    }
+    s_h2[u0 * kPad + l] = live && a0 > 0.f ? a0 : 0.f;
+    s_h2[u1 * kPad + l] = live && a1 > 0.f ? a1 : 0.f;
+  }
+  __syncthreads();
+  float y = q.b3[0];  // every wave: the errors need no exchange
+#pragma unroll
+  for (int i = 0; i < kH2; ++i) y = fmaf(s_h2[i * kPad + l], q.W3[i], y);
+  const float d = live ? y - target : 0.f;
+  const float dy = live ? 2.f * d * scale : 0.f;
+  s_d2[u0 * kPad + l] = s_h2[u0 * kPad + l] > 0.f ? dy * q.W3[u0] : 0.f;
+  s_d2[u1 * kPad + l] = s_h2[u1 * kPad + l] > 0.f ? dy * q.W3[u1] : 0.f;
+  if (wv == 0) {
+    s_dy[l] = dy;
+    s_loss[l] = d * d;
+  }
+  __syncthreads();
+  {
+    float a0 = 0.f, a1 = 0.f;
+#pragma unroll
+    for (int j = 0; j < kH2; ++j) {
+      const float e = s_d2[j * kPad + l];
+      a0 = fmaf(q.W2[u0 * kH2 + j], e, a0);
+      a1 = fmaf(q.W2[u1 * kH2 + j], e, a1);
+    }
+    s_d1[u0 * kPad + l] = s_h1[u0 * kPad + l] > 0.f ? a0 : 0.f;
+    s_d1[u1 * kPad + l] = s_h1[u1 * kPad + l] > 0.f ? a1 : 0.f;
+  }
+  __syncthreads();
+  float *out = partial + (uint64_t)blockIdx.x * kTrainFloats;
+  out[oW2 + t] = dot_rows(s_h1 + (t / kH2) * kPad, s_d2 + (t % kH2) * kPad);  // kStep entries
+  if (t < kFeat * kH1)
+    out[oW1 + t] = dot_rows(s_xn + (t / kH1) * kPad, s_d1 + (t % kH1) * kPad);
+  else if (t < kFeat * kH1 + kH1)
+    out[ob1 + t - kFeat * kH1] = sum_rows(s_d1 + (t - kFeat * kH1) * kPad);
+  else if (t < kFeat * kH1 + kH1 + kH2)
+    out[ob2 + t - kFeat * kH1 - kH1] = sum_rows(s_d2 + (t - kFeat * kH1 - kH1) * kPad);
+  else if (t < kFeat * kH1 + kH1 + 2 * kH2)
+    out[oW3 + t - kFeat * kH1 - kH1 - kH2] = dot_rows(s_dy, s_h2 + (t - kFeat * kH1 - kH1 - kH2) * kPad);
+  else if (t == kStep - 64)
+    out[ob3] = sum_rows(s_dy);
+  else if (t == kStep - 128)
+    loss_partial[blockIdx.x] = sum_rows(s_loss);
+}
+static_assert(kH1 * kH2 == kStep, "one W2 entry per thread");
+
 // grad[i] = sum over blocks (in order) of partial[b][i].
-__global__ __launch_bounds__(256) void reduce_partials_kernel(const float *partial, uint32_t blocks, float *grad,
-                                                              const float *loss_partial, float *loss) {
+__global__ __launch_bounds__(64) void reduce_partials_kernel(const float *partial, uint32_t blocks, float *grad,
+                                                             const float *loss_partial, float *loss) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < kTrainFloats) {
     float s = 0.f;
+#pragma unroll 8
     for (uint32_t b = 0; b < blocks; ++b) s += partial[(uint64_t)b * kTrainFloats + i];
     grad[i] = s;
   }
-  if (i == 0) {
+  if (i == kTrainFloats) {
     float s = 0.f;
     for (uint32_t b = 0; b < blocks; ++b) s += loss_partial[b];
     *loss = s;
   }
 }
 
-// Adam (Kingma & Ba 2015) on the trainable prefix of params.
-__global__ __launch_bounds__(256) void adam_kernel(float *params, const float *grad, float *m, float *v, float lr,
-                                                   float b1, float b2, float eps, float bc1, float bc2) {
+// The reduction and update of a step whose next one does not do it.
+__global__ __launch_bounds__(64) void adam_kernel(const float *params, AdamStep ap) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= kTrainFloats) return;
-  float g = grad[i];
-  float mi = b1 * m[i] + (1.f - b1) * g;
-  float vi = b2 * v[i] + (1.f - b2) * g * g;
-  m[i] = mi;
-  v[i] = vi;
-  params[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+  if (i < kTrainFloats) {
+    float g = 0.f;
+#pragma unroll 8
+    for (uint32_t b = 0; b < ap.blocks; ++b) g += ap.partial[(uint64_t)b * kTrainFloats + i];
+    float p = params[i], m = ap.m_in[i], v = ap.v_in[i];
+    adam_one(p, g, m, v, ap);
+    ap.m_out[i] = m;
+    ap.v_out[i] = v;
+    ap.p_out[i] = p;
+  } else if (i < kParamFloats) {
+    ap.p_out[i] = params[i];
+  } else if (i == kParamFloats) {
+    float s = 0.f;
+    for (uint32_t b = 0; b < ap.blocks; ++b) s += ap.loss_partial[b];
+    *ap.loss = s;
+  }
 }
 
 }  // namespace
@@ -244,24 +332,35 @@ hipError_t launch_forward(const float *params, const float *X, uint64_t n, float
 
 uint32_t backward_blocks(uint64_t count) { return (uint32_t)((count + kRows - 1) / kRows); }
 
-hipError_t launch_backward(const float *params, const float *X, const float *Y, const uint32_t *idx, uint64_t count,
-                           float *partial, float *loss_partial, float *grad, float *loss, hipStream_t s) {
+hipError_t launch_step(const float *params, const float *X, const float *Y, const uint32_t *idx, uint64_t count,
+                       float *partial, float *loss_partial, const AdamStep &apply, hipStream_t s) {
   uint32_t blocks = backward_blocks(count);
   if (!blocks) return hipSuccess;
-  hipLaunchKernelGGL(backward_partial_kernel, dim3(blocks), dim3(kRows), 0, s, params, X, Y, idx, count,
-                     1.0f / (float)count, partial, loss_partial);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(reduce_partials_kernel, dim3((kTrainFloats + 255) / 256), dim3(256), 0, s, partial, blocks,
-                     grad, loss_partial, loss);
+  hipLaunchKernelGGL(step_kernel, dim3(blocks), dim3(kStep), 0, s, params, X, Y, idx, count, 1.0f / (float)count,
+                     partial, loss_partial, apply);
   return hipGetLastError();
 }
 
-hipError_t launch_adam(float *params, const float *grad, float *m, float *v, float lr, int step, hipStream_t s) {
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-  float bc1 = 1.f - powf(b1, (float)step), bc2 = 1.f - powf(b2, (float)step);
-  hipLaunchKernelGGL(adam_kernel, dim3((kTrainFloats + 255) / 256), dim3(256), 0, s, params, grad, m, v, lr, b1, b2,
-                     eps, bc1, bc2);
+hipError_t launch_reduce(const float *partial, uint32_t blocks, float *grad, const float *loss_partial, float *loss,
+                         hipStream_t s) {
+  hipLaunchKernelGGL(reduce_partials_kernel, dim3(kTrainFloats / 64 + 1), dim3(64), 0, s, partial, blocks, grad,
+                     loss_partial, loss);
+  return hipGetLastError();
+}
+
+AdamStep adam_step(float lr, int step) {
+  AdamStep a{};
+  a.lr = lr;
+  a.b1 = 0.9f;
+  a.b2 = 0.999f;
+  a.eps = 1e-8f;
+  a.bc1 = 1.f - powf(a.b1, (float)step);
+  a.bc2 = 1.f - powf(a.b2, (float)step);
+  return a;
+}
+
+hipError_t launch_adam(const float *params, const AdamStep &apply, hipStream_t s) {
+  hipLaunchKernelGGL(adam_kernel, dim3(kParamFloats / 64 + 1), dim3(64), 0, s, params, apply);
   return hipGetLastError();
 }
 

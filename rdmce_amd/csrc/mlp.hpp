@@ -18,8 +18,28 @@ hipError_t launch_features(const uint64_t *rowoff, const uint32_t *col, const ui
                            const uint64_t *roots, uint64_t n_roots, float *out, hipStream_t s);
 hipError_t launch_forward(const float *params, const float *X, uint64_t n, float *out, hipStream_t s);
 uint32_t backward_blocks(uint64_t count);
-hipError_t launch_backward(const float *params, const float *X, const float *Y, const uint32_t *idx, uint64_t count,
-                           float *partial, float *loss_partial, float *grad, float *loss, hipStream_t s);
-hipError_t launch_adam(float *params, const float *grad, float *m, float *v, float lr, int step, hipStream_t s);
+// Adam settings of one step (bias corrections of step number `step`), the
+// partial gradients it sums (`blocks` of them; 0: no update) and the state it
+// reads and writes: m, v and the parameters go to other buffers than they are
+// read from.
+struct AdamStep {
+  float lr, b1, b2, eps, bc1, bc2;
+  uint32_t blocks;
+  const float *partial, *loss_partial;
+  const float *m_in, *v_in;
+  float *m_out, *v_out, *p_out, *loss;
+};
+AdamStep adam_step(float lr, int step);
+// Up to this many blocks a step's update is done by the next step's launch,
+// which every block repeats; beyond, the repeated reads (5.5 KB per block and
+// partial) outweigh the launch they save.
+constexpr uint32_t kFusedBlocks = 32;
+// Partial gradients of one step over samples idx[0, count) (nullptr: 0 ..),
+// after the update `apply` of the parameters when it has blocks.
+hipError_t launch_step(const float *params, const float *X, const float *Y, const uint32_t *idx, uint64_t count,
+                       float *partial, float *loss_partial, const AdamStep &apply, hipStream_t s);
+hipError_t launch_reduce(const float *partial, uint32_t blocks, float *grad, const float *loss_partial, float *loss,
+                         hipStream_t s);
+hipError_t launch_adam(const float *params, const AdamStep &apply, hipStream_t s);
 
 }  // namespace rdmce

@@ -170,7 +170,8 @@ mce_status mce_cost_model_gradient(const mce_cost_model *m, int32_t device, cons
   MTRY(hipMemcpy(dp, m->params.data(), kParamFloats * 4, hipMemcpyHostToDevice));
   MTRY(hipMemcpy(dx, X, n * kFeat * 4, hipMemcpyHostToDevice));
   MTRY(hipMemcpy(dy, Y, n * 4, hipMemcpyHostToDevice));
-  MTRY(launch_backward(dp, dx, dy, nullptr, n, dpart, dlp, dg, dl, nullptr));
+  MTRY(launch_step(dp, dx, dy, nullptr, n, dpart, dlp, AdamStep{}, nullptr));
+  MTRY(launch_reduce(dpart, blocks, dg, dlp, dl, nullptr));
   MTRY(hipMemcpy(grad, dg, kTrainFloats * 4, hipMemcpyDeviceToHost));
   MTRY(hipMemcpy(loss, dl, 4, hipMemcpyDeviceToHost));
   *loss /= (float)n;
@@ -207,45 +208,67 @@ mce_status mce_cost_model_train(mce_cost_model *m, int32_t device, const float *
   if (st) return st;
   MTRY(hipSetDevice(device));
   DevBufs d;
-  float *dp, *dx, *dy, *dpart, *dlp, *dg, *dl, *dm, *dv;
+  float *dp[2], *dm[2], *dv[2], *dpart[2], *dlp[2], *dx, *dy, *dl;
   uint32_t *didx;
-  uint32_t blocks = backward_blocks(batch);
-  MTRY(d.alloc(&dp, kParamFloats));
+  const uint32_t blocks = backward_blocks(std::min<uint64_t>(batch, n));
+  const uint64_t steps_per_epoch = (n + batch - 1) / batch;
+  for (int k = 0; k < 2; ++k) {  // state read by a step and written by it
+    MTRY(d.alloc(&dp[k], kParamFloats));
+    MTRY(d.alloc(&dm[k], kTrainFloats));
+    MTRY(d.alloc(&dv[k], kTrainFloats));
+    MTRY(d.alloc(&dpart[k], (uint64_t)blocks * kTrainFloats));
+    MTRY(d.alloc(&dlp[k], blocks));
+  }
   MTRY(d.alloc(&dx, n * kFeat));
   MTRY(d.alloc(&dy, n));
   MTRY(d.alloc(&didx, n));
-  MTRY(d.alloc(&dpart, (uint64_t)blocks * kTrainFloats));
-  MTRY(d.alloc(&dlp, blocks));
-  MTRY(d.alloc(&dg, kTrainFloats));
-  const uint64_t steps_per_epoch = (n + batch - 1) / batch;
   MTRY(d.alloc(&dl, steps_per_epoch));
-  MTRY(d.alloc(&dm, kTrainFloats));
-  MTRY(d.alloc(&dv, kTrainFloats));
-  MTRY(hipMemcpy(dp, m->params.data(), kParamFloats * 4, hipMemcpyHostToDevice));
+  MTRY(hipMemcpy(dp[0], m->params.data(), kParamFloats * 4, hipMemcpyHostToDevice));
   MTRY(hipMemcpy(dx, X, n * kFeat * 4, hipMemcpyHostToDevice));
   MTRY(hipMemcpy(dy, Y, n * 4, hipMemcpyHostToDevice));
-  MTRY(hipMemset(dm, 0, kTrainFloats * 4));
-  MTRY(hipMemset(dv, 0, kTrainFloats * 4));
+  MTRY(hipMemset(dm[0], 0, kTrainFloats * 4));
+  MTRY(hipMemset(dv[0], 0, kTrainFloats * 4));
   std::vector<uint32_t> idx(n);
-  int step = 0;
-  double epoch_loss = 0;
+  int step = 0, cur = 0;  // cur: which of the two buffers holds the newest state
+  AdamStep pend{};        // the newest step's update, not yet applied
+  auto settle = [&]() -> hipError_t {  // apply it on its own
+    if (!pend.blocks) return hipSuccess;
+    hipError_t e = launch_adam(dp[cur], pend, nullptr);
+    cur ^= 1;
+    pend = AdamStep{};
+    return e;
+  };
   for (uint32_t ep = 0; ep < epochs; ++ep) {
+    // (shuffled while the device works on the epoch before)
     for (uint64_t i = 0; i < n; ++i) idx[i] = (uint32_t)i;
     Xoshiro256ss rng(stream_seed(seed, ep));
     for (uint64_t i = n - 1; i > 0; --i) std::swap(idx[i], idx[rng.next_below(i + 1)]);
     MTRY(hipMemcpy(didx, idx.data(), n * 4, hipMemcpyHostToDevice));
-    epoch_loss = 0;
     for (uint64_t b = 0, k = 0; b < n; b += batch, ++k) {
       uint64_t cnt = std::min<uint64_t>(batch, n - b);
-      MTRY(launch_backward(dp, dx, dy, didx + b, cnt, dpart, dlp, dg, dl + k, nullptr));
-      MTRY(launch_adam(dp, dg, dm, dv, lr, ++step, nullptr));
+      const int part = step & 1;
+      MTRY(launch_step(dp[cur], dx, dy, didx + b, cnt, dpart[part], dlp[part], pend, nullptr));
+      if (pend.blocks) cur ^= 1;
+      pend = adam_step(lr, ++step);
+      pend.blocks = backward_blocks(cnt);
+      pend.partial = dpart[part];
+      pend.loss_partial = dlp[part];
+      pend.m_in = dm[cur];
+      pend.v_in = dv[cur];
+      pend.m_out = dm[cur ^ 1];
+      pend.v_out = dv[cur ^ 1];
+      pend.p_out = dp[cur ^ 1];
+      pend.loss = dl + k;
+      if (pend.blocks > kFusedBlocks) MTRY(settle());
     }
-    // per-step loss sums of this epoch (unscaled squared errors)
-    std::vector<float> ls(steps_per_epoch);
-    MTRY(hipMemcpy(ls.data(), dl, steps_per_epoch * 4, hipMemcpyDeviceToHost));
-    for (float l : ls) epoch_loss += l;
   }
-  MTRY(hipMemcpy(m->params.data(), dp, kTrainFloats * 4, hipMemcpyDeviceToHost));
+  MTRY(settle());
+  // per-step loss sums of the last epoch (unscaled squared errors)
+  double epoch_loss = 0;
+  std::vector<float> ls(steps_per_epoch);
+  MTRY(hipMemcpy(ls.data(), dl, steps_per_epoch * 4, hipMemcpyDeviceToHost));
+  for (float l : ls) epoch_loss += l;
+  MTRY(hipMemcpy(m->params.data(), dp[cur], kTrainFloats * 4, hipMemcpyDeviceToHost));
   if (final_loss) *final_loss = (float)(epoch_loss / (double)n);
   for (float v : m->params)
     if (!std::isfinite(v)) return mfail(MCE_ERR_INTERNAL, "training diverged (non-finite weights)");
