@@ -62,7 +62,6 @@ extern __shared__ uint64_t lds_dyn[];
 namespace rdmce {
 namespace {
 
-constexpr uint32_t kRecRoot = 1u << 24;  // meta flag: the record's one task is its root's top node
 // Passes between looks for idle waves (a power of two; a pass takes 10 - 20
 // us), and pending tasks from which on a wave gives some away.  R-MAT 14 /
 // community graph, ms: looks every 4 passes 12.7 / 27.1, 8 12.5 / 24.0, 16
@@ -78,8 +77,7 @@ struct PackCfg {
   static constexpr uint32_t HS = pack_hist_words(NW);
   // record fields (each a column of pk_cap words in the wave's stack):
   // P XP V (NW each), XX (NX), key, meta, R (NW, read and written only for
-  // clique lists).  meta = end << 40 | first << 32 | root flag | slot << 16 |
-  // |R|, where the record's remaining candidates are the members of V in
+  // clique lists).  meta = end << 40 | first << 32 | slot << 16 | |R|, where the record's remaining candidates are the members of V in
   // [first, end).
   static constexpr uint32_t oP = 0, oX = NW, oV = 2 * NW, oXX = 3 * NW, oKey = 3 * NW + NX, oMeta = 3 * NW + NX + 1,
                             oR = 3 * NW + NX + 2;
@@ -223,8 +221,38 @@ __device__ __forceinline__ void pk_columns(const PackWave<NW, NX> &w, uint32_t s
   }
 }
 
+// The top node of slot s's root (R = {}, P = P0, XP = {}, XX = X0'), a row per
+// lane: its pivot is the (|P0 \ N(u)|, row) argmin over all rows.  Returns
+// false when an X0' row covers P0 (pruned: no maximal clique below), else the
+// candidates V = P0 \ N(pivot).  As a task like the others, a top node kept one
+// lane busy with up to 64 NW + 64 NX rows while the rest of its pass had a
+// few each.
+template <int NW, int NX>
+__device__ __forceinline__ bool pk_top(const PackWave<NW, NX> &w, uint32_t s, uint32_t p, uint32_t xq,
+                                       uint64_t (&V)[NW]) {
+  const uint32_t l = cold_lane();
+  const lds64 *sl = w.slot(s);
+  uint32_t best = ~0u;
+#pragma unroll
+  for (int r = 0; r < NW + NX; ++r) {
+    const uint32_t row = 64u * r + l;  // (P0 rows first, then 64 NW + x)
+    if (r < NW ? row < p : row - 64u * NW < xq) {
+      uint32_t c = p;
+#pragma unroll
+      for (int q = 0; q < NW; ++q) c -= (uint32_t)__popcll((uint64_t)sl[row * NW + q]);
+      const uint32_t k = (c << 16) | row;
+      best = k < best ? k : best;
+    }
+  }
+  best = wave_min_u32(best);
+#pragma unroll
+  for (int q = 0; q < NW; ++q)
+    V[q] = low_mask(p > 64u * q ? p - 64u * q : 0u) & ~bcast64((uint64_t)sl[(best & 0xFFFF) * NW + q]);
+  return (best >> 16) != 0;
+}
+
 // Bookkeeping of slot s once its rows, columns, label hashes (and clique-list
-// ids) are in place.
+// ids) are in place; its top node is counted.
 template <int NW, int NX>
 __device__ __forceinline__ void pk_seal(const PackWave<NW, NX> &w, uint32_t s, uint64_t p, uint64_t xq, uint64_t canon,
                                         uint64_t base_key, uint32_t base_size, uint32_t graph, uint32_t v0,
@@ -238,8 +266,8 @@ __device__ __forceinline__ void pk_seal(const PackWave<NW, NX> &w, uint32_t s, u
     *w.m(mPX, s) = p | (xq << 32);
     *w.m(mBase, s) = (uint64_t)base_size | ((uint64_t)graph << 32);
     *w.m(mV, s) = (uint64_t)v0 | ((uint64_t)v1 << 32);
-    *w.m(mNodes, s) = 0;
-    *w.m(mRefs, s) = 1;  // the root record pushed next
+    *w.m(mNodes, s) = 1;
+    *w.m(mRefs, s) = 1;  // the top node's record, pushed next
     *w.m(mCount, s) = 0;
     *w.m(mHash, s) = 0;
   }
@@ -278,12 +306,14 @@ __device__ __forceinline__ void pk_emit_base(const PackWave<NW, NX> &w, uint64_t
 }
 
 // Builds root `canon` into slot s (the whole wave).  Returns 1 when the root
-// occupies the slot, 0 when it needs no search (its 2-clique, if maximal,
-// is counted here), 2 when it is too wide for this variant (the caller hands
-// it to the next launch).
+// occupies the slot (V: its top node's candidates), 0 when it needs no search
+// (its 2-clique, if maximal, is counted here), 2 when it is too wide for this
+// variant (the caller hands it to the next launch), 3 when its top node is
+// pruned by an X0' row covering P0.  1 and 3: the caller counts the top node,
+// px = |P0| | |X0'| << 32.
 template <int NW, int NX>
 __device__ __forceinline__ uint32_t pk_build(const PackWave<NW, NX> &w, uint8_t *scratch, uint32_t s, uint64_t canon,
-                                             Acc &acc, uint64_t &cnt, uint64_t &hsh) {
+                                             Acc &acc, uint64_t &cnt, uint64_t &hsh, uint64_t (&V)[NW], uint64_t &px) {
   using C = PackCfg<NW, NX>;
   const KArgs &a = cold_args(w.a);
   const uint32_t l = cold_lane();
@@ -327,6 +357,9 @@ __device__ __forceinline__ uint32_t pk_build(const PackWave<NW, NX> &w, uint8_t 
         or64_lds(sl + C::sProw + (uint64_t)j * NW + (i >> 6), 1ull << (i & 63));
       },
       [&](uint64_t i, uint32_t wd, uint64_t bits) { or64_lds(sl + C::sXrow + (i - p) * NW + wd, bits); });
+  wave_fence();
+  px = p | (xq << 32);
+  if (!pk_top<NW, NX>(w, s, (uint32_t)p, (uint32_t)xq, V)) return 3;
   pk_columns<NW, NX>(w, s, (uint32_t)p, (uint32_t)xq);
   pk_seal<NW, NX>(w, s, p, xq, canon, sub.base_key, sub.base_size, sub.graph, sub.v0, sub.v1);
   return 1;
@@ -424,11 +457,10 @@ __device__ __forceinline__ bool pk_group_build(const KArgs &a0, uint8_t *scratch
 }
 
 // Derives edge root `canon` = (v0, u_k) of group G into slot s (the whole
-// wave).  Returns as pk_build does, or 3 when the root's top node is pruned
-// by an X0' row covering P0 (its search words in `pruned`).
+// wave).  Returns as pk_build does.
 template <int NW, int NX>
 __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const PkGroup &G, uint32_t s, uint64_t canon,
-                                              Acc &acc, uint64_t &cnt, uint64_t &hsh, uint32_t &pruned) {
+                                              Acc &acc, uint64_t &cnt, uint64_t &hsh, uint64_t (&V)[NW], uint64_t &px) {
   using C = PackCfg<NW, NX>;
   const KArgs &a = cold_args(w.a);
   const uint32_t l = cold_lane();
@@ -468,19 +500,26 @@ __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const P
     return (readlane64(xu, b - nbx) >> l) & 1;
   };
   // X0' keeps the rows with a neighbour in P0.  Row numbers go to lists in the
-  // slot's column area (rewritten below): X0' rows, then P0 rows.
+  // slot's column area (rewritten below): X0' rows, then P0 rows.  A row that
+  // covers P0 prunes the root's top node: the root is done, whatever its width.
   lds64 *sl = w.slot(s);
   ldsu32 *xl = (ldsu32 *)(sl + C::sXcol), *pl = xl + 64 * NX;
   uint32_t xq = 0;
+  bool cov = false;
   for (uint32_t b = 0; b < nb; ++b) {
     uint32_t row;
     const bool cand = candidate(b, row);
     if (__ballot(cand) == 0) continue;
-    uint64_t hit = 0;
+    uint64_t hit = 0, miss = 0;
     for (uint32_t z = kq; z < G.W0; ++z) {  // (P0 lies above u_k)
       const uint64_t mz = readlane64(pk, z);
-      if (mz && cand) hit |= G.T[(uint64_t)z * G.rp + row] & mz;
+      if (mz && cand) {
+        const uint64_t t = G.T[(uint64_t)z * G.rp + row];
+        hit |= t & mz;
+        miss |= mz & ~t;
+      }
     }
+    cov |= cand && miss == 0;
     const uint64_t m = __ballot(hit != 0);
     const uint32_t at = xq + rank_below(m);
     if (hit != 0 && at < 64u * NX) xl[at] = row;
@@ -488,27 +527,12 @@ __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const P
   }
   const uint32_t nxu = __builtin_amdgcn_readlane(wave_scan_add_u32((uint32_t)__popcll(xu)), 63);
   words_read += (uint64_t)nbx * 64 + (uint64_t)nxu * G.W0;
-  if (xq > 64u * NX) {
-    // Too many X0' rows for this variant.  When one of them covers P0, the
-    // root's top node is pruned (no maximal clique below it): one node, no
-    // slot.  Otherwise the root goes to the next launch.
-    bool cov = false;
-    for (uint32_t b = 0; b < nb; ++b) {
-      uint32_t row;
-      const bool cand = candidate(b, row);
-      uint64_t miss = 0;
-      for (uint32_t z = kq; z < G.W0; ++z) {
-        const uint64_t mz = readlane64(pk, z);
-        if (mz && cand) miss |= mz & ~G.T[(uint64_t)z * G.rp + row];
-      }
-      cov |= cand && miss == 0;
-    }
-    if (__ballot(cov) == 0) return 2;
-    words_read += (uint64_t)(G.xq0 + nxu) * G.W0;
+  px = (uint64_t)p | ((uint64_t)xq << 32);
+  if (__ballot(cov) != 0) {
     acc.build += 8 * words_read;
-    pruned = (p + xq) * ((p + 63) / 64);  // the search words of evaluating the top node
     return 3;
   }
+  if (xq > 64u * NX) return 2;
   for (uint32_t z = kq, before = 0; z < G.W0; ++z) {
     const uint64_t mz = readlane64(pk, z);
     if ((mz >> l) & 1) pl[before + rank_below(mz)] = 64 * z + l;
@@ -596,6 +620,8 @@ __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const P
   }
   words_read += (uint64_t)(p + xq) * G.W0;
   acc.build += 8 * words_read + 8ull * NW * (p + xq);
+  wave_fence();
+  pk_top<NW, NX>(w, s, p, xq, V);
   pk_seal<NW, NX>(w, s, p, xq, canon, base_key, 2, graph, G.v0, uk);
   return 1;
 }
@@ -908,13 +934,14 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
         G.lh = G.cm + G.W0;
         derive = true;
       }
-      uint32_t pruned = 0;
-      const uint32_t built = derive ? pk_derive<NW, NX>(w, G, s, canon, acc, cnt, hsh, pruned)
-                                    : pk_build<NW, NX>(w, scratch, s, canon, acc, cnt, hsh);
-      if (built == 3 && l == 0) {  // one tree node, pruned
-        ++nodes;
-        words += pruned;
-        if (a.root_nodes) atomicAdd(&a.root_nodes[canon], 1ull);
+      uint64_t topV[NW], px = 0;
+      const uint32_t built = derive ? pk_derive<NW, NX>(w, G, s, canon, acc, cnt, hsh, topV, px)
+                                    : pk_build<NW, NX>(w, scratch, s, canon, acc, cnt, hsh, topV, px);
+      if (built & 1) {  // the top node: every row scanned, and the pivot's read unless it is pruned
+        const uint32_t p = (uint32_t)px, Wr = (p + 63) / 64;
+        acc.nodes += 1;
+        acc.words += (uint64_t)(p + (uint32_t)(px >> 32) + (built == 1)) * Wr;
+        if (built == 3 && a.root_nodes && l == 0) atomicAdd(&a.root_nodes[canon], 1ull);
       }
       if (built == 2) {  // too wide for this variant: to the next launch
         if (grouped && a.wide_h) {
@@ -926,15 +953,22 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
           if (a.wide_h) a.wide_h[at] = hk;
         }
       }
-      if (built == 1) {
-        if (l == 0) {  // one task (V = {0}): the root's top node
-          for (uint32_t f = 0; f < C::RS; ++f) fld(f, top) = 0;
-          fld(C::oV, top) = 1;
-          fld(C::oMeta, top) = (1ull << 40) | ((uint64_t)s << 16) | kRecRoot;
+      if (built == 1) {  // the top node's record: lane f writes field f
+        uint64_t v = 0;
+        const uint32_t p = (uint32_t)px, xq = (uint32_t)(px >> 32);
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+          v = l == C::oP + q ? low_mask(p > 64u * q ? p - 64u * q : 0u) : v;
+          v = l == C::oV + q ? topV[q] : v;
+          pending += (uint32_t)__popcll(topV[q]);
         }
+#pragma unroll
+        for (int j = 0; j < NX; ++j) v = l == C::oXX + j ? low_mask(xq > 64u * j ? xq - 64u * j : 0u) : v;
+        v = l == C::oKey ? *w.m(mKey, s) : v;
+        v = l == C::oMeta ? ((uint64_t)(64 * NW) << 40) | ((uint64_t)s << 16) : v;
+        if (l < C::RS) fld(l, top) = v;
         wave_fence();
         ++top;
-        ++pending;
         busy |= 1u << s;
       }
     }
@@ -1021,9 +1055,9 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
       t = base + select64(rw, kk);
     }
     // A child's P | XP lies within its parent's P | XP: when no parent of
-    // this pass reaches the last word (a root's top node may), the tasks
-    // skip that word of every row they scan.
-    const bool wlast = NW == 1 || __ballot(act && ((meta & kRecRoot) || (P[NW - 1] | XP[NW - 1]) != 0)) != 0;
+    // this pass reaches the last word, the tasks skip that word of every row
+    // they scan.
+    const bool wlast = NW == 1 || __ballot(act && (P[NW - 1] | XP[NW - 1]) != 0) != 0;
     wave_fence();  // every parent is read before records are rewritten below
     if (lpart) {   // the partly taken record keeps its candidates from the (T - excl)-th on
       uint32_t kk = T - excl, base = 0;
@@ -1052,25 +1086,13 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     if (act) {
       const lds64 *sl = w.slot(s);
       const uint64_t px = *w.m(mPX, s);
-      const uint32_t p = (uint32_t)px, xq = (uint32_t)(px >> 32);
+      const uint32_t p = (uint32_t)px;
       const uint32_t Wr = (p + 63) / 64;  // the root's own width (accounting as the other kernel)
-      uint32_t rsize;
-      if (meta & kRecRoot) {  // the root's top node: R = {}, P = P0, XP = {}, XX = X0'
-#pragma unroll
-        for (int q = 0; q < NW; ++q) {
-          R[q] = 0;
-          P[q] = low_mask(p > 64u * q ? p - 64u * q : 0u);
-          XP[q] = 0;
-        }
-#pragma unroll
-        for (int j = 0; j < NX; ++j) XX[j] = low_mask(xq > 64u * j ? xq - 64u * j : 0u);
-        key = *w.m(mKey, s);
-        rsize = 0;
-      } else {
+      uint32_t rsize, xpop = 0;  // xpop: rows of the parent's XX
+      {
         // Child of candidate t: the parent's candidates below t have moved
         // from P to XP, as when the sequential search reaches t.
         const uint32_t jt = t >> 6, bt = t & 63;
-        uint32_t xpop = 0;
 #pragma unroll
         for (int q = 0; q < NW; ++q) {
           const uint64_t below = (uint32_t)q < jt ? V[q] : ((uint32_t)q == jt ? V[q] & low_mask(bt) : 0ull);
@@ -1087,87 +1109,113 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
         key += sl[C::sG + t];
         rsize = (meta & 0xFFFF) + 1;
         words += Wr;
-        // Aggressive node generation: every vertex of P' adjacent to all of
-        // P' \ {itself} moves to R; XP' and XX' keep what is adjacent to it.
-        uint32_t psz = 0;
+      }
+      // Row scans: the rows of P0 and X0' follow each other in the slot, so row
+      // r (P0 rows first, then 64 NW + x) is at r * NW.  Two rows a pass, both
+      // loads in flight before either is used; a lane goes on to its next word
+      // when one is used up, so that a pass of the wave is lost only to the
+      // lane with the most rows, not once per word.
+      auto row_pair = [&](uint64_t &m, uint32_t wb, uint64_t &b0, uint64_t &b1, uint32_t &i0, uint32_t &i1,
+                          uint64_t (&r0)[NW], uint64_t (&r1)[NW], uint32_t &c0, uint32_t &c1) {
+        b0 = m & (~m + 1);
+        m ^= b0;
+        b1 = m & (~m + 1);
+        m ^= b1;
+        i0 = wb + (uint32_t)__builtin_ctzll(b0);
+        i1 = b1 ? wb + (uint32_t)__builtin_ctzll(b1) : i0;
 #pragma unroll
-        for (int q = 0; q < NW; ++q) psz += (uint32_t)__popcll(P[q]);
-        bool anym = false;
-        if (psz > 1) {
-          words += (uint64_t)psz * Wr;
-          uint64_t mk[NW], xacc[NW];
+        for (int z = 0; z < NW; ++z) {
+          r0[z] = z + 1 < NW || wlast ? (uint64_t)sl[i0 * NW + z] : 0ull;
+          r1[z] = z + 1 < NW || wlast ? (uint64_t)sl[i1 * NW + z] : 0ull;
+        }
+        c0 = c1 = 0;
 #pragma unroll
-          for (int q = 0; q < NW; ++q) {
-            mk[q] = 0;
-            xacc[q] = ~0ull;
-          }
-#pragma unroll
-          for (int q = 0; q < NW; ++q) {
-            // two rows per pass, both loads in flight before either is used
-            for (uint64_t m = P[q]; m;) {
-              const uint64_t b0 = m & (~m + 1);
-              m ^= b0;
-              const uint64_t b1 = m & (~m + 1);
-              m ^= b1;
-              const uint32_t i0 = 64u * q + (uint32_t)__builtin_ctzll(b0);
-              const uint32_t i1 = b1 ? 64u * q + (uint32_t)__builtin_ctzll(b1) : i0;
-              uint64_t r0[NW], r1[NW];
-              uint32_t c0 = 0, c1 = 0;
-#pragma unroll
-              for (int z = 0; z < NW; ++z) {
-                r0[z] = z + 1 < NW || wlast ? (uint64_t)sl[C::sProw + i0 * NW + z] : 0ull;
-                r1[z] = z + 1 < NW || wlast ? (uint64_t)sl[C::sProw + i1 * NW + z] : 0ull;
-              }
-#pragma unroll
-              for (int z = 0; z < NW; ++z) {
-                if (z + 1 < NW || wlast) {
-                  c0 += (uint32_t)__popcll(P[z] & ~r0[z]);
-                  c1 += (uint32_t)__popcll(P[z] & ~r1[z]);
-                }
-              }
-              if (c0 == 1) {
-                mk[q] |= b0;
-#pragma unroll
-                for (int z = 0; z < NW; ++z)
-                  if (z + 1 < NW || wlast) xacc[z] &= r0[z];
-              }
-              if (b1 && c1 == 1) {
-                mk[q] |= b1;
-#pragma unroll
-                for (int z = 0; z < NW; ++z)
-                  if (z + 1 < NW || wlast) xacc[z] &= r1[z];
-              }
-            }
-          }
-          uint32_t nm = 0;
-#pragma unroll
-          for (int q = 0; q < NW; ++q) nm += (uint32_t)__popcll(mk[q]);
-          if (nm) {
-            anym = true;
-#pragma unroll
-            for (int q = 0; q < NW; ++q) {
-              R[q] |= mk[q];
-              P[q] &= ~mk[q];
-              XP[q] &= xacc[q];
-              for (uint64_t m = mk[q]; m; m &= m - 1) {
-                const uint32_t i = 64u * q + (uint32_t)__builtin_ctzll(m);
-#pragma unroll
-                for (int j = 0; j < NX; ++j) XX[j] &= sl[C::sXcol + i * NX + j];
-                key += sl[C::sG + i];
-              }
-            }
-            rsize += nm;
-            words += (uint64_t)nm * Wr;
+        for (int z = 0; z < NW; ++z) {
+          if (z + 1 < NW || wlast) {
+            c0 += (uint32_t)__popcll(P[z] & ~r0[z]);
+            c1 += (uint32_t)__popcll(P[z] & ~r1[z]);
           }
         }
-        words += (uint64_t)xpop * (anym ? Wr + 1 : 1);
+      };
+      // P' against itself: aggressive node generation moves every vertex
+      // adjacent to all of P' \ {itself} (it misses one: itself) to R, and the
+      // others' counts are those of the pivot choice - the moved vertices are
+      // adjacent to all of them, so P' without them gives the same counts.
+      uint32_t psz = 0, best = ~0u;
+#pragma unroll
+      for (int q = 0; q < NW; ++q) psz += (uint32_t)__popcll(P[q]);
+      bool anym = false;
+      if (psz == 1) {
+        uint32_t i = 0;
+#pragma unroll
+        for (int q = NW - 1; q >= 0; --q)
+          if (P[q]) i = 64u * q + (uint32_t)__builtin_ctzll(P[q]);
+        best = (1u << 16) | i;
+      } else if (psz > 1) {
+        uint64_t mk[NW], xacc[NW], nx[NW];
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+          mk[q] = 0;
+          xacc[q] = ~0ull;
+          nx[q] = P[q];
+        }
+        uint32_t wb = 0;
+        for (;;) {
+          uint64_t left = 0;
+#pragma unroll
+          for (int q = 0; q < NW; ++q) left |= nx[q];
+          if (left == 0) break;
+          if (NW > 1 && nx[0] == 0) {
+#pragma unroll
+            for (int q = 0; q + 1 < NW; ++q) nx[q] = nx[q + 1];
+            nx[NW - 1] = 0;
+            wb += 64;
+          }
+          uint64_t b0, b1, r0[NW], r1[NW];
+          uint32_t i0, i1, c0, c1;
+          row_pair(nx[0], wb, b0, b1, i0, i1, r0, r1, c0, c1);
+          const bool mv0 = c0 == 1, mv1 = c1 == 1 && b1;
+          if (mv0 || mv1) {
+#pragma unroll
+            for (int q = 0; q < NW; ++q)
+              mk[q] |= wb == 64u * q ? (mv0 ? b0 : 0ull) | (mv1 ? b1 : 0ull) : 0ull;
+#pragma unroll
+            for (int z = 0; z < NW; ++z)
+              if (z + 1 < NW || wlast) xacc[z] &= (mv0 ? r0[z] : ~0ull) & (mv1 ? r1[z] : ~0ull);
+          }
+          const uint32_t k0 = mv0 ? ~0u : (c0 << 16) | i0, k1 = mv1 ? ~0u : (c1 << 16) | i1;
+          best = k0 < best ? k0 : best;
+          best = k1 < best && b1 ? k1 : best;
+        }
+        words += (uint64_t)psz * Wr;
+        uint32_t nm = 0;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) nm += (uint32_t)__popcll(mk[q]);
+        if (nm) {
+          anym = true;
+#pragma unroll
+          for (int q = 0; q < NW; ++q) {
+            R[q] |= mk[q];
+            P[q] &= ~mk[q];
+            XP[q] &= xacc[q];
+            for (uint64_t m = mk[q]; m; m &= m - 1) {
+              const uint32_t i = 64u * q + (uint32_t)__builtin_ctzll(m);
+#pragma unroll
+              for (int j = 0; j < NX; ++j) XX[j] &= sl[C::sXcol + i * NX + j];
+              key += sl[C::sG + i];
+            }
+          }
+          rsize += nm;
+          words += (uint64_t)nm * Wr;
+          psz -= nm;
+        }
       }
+      words += (uint64_t)xpop * (anym ? Wr + 1 : 1);
       // Evaluate the node.
-      uint32_t psz = 0, cw = 0, xw = 0;
+      uint32_t cw = 0, xw = 0;
       uint64_t xany = 0;
 #pragma unroll
       for (int q = 0; q < NW; ++q) {
-        psz += (uint32_t)__popcll(P[q]);
         cw += (uint32_t)__popcll(P[q] | XP[q]);
         xany |= XP[q];
       }
@@ -1182,47 +1230,40 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
         if (xany == 0) pk_emit<NW, NX, LISTS>(w, s, (uint32_t)*w.m(mBase, s) + rsize, key, R, cnt, hsh);
       } else {
         words += (uint64_t)(cw + xw) * Wr;
-        // pivot: (|P' \ N(u)|, row) argmin; rows of P0 first, then X0'
-        uint32_t best = ~0u;
+        // pivot: (|P' \ N(u)|, row) argmin over P' (above), then XP' and XX';
+        // an excluded row that covers P' ends the scan (the minimum does not
+        // depend on the order rows are visited in).
+        uint64_t nx[NW + NX];
+#pragma unroll
+        for (int q = 0; q < NW; ++q) nx[q] = XP[q];
+#pragma unroll
+        for (int j = 0; j < NX; ++j) nx[NW + j] = XX[j];
+        uint32_t wb = 0;
         bool zero = false;
-        // Rows two per pass (both loads in flight first); the minimum does
-        // not depend on the order rows are visited in.
-        auto scan = [&](uint64_t m, uint32_t rbase, uint32_t kbase) {
-          while (m && !zero) {
-            const uint64_t b0 = m & (~m + 1);
-            m ^= b0;
-            const uint64_t b1 = m & (~m + 1);
-            m ^= b1;
-            const uint32_t u0 = (uint32_t)__builtin_ctzll(b0);
-            const uint32_t u1 = b1 ? (uint32_t)__builtin_ctzll(b1) : u0;
-            uint64_t r0[NW], r1[NW];
+        for (;;) {
+          uint64_t left = 0;
 #pragma unroll
-            for (int z = 0; z < NW; ++z) {
-              r0[z] = z + 1 < NW || wlast ? (uint64_t)sl[rbase + u0 * NW + z] : 0ull;
-              r1[z] = z + 1 < NW || wlast ? (uint64_t)sl[rbase + u1 * NW + z] : 0ull;
-            }
-            uint32_t c0 = 0, c1 = 0;
+          for (int q = 0; q < NW + NX; ++q) left |= nx[q];
+          if (left == 0 || zero) break;
+          if (nx[0] == 0) {
 #pragma unroll
-            for (int z = 0; z < NW; ++z) {
-              if (z + 1 < NW || wlast) {
-                c0 += (uint32_t)__popcll(P[z] & ~r0[z]);
-                c1 += (uint32_t)__popcll(P[z] & ~r1[z]);
-              }
-            }
-            const uint32_t k0 = (c0 << 16) | (kbase + u0), k1 = (c1 << 16) | (kbase + u1);
+            for (int q = 0; q + 1 < NW + NX; ++q) nx[q] = nx[q + 1];
+            nx[NW + NX - 1] = 0;
+            wb += 64;
+          }
+          if (nx[0]) {
+            uint64_t b0, b1, r0[NW], r1[NW];
+            uint32_t i0, i1, c0, c1;
+            row_pair(nx[0], wb, b0, b1, i0, i1, r0, r1, c0, c1);
+            const uint32_t k0 = (c0 << 16) | i0, k1 = (c1 << 16) | i1;
             best = k0 < best ? k0 : best;
             best = k1 < best ? k1 : best;
             zero = c0 == 0 || c1 == 0;
           }
-        };
-#pragma unroll
-        for (int q = 0; q < NW; ++q) scan(P[q] | XP[q], C::sProw + 64u * q * NW, 64u * q);
-#pragma unroll
-        for (int j = 0; j < NX; ++j) scan(XX[j], C::sXrow + 64u * j * NW, p + 64u * j);
+        }
         if (!zero) {  // else an excluded row covers P': no maximal clique below
           words += Wr;
-          const uint32_t piv = best & 0xFFFF;
-          const lds64 *pr = piv < p ? sl + C::sProw + piv * NW : sl + C::sXrow + (piv - p) * NW;
+          const lds64 *pr = sl + (best & 0xFFFF) * NW;
 #pragma unroll
           for (int q = 0; q < NW; ++q) V[q] = P[q] & ~(uint64_t)pr[q];
           branch = true;
@@ -1279,8 +1320,8 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
   // Exit: the wave's sums.
   acc.count = wave_sum64(cnt);
   acc.hash = wave_sum64(hsh);
-  acc.words = wave_sum64(words);
-  acc.nodes = wave_sum64(nodes);
+  acc.words += wave_sum64(words);
+  acc.nodes += wave_sum64(nodes);
   acc.build += 4 * wave_sum64(acc.scan);
   wave_fence();
   flush_sums(a, w.me, acc, w.L.hist);
