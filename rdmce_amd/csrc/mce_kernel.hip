@@ -220,10 +220,18 @@ __device__ __forceinline__ Lvl make_child(const Sub &s, const Lvl &par, XxP par_
 
 // Tries to take one task from record r (lane 0 only).  Returns the task
 // index or -1; *last is set when it was the final task of the publication.
-__device__ __forceinline__ int claim_task(ShareRec *r, bool *last) {
+// A device-scope release writes back an L2 and an acquire invalidates one, for
+// every wave of the XCD, so sharing uses them only where data passes: the
+// publisher's release and the thief's acquire here.  The publisher claiming
+// its own tasks, and what only says that reading is over (done_reading), go
+// without: 5 of them per task made vertex roots of a 20k-vertex community graph
+// take 14.4 ms against 11.5, G(300, 0.4) 1.70 against 1.03.
+__device__ __forceinline__ int claim_task(ShareRec *r, bool *last, bool own) {
   unsigned long long c = ld_relaxed(&r->ctl);
   if ((c & 0xFFFF) >= ((c >> 16) & 0xFFFF)) return -1;
-  unsigned long long old = __hip_atomic_fetch_add(&r->ctl, 1ull, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned long long old =
+      own ? __hip_atomic_fetch_add(&r->ctl, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+          : __hip_atomic_fetch_add(&r->ctl, 1ull, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
   uint32_t next = (uint32_t)(old & 0xFFFF), ntot = (uint32_t)((old >> 16) & 0xFFFF);
   if (next >= ntot) return -1;
   *last = next + 1 == ntot;
@@ -256,6 +264,15 @@ __device__ __forceinline__ Lvl materialize(const Sub &s, SnapP snap, uint32_t id
   par.pk &= ~below;
   par.xpk |= below;
   return make_child(s, par, snap + 4 * W, jt * 64 + bt, out, bm, gP, acc);
+}
+
+// Counts one reader less, once this wave's loads have returned.
+__device__ __forceinline__ void done_reading(unsigned int *n) {
+#ifdef __AMDGCN__
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+#endif
+  wave_fence();
+  if (lane() == 0) __hip_atomic_fetch_sub(n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void publish_bit(const KArgs &a, uint32_t w, bool set) {
@@ -366,14 +383,14 @@ __device__ __forceinline__ uint64_t run_dfs(const KArgs &a, const Sub &s, BmP bm
         // The parent level is frozen: serve its remaining tasks.
         int idx = -1;
         bool last = false;
-        if (l == 0) idx = claim_task(my, &last);
+        if (l == 0) idx = claim_task(my, &last, true);
         idx = (int)bcast32((uint32_t)idx);
         if (idx < 0) {
           // All tasks taken; wait until the takers have copied their part of
           // the frozen levels out.
           if (l == 0) {
             uint32_t n = 1;
-            while (ld_acquire(&my->pending) != 0) {
+            while (ld_relaxed(&my->pending) != 0) {
               nap(n);
               n = n < 8 ? n * 2 : 8;
             }
@@ -385,7 +402,7 @@ __device__ __forceinline__ uint64_t run_dfs(const KArgs &a, const Sub &s, BmP bm
         ++acc.owner;
         level = S + 1;
         L = materialize(s, stk + (uint64_t)S * LS, (uint32_t)idx, stk + (uint64_t)level * LS, bm, gP, acc);
-        if (l == 0) __hip_atomic_fetch_sub(&my->pending, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        done_reading(&my->pending);
         Lstar = Lstar < S ? Lstar : S;
         task = true;
         break;
@@ -755,14 +772,14 @@ __device__ __forceinline__ uint64_t run_dfsr(const KArgs &a, const Sub &s, const
         // The parent level is frozen: serve its remaining tasks.
         int idx = -1;
         bool last = false;
-        if (l == 0) idx = claim_task(my, &last);
+        if (l == 0) idx = claim_task(my, &last, true);
         idx = (int)bcast32((uint32_t)idx);
         if (idx < 0) {
           // All tasks taken; wait until the takers have copied their part of
           // the frozen levels out.
           if (l == 0) {
             uint32_t n = 1;
-            while (ld_acquire(&my->pending) != 0) {
+            while (ld_relaxed(&my->pending) != 0) {
               nap(n);
               n = n < 8 ? n * 2 : 8;
             }
@@ -794,7 +811,7 @@ __device__ __forceinline__ uint64_t run_dfsr(const KArgs &a, const Sub &s, const
           L.p[k] &= ~below;
           L.x[k] |= below;
         }
-        if (l == 0) __hip_atomic_fetch_sub(&my->pending, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        done_reading(&my->pending);
         Lstar = Lstar < S ? Lstar : S;
         level = S;
         task = true;
@@ -1148,7 +1165,7 @@ __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk
   ShareRec *r = a.recs + victim;
   int idx = -1;
   bool last = false;
-  if (l == 0) idx = claim_task(r, &last);
+  if (l == 0) idx = claim_task(r, &last, false);
   idx = (int)bcast32((uint32_t)idx);
   if (idx < 0) return false;
   if (l == 0 && last) publish_bit(a, (uint32_t)victim, false);
@@ -1175,7 +1192,7 @@ __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk
   } else {
     materialize(s, snap, (uint32_t)idx, stk_g, s.bm, s.gP, acc);
   }
-  if (l == 0) __hip_atomic_fetch_sub(&r->pending, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  done_reading(&r->pending);
   uint64_t t0 = clock64();
   bool pub_unused = false;
   uint64_t nodes;
@@ -1190,8 +1207,8 @@ __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk
   if (l == 0) {
     if (a.root_nodes && nodes) atomicAdd(&a.root_nodes[s.canon], (unsigned long long)nodes);
     if (a.root_cycles) atomicAdd(&a.root_cycles[s.canon], (unsigned long long)(clock64() - t0));
-    __hip_atomic_fetch_sub(&a.users[s.bm_owner], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
   }
+  done_reading(&a.users[s.bm_owner]);
   acc.nodes += nodes;
   ++acc.shared;
   return true;
@@ -1233,10 +1250,7 @@ __device__ __forceinline__ void mce_main(const KArgs &a) {
       if (published) {
         if (l == 0) free_slot = ld_relaxed(&a.users[me]) == 0;
         free_slot = bcast32(free_slot);
-        if (free_slot) {
-          if (l == 0) (void)ld_acquire(&a.users[me]);  // order our rebuild after their reads
-          published = false;
-        }
+        published = !free_slot;
       }
       if (free_slot) {
         uint64_t i = 0;
