@@ -168,6 +168,7 @@ struct Acc {
   unsigned long long words;
   unsigned long long build;
   unsigned long long scan;  // per lane: adjacency entries of the bitmap rows' runs
+  unsigned long long lwords;  // per lane: more of `words`
   unsigned long long nodes;
   uint32_t shared, published, owner;  // sharing: see Sum
 };
@@ -340,7 +341,7 @@ __device__ __forceinline__ void or64_lds(lds64 *p, uint64_t v) {
 //   X = N(v0) & N-(v1) below v1 (only its emptiness when P is empty).
 __device__ __forceinline__ uint32_t root_lists(const KArgs &a, uint64_t canon, uint32_t *Pl, uint64_t ccap, Sub &s,
                                                uint64_t &p, uint64_t &x, Acc &acc) {
-  const uint32_t l = lane();
+  const uint32_t l = cold_lane();
   const uint64_t desc = bcast64(a.roots[canon]);
   const uint32_t *col = a.col;
   p = 0;
@@ -428,7 +429,7 @@ __device__ __forceinline__ uint32_t root_lists(const KArgs &a, uint64_t canon, u
 // (graph_gpu.cuh:90-106 drops those rows after building them).
 __device__ __forceinline__ uint64_t compact_x(const KArgs &a, const uint32_t *P, uint64_t p, uint32_t *X, uint64_t x,
                                               uint32_t above) {
-  const uint32_t l = lane();
+  const uint32_t l = cold_lane();
   const uint32_t *col = a.col;
   uint64_t xq = 0;
   for (uint64_t base = 0; base < x; base += 64) {
@@ -467,7 +468,7 @@ __device__ __forceinline__ uint64_t compact_x(const KArgs &a, const uint32_t *P,
 template <class PP, class XW>
 __device__ __forceinline__ uint64_t match_rows(const KArgs &a, const uint32_t *P, uint64_t p, const uint32_t *X,
                                                uint64_t rows, uint32_t above, PP pp, XW xw, ldsu32 *claim = nullptr) {
-  const uint32_t l = lane();
+  const uint32_t l = cold_lane();
   const uint32_t *col = a.col;
   uint64_t scanned = 0;
   const uint32_t g = rows <= 16 ? 4u : (rows <= 32 ? 2u : 1u);

@@ -991,7 +991,7 @@ __device__ __forceinline__ uint32_t p0_degeneracy(const lds64 *T, uint32_t rp, u
 __device__ __forceinline__ uint64_t solve_root(const KArgs &a, uint8_t *slot, uint64_t *stk_g, lds64 *lds, uint32_t me,
                                uint64_t canon, Acc &acc, ldsu64 *s_hist, bool &published,
                                bool eager) {
-  const uint32_t l = lane();
+  const uint32_t l = cold_lane();
   uint32_t *Pl = (uint32_t *)slot;  // P list, then X (later X') list
   const uint64_t ccap = a.slot_bytes / 4;
   Sub s;
@@ -1159,7 +1159,7 @@ __device__ __forceinline__ Sub uniform_sub(const Sub &r) {
 // this wave's L2) and runs it.  Returns true when a task was run.
 __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk_g, lds64 *lds, Acc &acc,
                       ldsu64 *s_hist, bool &is_idle) {
-  const uint32_t l = lane();
+  const uint32_t l = cold_lane();
   const int victim = find_wave(a.has_work, a.n_waves, me);
   if (victim < 0) return false;
   ShareRec *r = a.recs + victim;
@@ -1214,7 +1214,8 @@ __device__ __forceinline__ bool steal(const KArgs &a, uint32_t me, uint64_t *stk
   return true;
 }
 
-__device__ __forceinline__ void mce_main(const KArgs &a) {
+__device__ __forceinline__ void mce_main(const KArgs &a0) {
+  const KArgs &a = a0;
   // The wave's LDS: the clique-size histogram of sizes < kLdsHist, then the
   // area of the LDS tiers (lds_bytes).
   ldsu64 *s_hist = (ldsu64 *)lds_dyn;
@@ -1244,6 +1245,8 @@ __device__ __forceinline__ void mce_main(const KArgs &a) {
   const bool sharing = a.share_bound > 0;
   if (sharing) state_add(a, me, kWorking);
   for (;;) {
+    const KArgs &a = cold_args(a0);
+    const uint32_t l = cold_lane();
     bool did = false;
     if (roots_left) {
       bool free_slot = true;
