@@ -626,20 +626,23 @@ __device__ __forceinline__ uint32_t pk_derive(const PackWave<NW, NX> &w, const P
   return 1;
 }
 
-// Moves what slot s accumulated (batches: count, hash, clique sizes; root
-// statistics: its node count) to the results.  Per lane (lane s).
+// Moves what slot s (uniform) accumulated - batches: count, hash, clique
+// sizes; root statistics: its node count - to the results, a word per lane.
+// (One lane per finished slot, going through its sizes one by one, took 67 LDS
+// round trips a root: 400 small graphs in one replay 7.9 ms against 7.7.)
 template <int NW, int NX>
 __device__ __forceinline__ void pk_finish(const PackWave<NW, NX> &w, uint32_t s) {
   using C = PackCfg<NW, NX>;
-  const KArgs &a = w.a;
-  const uint64_t canon = *w.m(mCanon, s);
-  if (a.root_nodes) atomicAdd(&a.root_nodes[canon], (unsigned long long)*w.m(mNodes, s));
+  const KArgs &a = cold_args(w.a);
+  const uint32_t l = cold_lane();
+  if (a.root_nodes && l == 0) atomicAdd(&a.root_nodes[*w.m(mCanon, s)], (unsigned long long)*w.m(mNodes, s));
   if (a.root_graph) {
-    const uint32_t g = (uint32_t)(*w.m(mBase, s) >> 32);
-    const uint64_t c = *w.m(mCount, s), h = *w.m(mHash, s);
-    if (c) atomicAdd(&a.g_count[g], (unsigned long long)c);
-    if (h) atomicAdd(&a.g_hash[g], (unsigned long long)h);
-    for (uint32_t i = 0; i < C::HS; ++i) {
+    const uint32_t g = bcast32((uint32_t)(*w.m(mBase, s) >> 32));
+    if (l < 2) {
+      const uint64_t v = *w.m(l ? mHash : mCount, s);
+      if (v) atomicAdd(l ? &a.g_hash[g] : &a.g_count[g], (unsigned long long)v);
+    }
+    for (uint32_t i = l; i < C::HS; i += 64) {
       const uint64_t v = w.L.bhist[s * C::HS + i];
       if (v) {
         if (i < a.g_hist_stride) atomicAdd(&a.g_hist[(uint64_t)g * a.g_hist_stride + i], (unsigned long long)v);
@@ -1305,7 +1308,8 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     // Slots whose last record is consumed are done.
     const bool done = l < S && ((busy >> l) & 1) && *w.m(mRefs, l) == 0;
     const uint64_t dm = __ballot(done);
-    if (done) pk_finish<NW, NX>(w, l);
+    if (a.root_nodes || a.root_graph)
+      for (uint64_t d = dm; d; d &= d - 1) pk_finish<NW, NX>(w, (uint32_t)__builtin_ctzll(d));
     busy &= ~(uint32_t)dm;
     if (__builtin_expect_with_probability(__ballot((seen >> 32) != 0) != 0, 0, 0.999)) {
       // Of the working waves about one per idle one tries: when all tried,
