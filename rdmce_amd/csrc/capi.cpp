@@ -382,6 +382,7 @@ struct mce_plan {
   uint64_t deferred_cap = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+  uint8_t *d_inputs = nullptr;      // the inputs below, d_rowoff .. d_eager and the packed search's, in one allocation
   uint64_t *d_rowoff = nullptr;
   uint64_t *d_outoff = nullptr;
   uint32_t *d_col = nullptr;
@@ -478,12 +479,11 @@ void plan_release(mce_plan *p) {
   if (!p) return;
   (void)hipSetDevice(p->device);
   drop_graph(p);
-  void *ptrs[] = {p->d_rowoff,   p->d_outoff,  p->d_col,         p->d_lhash,      p->d_labels,      p->d_roots,
-                  p->d_perm,     p->d_eager,       p->d_slots,      p->d_ctr,         p->d_hist,
-                  p->d_root_nodes, p->d_root_cycles, p->d_list,     p->d_deferred,    p->d_deferred2,
-                  p->d_slots2,   p->d_stacks,      p->d_stacks2,    p->d_recs,        p->d_users,
-                  p->d_has_work, p->d_root_graph,  p->d_gcount,     p->d_ghash,       p->d_ghist,
-                  p->d_work,     p->d_pk_stack,    p->d_pk_plist,   p->d_wide_h[0], p->d_wide_h[1],   p->d_mail,    p->d_pk_idle,  p->d_pool,        p->d_rfirst,     p->d_gstart};
+  void *ptrs[] = {p->d_inputs,      p->d_slots,       p->d_ctr,     p->d_root_nodes, p->d_root_cycles, p->d_list,
+                  p->d_deferred,    p->d_deferred2,   p->d_slots2,  p->d_stacks,     p->d_stacks2,     p->d_recs,
+                  p->d_users,       p->d_has_work,    p->d_gcount,  p->d_ghash,      p->d_ghist,       p->d_work,
+                  p->d_pk_stack,    p->d_pk_plist,    p->d_wide_h[0], p->d_wide_h[1], p->d_mail,       p->d_pk_idle,
+                  p->d_pool};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   for (void *q : p->d_wide)
@@ -548,6 +548,41 @@ std::vector<uint64_t> dispatch_runs(const std::vector<uint64_t> &rfirst, uint64_
   return out;
 }
 
+// A plan's input arrays: one device allocation, each array aligned to 256
+// bytes, filled by one copy when they are small (a copy costs 12 us however
+// short; ten of them were a third of a solve of G(200, 0.1)) and by one each
+// when gathering them on the host first would cost more (1 MB takes 93 us to
+// copy).
+struct Inputs {
+  struct Item {
+    void **dst;
+    const void *src;
+    uint64_t bytes, at;
+  };
+  std::vector<Item> items;
+  uint64_t total = 0;
+  // `src` has to stay until upload(); *dst is set there.
+  template <class T>
+  void add(T **dst, const T *src, uint64_t count) {
+    items.push_back({(void **)dst, src, count * sizeof(T), total});
+    total += (std::max<uint64_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+  }
+  hipError_t upload(uint8_t **base) const {
+    hipError_t e = hipMalloc((void **)base, std::max<uint64_t>(total, 256));
+    if (e != hipSuccess) return e;
+    for (const Item &it : items) *it.dst = *base + it.at;
+    if (total <= (1u << 20)) {
+      std::vector<uint8_t> stage(total);
+      for (const Item &it : items)
+        if (it.bytes) std::memcpy(stage.data() + it.at, it.src, it.bytes);
+      return total ? hipMemcpy(*base, stage.data(), total, hipMemcpyHostToDevice) : hipSuccess;
+    }
+    for (const Item &it : items)
+      if (it.bytes && e == hipSuccess) e = hipMemcpy(*base + it.at, it.src, it.bytes, hipMemcpyHostToDevice);
+    return e;
+  }
+};
+
 // What a plan is built from: a (possibly concatenated) graph, and for
 // batches the graph index of every vertex range.
 struct PlanSpec {
@@ -598,12 +633,12 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
   p->hist_len = (uint32_t)std::min<uint64_t>(max_out + 3, 1ull << 20);
   if (p->hist_len < kLdsHist) p->hist_len = kLdsHist;
 
+  Inputs in;
   std::vector<uint64_t> lhash(g.n);
   for (uint64_t v = 0; v < g.n; ++v) lhash[v] = splitmix64_mix(g.labels[v]);
 
-  PTRY(dalloc(&p->d_rowoff, g.n + 1));
+  std::vector<uint64_t> outoff(g.n + 1, 0);
   {
-    std::vector<uint64_t> outoff(g.n + 1, 0);
     parallel_chunks(g.n, [&](int, uint64_t b, uint64_t e) {
       for (uint64_t v = b; v < e; ++v) {
         const uint32_t *rb = g.col.data() + g.rowoff[v], *re = g.col.data() + g.rowoff[v + 1];
@@ -618,20 +653,13 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
       p->max_deg = std::max(p->max_deg, d + x);
       if (d >= 2 && d <= 1024) p->pool_bound += 8 + (d + 63) / 64 * (align_up(d + x, 64) + 1) + d;
     }
-    PTRY(dalloc(&p->d_outoff, g.n + 1));
-    PTRY(hipMemcpy(p->d_outoff, outoff.data(), (g.n + 1) * 8, hipMemcpyHostToDevice));
   }
-  PTRY(dalloc(&p->d_col, g.col.size()));
-  PTRY(dalloc(&p->d_lhash, g.n));
-  PTRY(dalloc(&p->d_labels, g.n));
-  PTRY(dalloc(&p->d_roots, p->n_roots));
-  PTRY(hipMemcpy(p->d_rowoff, g.rowoff.data(), (g.n + 1) * 8, hipMemcpyHostToDevice));
-  if (!g.col.empty()) PTRY(hipMemcpy(p->d_col, g.col.data(), g.col.size() * 4, hipMemcpyHostToDevice));
-  if (g.n) {
-    PTRY(hipMemcpy(p->d_lhash, lhash.data(), g.n * 8, hipMemcpyHostToDevice));
-    PTRY(hipMemcpy(p->d_labels, g.labels.data(), g.n * 4, hipMemcpyHostToDevice));
-  }
-  if (p->n_roots) PTRY(hipMemcpy(p->d_roots, roots.data(), p->n_roots * 8, hipMemcpyHostToDevice));
+  in.add(&p->d_rowoff, g.rowoff.data(), g.n + 1);
+  in.add(&p->d_outoff, outoff.data(), g.n + 1);
+  in.add(&p->d_col, g.col.data(), g.col.size());
+  in.add(&p->d_lhash, lhash.data(), g.n);
+  in.add(&p->d_labels, g.labels.data(), g.n);
+  in.add(&p->d_roots, roots.data(), p->n_roots);
   if (opt.schedule == MCE_SCHED_CUSTOM) {
     if (!opt.roots) return bail(fail(MCE_ERR_ARG, "custom schedule without a root list"));
     if (opt.n_roots > p->n_roots) return bail(fail(MCE_ERR_ARG, "custom root list longer than the root set"));
@@ -644,8 +672,7 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
       seen[opt.roots[i]] = 1;
     }
     p->n_dispatch = opt.n_roots;
-    PTRY(dalloc(&p->d_perm, opt.n_roots));
-    if (opt.n_roots) PTRY(hipMemcpy(p->d_perm, opt.roots, opt.n_roots * 8, hipMemcpyHostToDevice));
+    in.add(&p->d_perm, opt.roots, opt.n_roots);
   }
   if (mode == MCE_ROOT_EDGE) {
     p->h_rfirst.assign(g.n + 1, 0);
@@ -655,8 +682,7 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
       while (r < p->n_roots && (roots[r] >> 32) == v) ++r;
     }
     p->h_rfirst[g.n] = r;
-    PTRY(dalloc(&p->d_rfirst, g.n + 1));
-    PTRY(hipMemcpy(p->d_rfirst, p->h_rfirst.data(), (g.n + 1) * 8, hipMemcpyHostToDevice));
+    in.add(&p->d_rfirst, p->h_rfirst.data(), g.n + 1);
     const uint64_t nd = p->n_dispatch;
     const uint64_t *cr = opt.schedule == MCE_SCHED_CUSTOM ? opt.roots : nullptr;
     std::vector<uint64_t> runs;
@@ -676,29 +702,27 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
       runs = dispatch_runs(p->h_rfirst, nd, [&](uint64_t i) { return cr ? cr[i] : nd - 1 - i; });
     }
     p->n_groups = runs.size() - 1;
-    PTRY(dalloc(&p->d_gstart, runs.size()));
-    PTRY(hipMemcpy(p->d_gstart, runs.data(), runs.size() * 8, hipMemcpyHostToDevice));
     p->h_runs = std::move(runs);
+    in.add(&p->d_gstart, p->h_runs.data(), p->h_runs.size());
   }
-  if (opt.eager) {
-    PTRY(dalloc(&p->d_eager, p->n_dispatch));
-    if (p->n_dispatch) PTRY(hipMemcpy(p->d_eager, opt.eager, p->n_dispatch, hipMemcpyHostToDevice));
-  }
+  if (opt.eager) in.add(&p->d_eager, opt.eager, p->n_dispatch);
+  std::vector<uint32_t> rg;
   if (spec.graph_vstart) {
     const auto &vs = *spec.graph_vstart;
     p->n_graphs = vs.size() - 1;
     p->g_hist_stride = std::max<uint32_t>(p->hist_len, kLdsHist);
-    std::vector<uint32_t> rg(p->n_roots);
+    rg.resize(p->n_roots);
     for (uint64_t r = 0; r < p->n_roots; ++r) {
       uint64_t v0 = mode == MCE_ROOT_EDGE ? (roots[r] >> 32) : roots[r];
       rg[r] = (uint32_t)(std::upper_bound(vs.begin(), vs.end(), v0) - vs.begin() - 1);
     }
-    PTRY(dalloc(&p->d_root_graph, p->n_roots));
-    if (p->n_roots) PTRY(hipMemcpy(p->d_root_graph, rg.data(), p->n_roots * 4, hipMemcpyHostToDevice));
+    in.add(&p->d_root_graph, rg.data(), p->n_roots);
     PTRY(dalloc(&p->d_gcount, p->n_graphs));
     PTRY(dalloc(&p->d_ghash, p->n_graphs));
     PTRY(dalloc(&p->d_ghist, p->n_graphs * p->g_hist_stride));
   }
+
+  PTRY(in.upload(&p->d_inputs));
 
   const int wpc = opt.waves_per_cu > 0 ? opt.waves_per_cu : 16;
   p->max_waves = (uint32_t)std::min<uint64_t>(16384, (uint64_t)p->cus * std::max(wpc, 32));
@@ -720,8 +744,8 @@ mce_status plan_create_impl(const PlanSpec &spec, const mce_options &opt, mce_pl
   PTRY(dalloc(&p->d_work, kWorkWords));
   set_config(p, wpc, opt.share_bound == 0 ? 24 : opt.share_bound, opt.lds_tier ? 1 : 0);
 
-  PTRY(dalloc(&p->d_ctr, kNumCtr));
-  PTRY(dalloc(&p->d_hist, p->hist_len));
+  PTRY(dalloc(&p->d_ctr, kNumCtr + (uint64_t)p->hist_len));
+  p->d_hist = p->d_ctr + kNumCtr;  // read back with the counters
   if (opt.want_root_stats) {
     PTRY(dalloc(&p->d_root_nodes, p->n_roots));
     PTRY(dalloc(&p->d_root_cycles, p->n_roots));
@@ -963,10 +987,20 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
 
 struct RunOut {
   unsigned long long ctr[kNumCtr];
+  std::vector<unsigned long long> hist;  // of the last pass
   float kernel_ms = 0;
   int passes = 0;
   bool replay = false;
 };
+
+// Counters and clique sizes, which follow each other, in one copy.
+hipError_t read_back(const mce_plan *p, RunOut &ro) {
+  std::vector<unsigned long long> buf(kNumCtr + (uint64_t)p->hist_len);
+  hipError_t e = hipMemcpy(buf.data(), p->d_ctr, buf.size() * 8, hipMemcpyDeviceToHost);
+  std::copy(buf.begin(), buf.begin() + kNumCtr, ro.ctr);
+  ro.hist.assign(buf.begin() + kNumCtr, buf.end());
+  return e;
+}
 
 // One enumeration (plus the deferred pass when needed).  `a` may carry a
 // dispatch list other than the plan's (autotuner samples).
@@ -981,6 +1015,7 @@ mce_status run_core(mce_plan *p, const KArgs &a0, bool allow_graph, RunOut &ro) 
     HIP_TRY(launch_fill_zero(f, s));
     HIP_TRY(hipStreamSynchronize(s));
     std::memset(ro.ctr, 0, sizeof(ro.ctr));
+    ro.hist.assign(p->hist_len, 0);
     return MCE_OK;
   }
   if (p->pack) {
@@ -1013,7 +1048,7 @@ mce_status run_core(mce_plan *p, const KArgs &a0, bool allow_graph, RunOut &ro) 
   HIP_TRY(hipEventElapsedTime(&ms, p->ev[0], p->ev[1]));
   ro.kernel_ms += ms;
   ro.passes = 1;
-  HIP_TRY(hipMemcpy(ro.ctr, p->d_ctr, sizeof(ro.ctr), hipMemcpyDeviceToHost));
+  HIP_TRY(read_back(p, ro));
   uint64_t nd = ro.ctr[kNDeferred];
   if (nd > p->deferred_cap) return fail(MCE_ERR_NOMEM, "deferred-root list overflow");
   if (nd) {
@@ -1064,11 +1099,9 @@ mce_status run_core(mce_plan *p, const KArgs &a0, bool allow_graph, RunOut &ro) 
     HIP_TRY(hipEventElapsedTime(&ms, p->ev[2], p->ev[3]));
     ro.kernel_ms += ms;
     ro.passes = 2;
-    unsigned long long c2[kNumCtr];
-    HIP_TRY(hipMemcpy(c2, p->d_ctr, sizeof(c2), hipMemcpyDeviceToHost));
-    if (c2[kNDeferred]) return fail(MCE_ERR_INTERNAL, "root deferred twice");
     uint64_t deferred_first = ro.ctr[kNDeferred];
-    std::memcpy(ro.ctr, c2, sizeof(c2));
+    HIP_TRY(read_back(p, ro));
+    if (ro.ctr[kNDeferred]) return fail(MCE_ERR_INTERNAL, "root deferred twice");
     ro.ctr[kNDeferred] = deferred_first;
   }
   uint32_t err = (uint32_t)ro.ctr[kErr];
@@ -1115,7 +1148,7 @@ mce_status plan_run_impl(mce_plan *p, mce_result **out) {
   }
   res->hist_len = p->hist_len;
   res->hist = (uint64_t *)std::calloc(p->hist_len, 8);
-  RTRY(hipMemcpy(res->hist, p->d_hist, p->hist_len * 8ull, hipMemcpyDeviceToHost));
+  std::copy(ro.hist.begin(), ro.hist.end(), res->hist);
   res->n_roots = p->n_roots;
   if (p->d_root_nodes) {
     res->root_nodes = (uint64_t *)std::malloc(std::max<uint64_t>(p->n_roots, 1) * 8);
