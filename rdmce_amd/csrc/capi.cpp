@@ -957,9 +957,11 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
       b.n_dispatch_dev = p->d_ctr + kNWide0 + v - 1;
       b.next_root = p->d_work + v * kNextWords;
     }
-    // Waves: those that fit a CU's LDS; without sharing, no more than the runs
+    // Waves: those that fit a CU's LDS and the registers of the variant that
+    // launch_pack picks (a wave that has to wait starts late); without sharing, no more than the runs
     // the first launch hands out (the others' list lengths are not known here).
-    const uint64_t fit = std::max<uint64_t>(1, p->lds_per_cu / pack_lds_bytes(nw, nx, slots, batch));
+    uint64_t fit = std::max<uint64_t>(1, p->lds_per_cu / pack_lds_bytes(nw, nx, slots, batch));
+    if (v == 2 || (v == 1 && p->pack_wpc <= 16)) fit = std::min<uint64_t>(fit, 12);
     uint32_t pw = (uint32_t)std::min<uint64_t>(pack_waves(p), fit * p->cus);
     if (v == 0 && !share) pw = (uint32_t)std::min<uint64_t>(pw, std::max<uint64_t>(units, 1));
     b.state = p->d_work + kStateAt + v * kStateWords;

@@ -216,10 +216,12 @@ constexpr uint64_t pack_lds_bytes(uint32_t nw, uint32_t nx, uint32_t slots, bool
 // (<= 16: 4 waves per SIMD, <= 20: 5, <= 24: 6, else 8).
 hipError_t launch_mce(const KArgs &a, uint32_t waves, uint32_t waves_per_cu, hipStream_t stream);
 // Packed search: variant v = (kPackNW[v], kPackNX[v]); waves_per_cu selects
-// the kernel compiled for that occupancy (<= 16: 4 waves per SIMD, <= 20: 5,
-// <= 24: 6, else 8), except for the last variant, of which LDS lets 13 waves
-// share a CU: 3 per SIMD (39 spilled registers against 134 at 4; R-MAT 14
-// 11.5 ms against 13.9 over all launches).
+// the kernel compiled for that occupancy (<= 16: 4 waves per SIMD, 3 for the
+// wider variants, whose records do not fit 128 registers; <= 20: 5, <= 24: 6,
+// else 8).  The last variant is always compiled for 3: LDS lets 13 of its waves
+// share a CU.  3 against 4: (2, 4) spills 43 registers instead of 134 and R-MAT
+// 14 takes 11.5 ms against 13.9 over all launches; (2, 2) also, the 200k-vertex
+// community graph 21.9 against 22.3.
 hipError_t launch_pack(const KArgs &a, int variant, uint32_t waves, uint32_t waves_per_cu, hipStream_t stream);
 hipError_t launch_copy_probe(const void *src, void *dst, uint64_t bytes, hipStream_t stream);
 // Zero-fills n 64-bit words with a kernel (safe inside captured hipGraphs,

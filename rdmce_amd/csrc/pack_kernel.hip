@@ -1345,7 +1345,7 @@ hipError_t launch_variant(const KArgs &a, uint32_t waves, uint32_t wpc, size_t l
   if (a.list)
     hipLaunchKernelGGL((pack_kernel<NW, NX, 4, true>), dim3(waves), dim3(64), lds, stream, a);
   else if (wpc <= 16)
-    hipLaunchKernelGGL((pack_kernel<NW, NX, 4, false>), dim3(waves), dim3(64), lds, stream, a);
+    hipLaunchKernelGGL((pack_kernel<NW, NX, (NW == 1 ? 4 : 3), false>), dim3(waves), dim3(64), lds, stream, a);
   else if (wpc <= 20)
     hipLaunchKernelGGL((pack_kernel<NW, NX, 5, false>), dim3(waves), dim3(64), lds, stream, a);
   else if (wpc <= 24)
