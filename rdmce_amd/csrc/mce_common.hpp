@@ -78,6 +78,15 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   t = __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xC, 0xF, false); v = v > t ? v : t;
   return __builtin_amdgcn_readlane(v, 63);
 }
+__device__ __forceinline__ uint32_t wave_or_u32(uint32_t v) {
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x111, 0xF, 0xF, false);
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x112, 0xF, 0xF, false);
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x114, 0xF, 0xF, false);
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x118, 0xF, 0xF, false);
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x142, 0xA, 0xF, false);
+  v |= __builtin_amdgcn_update_dpp(0u, v, 0x143, 0xC, 0xF, false);
+  return __builtin_amdgcn_readlane(v, 63);
+}
 // Population count of a set whose words are held one per lane (lanes < W).
 __device__ __forceinline__ uint32_t set_popc(uint64_t wk, uint32_t W) {
   uint32_t s = 0;
