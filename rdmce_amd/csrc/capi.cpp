@@ -1234,10 +1234,12 @@ mce_status autotune_impl(mce_plan *p, uint64_t stride, mce_tune_result *out) {
   if (!st) best = base_ms;
   if (p->pack) {
     // Packed plans: subproblems per wave (the LDS tile width), packed waves
-    // per CU, then the sharing bound of the wide roots' kernel.  Sample runs
-    // vary by a few percent from run to run, so the default is timed twice
-    // more and a setting replaces the best one only when the better of two
-    // runs beats it by kPackTuneMargin.
+    // per CU, then the default sharing bound if the plan has another.  Sharing
+    // is never turned off: a sample holds few of the heavy roots that it is for
+    // (Chung-Lu 4M: the sample took 34.6 ms without against 36.4, and the
+    // vertex roots then 3,077 ms against 32).  Sample runs vary by a few percent
+    // from run to run, so the default is timed twice more and a setting replaces
+    // the best one only when the better of two runs beats it by kPackTuneMargin.
     constexpr double kPackTuneMargin = 0.97;
     if (!st) st = trial(base_wpc, base_tau, base_lds, ms);
     if (!st) best = base_ms = std::min(base_ms, ms);
@@ -1274,10 +1276,9 @@ mce_status autotune_impl(mce_plan *p, uint64_t stride, mce_tune_result *out) {
       if (!st && better) best_pwpc = pw;
     }
     p->pack_wpc = best_pwpc;
-    for (int tau : {24, -1}) {
-      if (st || tau == base_tau) continue;
-      st = challenge(tau, better);
-      if (!st && better) best_tau = tau;
+    if (!st && base_tau != 24) {
+      st = challenge(24, better);
+      if (!st && better) best_tau = 24;
     }
     (void)hipFree(d_sample);
     if (d_sruns) (void)hipFree(d_sruns);
