@@ -244,7 +244,7 @@ typedef struct mce_tune_result {
  * at the best occupancy, then waves per CU again when the bound changed, then
  * the LDS tier off.  Packed plans (mce_options.pack): subproblems per
  * wavefront in {1, 2, 4, 8}, then packed wavefronts per CU in {12, 16, 20,
- * 24}, then the sharing bound of the wide roots' kernel in {24, off}.
+ * 24}, then the default sharing bound if the plan has another.
  * Checks that every setting gives the same clique count and hash, and keeps
  * the fastest for later mce_plan_run calls. */
 mce_status mce_plan_autotune(mce_plan *p, uint64_t stride, mce_tune_result *out);
