@@ -423,6 +423,7 @@ struct mce_plan {
   int pack = 0;
   uint32_t pack_slots = 4;
   int pack_wpc = 16;
+  bool pack_ready = false;           // every packed arena below is allocated
   uint32_t pack_waves_alloc = 0;     // waves the arenas below are sized for
   uint64_t pk_stack_words = 0;       // record stack words per wave
   uint64_t *d_pk_stack = nullptr;
@@ -475,19 +476,18 @@ void drop_graph(mce_plan *p) {
   p->graph = nullptr;
 }
 
+void free_pack(mce_plan *p);
+
 void plan_release(mce_plan *p) {
   if (!p) return;
   (void)hipSetDevice(p->device);
   drop_graph(p);
   void *ptrs[] = {p->d_inputs,      p->d_slots,       p->d_ctr,     p->d_root_nodes, p->d_root_cycles, p->d_list,
                   p->d_deferred,    p->d_deferred2,   p->d_slots2,  p->d_stacks,     p->d_stacks2,     p->d_recs,
-                  p->d_users,       p->d_has_work,    p->d_gcount,  p->d_ghash,      p->d_ghist,       p->d_work,
-                  p->d_pk_stack,    p->d_pk_plist,    p->d_wide_h[0], p->d_wide_h[1], p->d_mail,       p->d_pk_idle,
-                  p->d_pool};
+                  p->d_users,       p->d_has_work,    p->d_gcount,  p->d_ghash,      p->d_ghist,       p->d_work};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
-  for (void *q : p->d_wide)
-    if (q) (void)hipFree(q);
+  free_pack(p);
   for (auto &e : p->ev)
     if (e) (void)hipEventDestroy(e);
   if (p->stream) (void)hipStreamDestroy(p->stream);
@@ -827,33 +827,62 @@ uint64_t pack_need_records(const mce_plan *p, uint32_t nw) {
   return kPackThr + 64 * (std::min<uint64_t>(64ull * nw, p->max_out) + 3);
 }
 
-// Allocates the packed search's arenas (once per plan, for 32 waves per CU).
-mce_status ensure_pack(mce_plan *p) {
-  if (p->d_pk_stack && (!p->opt.want_list || p->d_pk_plist)) return MCE_OK;
+// Frees the packed search's arenas.
+void free_pack(mce_plan *p) {
+  void *ptrs[] = {p->d_pk_stack, p->d_pk_plist, p->d_wide_h[0], p->d_wide_h[1], p->d_mail, p->d_pk_idle, p->d_pool};
+  for (void *q : ptrs)
+    if (q) (void)hipFree(q);
+  for (void *q : p->d_wide)
+    if (q) (void)hipFree(q);
+  p->d_pk_stack = p->d_mail = p->d_pool = nullptr;
+  p->d_pk_plist = nullptr;
+  p->d_pk_idle = nullptr;
+  for (auto &q : p->d_wide) q = nullptr;
+  for (auto &q : p->d_wide_h) q = nullptr;
+  p->pk_stack_words = p->pool_words = 0;
+  p->pack_waves_alloc = 0;
+  p->pack_ready = false;
+}
+
+hipError_t alloc_pack(mce_plan *p) {
   const uint32_t waves = (uint32_t)std::min<uint64_t>(p->max_waves, (uint64_t)p->cus * 32);
   uint64_t words = 0;
   for (int v = 0; v < kPackVariants; ++v)
     words = std::max(words, pack_need_records(p, kPackNW[v]) * pack_rec_words(kPackNW[v], kPackNX[v]));
-  if (!p->d_pk_stack) {
-    HIP_TRY(dalloc(&p->d_pk_stack, words * waves));
-    p->pk_stack_words = words;
-    p->pack_waves_alloc = waves;
-    p->wide_cap = std::max<uint64_t>(p->n_dispatch, 1);
-    for (auto &q : p->d_wide) HIP_TRY(dalloc(&q, p->wide_cap));
-    for (auto &q : p->d_wide_h) HIP_TRY(dalloc(&q, p->wide_cap));
-    HIP_TRY(dalloc(&p->d_mail, (uint64_t)kPackMailWords * waves));
-    HIP_TRY(dalloc(&p->d_pk_idle, (waves + 63) / 64));
-    // Kept vertex bitmaps: at most one per vertex with two or more edge
-    // roots, within a quarter of the free device memory.
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-    p->pool_words = std::min<uint64_t>(p->pool_bound, free_b / 4 / 8);
+  hipError_t e = dalloc(&p->d_pk_stack, words * waves);
+  p->pk_stack_words = words;
+  p->pack_waves_alloc = waves;
+  p->wide_cap = std::max<uint64_t>(p->n_dispatch, 1);
+  for (auto &q : p->d_wide)
+    if (e == hipSuccess) e = dalloc(&q, p->wide_cap);
+  for (auto &q : p->d_wide_h)
+    if (e == hipSuccess) e = dalloc(&q, p->wide_cap);
+  if (e == hipSuccess) e = dalloc(&p->d_mail, (uint64_t)kPackMailWords * waves);
+  if (e == hipSuccess) e = dalloc(&p->d_pk_idle, (waves + 63) / 64);
+  if (e == hipSuccess && p->opt.want_list) e = dalloc(&p->d_pk_plist, (uint64_t)waves * kPackMaxSlots * kPackMaxP);
+  if (e != hipSuccess) return e;
+  // Kept vertex bitmaps: at most one per vertex with two or more edge
+  // roots, within a quarter of the free device memory.
+  size_t free_b = 0, total_b = 0;
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
+  p->pool_words = std::min<uint64_t>(p->pool_bound, free_b / 4 / 8);
 #ifdef RDMCE_PACK_POOL_MAX  // test builds: a pool that runs out after a few bitmaps
-    p->pool_words = std::min<uint64_t>(p->pool_words, RDMCE_PACK_POOL_MAX);
+  p->pool_words = std::min<uint64_t>(p->pool_words, RDMCE_PACK_POOL_MAX);
 #endif
-    if (p->pool_words) HIP_TRY(dalloc(&p->d_pool, p->pool_words));
+  return p->pool_words ? dalloc(&p->d_pool, p->pool_words) : hipSuccess;
+}
+
+// Allocates the packed search's arenas (once per plan, for 32 waves per CU):
+// all of them, or none, so that a run after one that failed here starts over.
+mce_status ensure_pack(mce_plan *p) {
+  if (p->pack_ready) return MCE_OK;
+  const hipError_t e = alloc_pack(p);
+  if (e != hipSuccess) {
+    free_pack(p);
+    (void)hipGetLastError();  // or the next launch would report it
+    return fail(MCE_ERR_DEVICE, std::string("packed search memory: ") + hipGetErrorString(e));
   }
-  if (p->opt.want_list && !p->d_pk_plist) HIP_TRY(dalloc(&p->d_pk_plist, (uint64_t)waves * kPackMaxSlots * kPackMaxP));
+  p->pack_ready = true;
   return MCE_OK;
 }
 

@@ -397,7 +397,18 @@ bool emu_capture(hipStream_t s, const EmuLaunch &L) {
 }
 
 // ---- runtime API ---------------------------------------------------------
+// For tests of running out of memory: the emu_malloc_fail_in-th allocation
+// from now fails (0: none), and the bytes allocated so far.
+extern "C" {
+long emu_malloc_fail_in = 0;
+unsigned long long emu_malloc_bytes = 0;
+}
 hipError_t hipMalloc(void **p, size_t bytes) {
+  if (emu_malloc_fail_in && --emu_malloc_fail_in == 0) {
+    *p = nullptr;
+    return hipErrorOutOfMemory;
+  }
+  emu_malloc_bytes += bytes;
   *p = guarded_alloc(bytes ? bytes : 1, 0xA5);
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }

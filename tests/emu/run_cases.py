@@ -8,6 +8,7 @@ so the cases are small graphs and few waves (EMU_CUS compute units).
 
     RDMCE_LIB=tests/emu/_build/librdmce_emu.so EMU_CUS=1 python tests/emu/run_cases.py [filter]
 """
+import ctypes
 import os
 import sys
 import time
@@ -208,6 +209,34 @@ def cases():
                 return f"packed batch graph {i} differs"
         return None
     yield "pack batch", pack_batch
+
+    def pack_out_of_memory(lists):
+        # the k-th allocation of a packed plan's first run fails: that run
+        # reports it, one that fails again reports it again, and one with
+        # memory gives the right result
+        rg = graph(dense_core_graph(70, 4, 60, 0.05, 3))
+        ref = oracle_for(rg, list_cap=1 << 20)
+        fail_in = ctypes.c_long.in_dll(R.lib(), "emu_malloc_fail_in")
+        k = 0
+        while True:
+            k += 1
+            p = R.Plan(rg, waves_per_cu=wpc, pack=True, pack_waves_per_cu=2, want_list=lists, want_root_stats=True)
+            for _ in range(2):
+                fail_in.value = k
+                try:
+                    p.run()
+                except Exception:
+                    pass
+                left, fail_in.value = fail_in.value, 0
+                if left:  # fewer allocations than that: nothing failed
+                    break
+            err = same(p.run(), ref, lists=lists)
+            p.free()
+            if err:
+                return f"after allocation {k} failed: {err}"
+            if left:
+                return None if k > 1 else "a first run without an allocation"
+    yield "pack out of memory", lambda: pack_out_of_memory(False) or pack_out_of_memory(True)
 
 
 def main():
