@@ -360,6 +360,19 @@ int32_t mce_device_count(void) {
 // Plan: one graph, or a batch of disjoint graphs concatenated, resident in
 // HBM with its roots and per-wave scratch.
 // ---------------------------------------------------------------------------
+// What the packed search of a plan needs in device memory.
+struct PackNeed {
+  uint64_t stack = 0;       // words of a wave's record stack
+  uint32_t waves = 0;       // waves with a stack (and clique-list ids in plans with lists)
+  uint32_t mail_waves = 0;  // waves with mail (0: nothing is ever given away)
+  uint32_t lists = 0;       // lists of roots too wide for a variant: one less than the launches
+  uint64_t pool = 0;        // words for kept vertex bitmaps
+  bool covers(const PackNeed &o) const {
+    return stack >= o.stack && waves >= o.waves && mail_waves >= o.mail_waves && lists >= o.lists &&
+           (pool > 0 || o.pool == 0);
+  }
+};
+
 struct mce_plan {
   mce_options opt{};
   int device = 0;
@@ -423,9 +436,9 @@ struct mce_plan {
   int pack = 0;
   uint32_t pack_slots = 4;
   int pack_wpc = 16;
-  bool pack_ready = false;           // every packed arena below is allocated
-  uint32_t pack_waves_alloc = 0;     // waves the arenas below are sized for
-  uint64_t pk_stack_words = 0;       // record stack words per wave
+  uint64_t pool_bound = 0;           // words that every vertex's bitmap would take
+  PackNeed pk;                       // what the arenas below hold
+  uint8_t *d_pack = nullptr;         // all of them, in one allocation
   uint64_t *d_pk_stack = nullptr;
   uint32_t *d_pk_plist = nullptr;
   uint64_t *d_wide[kPackVariants] = {};  // roots too wide for variant v, in the order met
@@ -433,9 +446,6 @@ struct mce_plan {
   unsigned long long *d_pk_idle = nullptr;
   uint64_t *d_wide_h[2] = {};       // per entry of list v (in turn): its kept vertex bitmap in d_pool
   uint64_t *d_pool = nullptr;
-  uint64_t pool_words = 0;
-  uint64_t pool_bound = 0;           // words that every vertex's bitmap would take
-  uint64_t wide_cap = 0;
   std::vector<uint64_t> h_rfirst;    // edge roots: canonical id of the first root of each vertex, + m
   uint64_t *d_rfirst = nullptr;
   uint64_t *d_gstart = nullptr;      // runs of the plan's dispatch list sharing their first vertex
@@ -476,8 +486,6 @@ void drop_graph(mce_plan *p) {
   p->graph = nullptr;
 }
 
-void free_pack(mce_plan *p);
-
 void plan_release(mce_plan *p) {
   if (!p) return;
   (void)hipSetDevice(p->device);
@@ -487,7 +495,7 @@ void plan_release(mce_plan *p) {
                   p->d_users,       p->d_has_work,    p->d_gcount,  p->d_ghash,      p->d_ghist,       p->d_work};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
-  free_pack(p);
+  if (p->d_pack) (void)hipFree(p->d_pack);
   for (auto &e : p->ev)
     if (e) (void)hipEventDestroy(e);
   if (p->stream) (void)hipStreamDestroy(p->stream);
@@ -827,67 +835,123 @@ uint64_t pack_need_records(const mce_plan *p, uint32_t nw) {
   return kPackThr + 64 * (std::min<uint64_t>(64ull * nw, p->max_out) + 3);
 }
 
-// Frees the packed search's arenas.
-void free_pack(mce_plan *p) {
-  void *ptrs[] = {p->d_pk_stack, p->d_pk_plist, p->d_wide_h[0], p->d_wide_h[1], p->d_mail, p->d_pk_idle, p->d_pool};
-  for (void *q : ptrs)
-    if (q) (void)hipFree(q);
-  for (void *q : p->d_wide)
-    if (q) (void)hipFree(q);
-  p->d_pk_stack = p->d_mail = p->d_pool = nullptr;
-  p->d_pk_plist = nullptr;
-  p->d_pk_idle = nullptr;
-  for (auto &q : p->d_wide) q = nullptr;
-  for (auto &q : p->d_wide_h) q = nullptr;
-  p->pk_stack_words = p->pool_words = 0;
-  p->pack_waves_alloc = 0;
-  p->pack_ready = false;
+// Whether a level can ever be exposed, or records given away: |P| >=
+// share_bound takes a root with that many candidates (at most the largest
+// out-degree), or an eager root.
+bool can_share(const mce_plan *p, const KArgs &a) {
+  return a.share_bound > 0 && ((uint64_t)a.share_bound <= p->max_out || a.eager);
 }
 
-hipError_t alloc_pack(mce_plan *p) {
-  const uint32_t waves = (uint32_t)std::min<uint64_t>(p->max_waves, (uint64_t)p->cus * 32);
-  uint64_t words = 0;
+// Launches of a packed run: its variants up to the first one that no root of
+// this graph is too wide for (|P0| is at most the largest out-degree, |X0'| the
+// largest degree), else all of them and the one-root-per-wave kernel, which
+// also takes the eager roots.
+int pack_launches(const mce_plan *p, const KArgs &a) {
   for (int v = 0; v < kPackVariants; ++v)
-    words = std::max(words, pack_need_records(p, kPackNW[v]) * pack_rec_words(kPackNW[v], kPackNX[v]));
-  hipError_t e = dalloc(&p->d_pk_stack, words * waves);
-  p->pk_stack_words = words;
-  p->pack_waves_alloc = waves;
-  p->wide_cap = std::max<uint64_t>(p->n_dispatch, 1);
-  for (auto &q : p->d_wide)
-    if (e == hipSuccess) e = dalloc(&q, p->wide_cap);
-  for (auto &q : p->d_wide_h)
-    if (e == hipSuccess) e = dalloc(&q, p->wide_cap);
-  if (e == hipSuccess) e = dalloc(&p->d_mail, (uint64_t)kPackMailWords * waves);
-  if (e == hipSuccess) e = dalloc(&p->d_pk_idle, (waves + 63) / 64);
-  if (e == hipSuccess && p->opt.want_list) e = dalloc(&p->d_pk_plist, (uint64_t)waves * kPackMaxSlots * kPackMaxP);
-  if (e != hipSuccess) return e;
-  // Kept vertex bitmaps: at most one per vertex with two or more edge
-  // roots, within a quarter of the free device memory.
+    if (p->max_out <= 64 * kPackNW[v] && p->max_deg <= 64 * kPackNX[v] && !a.eager) return v + 1;
+  return kPackVariants + 1;
+}
+
+// Slots and waves of variant v's launch.
+struct PackShape {
+  uint32_t slots, waves;
+};
+PackShape pack_shape(const mce_plan *p, const KArgs &a, int v) {
+  const uint32_t nw = kPackNW[v], nx = kPackNX[v];
+  const bool batch = a.root_graph != nullptr;
+  // the wider variants' slots are 3.5 and 5.5 times larger: half and a
+  // quarter as many; and no more than let the requested waves per CU all be
+  // resident in its LDS (a wave that waited for LDS started late)
+  uint32_t slots = std::max<uint32_t>(1, p->pack_slots >> v);
+  while (slots > 1 && (pack_lds_bytes(nw, nx, slots, batch) > p->lds_per_block_max ||
+                       pack_lds_bytes(nw, nx, slots, batch) * (uint64_t)p->pack_wpc > p->lds_per_cu))
+    --slots;
+  // Waves: those that fit a CU's LDS and the registers of the variant that
+  // launch_pack picks (a wave that has to wait starts late); without sharing,
+  // no more than the runs the first launch hands out (the others' list lengths
+  // are not known here).
+  uint64_t fit = std::max<uint64_t>(1, p->lds_per_cu / pack_lds_bytes(nw, nx, slots, batch));
+  if (v == 2 || (v == 1 && p->pack_wpc <= 16)) fit = std::min<uint64_t>(fit, 12);
+  uint64_t waves = std::min<uint64_t>({(uint64_t)p->max_waves, (uint64_t)p->cus * 32, fit * p->cus,
+                                       std::max<uint64_t>(1, (uint64_t)p->cus * p->pack_wpc)});
+  if (v == 0 && !can_share(p, a))
+    waves = std::min<uint64_t>(waves, std::max<uint64_t>(a.pk_gstart ? a.pk_ngroups : a.n_dispatch, 1));
+  return {slots, (uint32_t)waves};
+}
+
+// What a run with these arguments and the plan's present settings needs: the
+// variants and waves that it launches, not the widest and most there could be.
+// A solve allocates and frees this in every call, and what is freed has to be
+// cleared before it is handed out again, at some 30 GB/s.  Solves one after the
+// other, with arenas for 8,192 waves of the widest variant against this:
+// G(91, 0.157), 1.1 GB, 32.1 ms a call against 0.26; G(3854, 0.0038), 1.5 GB, 33
+// to 49 against 6.6.
+PackNeed pack_need(const mce_plan *p, const KArgs &a) {
+  PackNeed n;
+  const int launches = pack_launches(p, a);
+  for (int v = 0; v < launches && v < kPackVariants; ++v) {
+    n.stack = std::max(n.stack, pack_need_records(p, kPackNW[v]) * pack_rec_words(kPackNW[v], kPackNX[v]));
+    n.waves = std::max(n.waves, pack_shape(p, a, v).waves);
+  }
+  if (can_share(p, a)) n.mail_waves = n.waves;
+  n.lists = (uint32_t)launches - 1;
+  if (n.lists) n.pool = p->pool_bound;
+  return n;
+}
+
+// Allocates the packed search's arenas for a run with these arguments, again
+// when settings or arguments ask for more: one allocation, so they are all
+// there or none is.
+mce_status ensure_pack(mce_plan *p, const KArgs &a) {
+  const PackNeed need = pack_need(p, a);
+  if (p->d_pack && p->pk.covers(need)) return MCE_OK;
+  PackNeed n = p->pk;
+  n.stack = std::max(n.stack, need.stack);
+  n.waves = std::max(n.waves, need.waves);
+  n.mail_waves = std::max(n.mail_waves, need.mail_waves);
+  n.lists = std::max(n.lists, need.lists);
+  n.pool = std::max(n.pool, need.pool);
+  drop_graph(p);  // (it would launch with the old ones)
+  if (p->d_pack) (void)hipFree(p->d_pack);
+  p->d_pack = nullptr;
+  p->pk = PackNeed{};
+  uint64_t bytes = 0;
+  auto take = [&](uint64_t b) {
+    const uint64_t at = bytes;
+    bytes = align_up(bytes + b, 256);
+    return at;
+  };
+  const uint64_t list = 8 * std::max<uint64_t>(p->n_dispatch, 1);
+  const uint64_t o_stack = take(8 * n.stack * n.waves), o_mail = take(8ull * kPackMailWords * n.mail_waves),
+                 o_idle = take((n.mail_waves + 63) / 64 * 8), o_wide = take(n.lists * list),
+                 o_wide_h = take(2 * list),
+                 o_ids = take(p->opt.want_list ? 4ull * kPackMaxSlots * kPackMaxP * n.waves : 0);
+  // Kept vertex bitmaps: room for one per vertex with two or more edge roots,
+  // within a quarter of the free device memory (a run that was split keeps one
+  // per part; what finds no room is built again).
   size_t free_b = 0, total_b = 0;
   if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 0;
-  p->pool_words = std::min<uint64_t>(p->pool_bound, free_b / 4 / 8);
+  n.pool = std::min<uint64_t>(n.pool, free_b > bytes ? (free_b - bytes) / 4 / 8 : 0);
 #ifdef RDMCE_PACK_POOL_MAX  // test builds: a pool that runs out after a few bitmaps
-  p->pool_words = std::min<uint64_t>(p->pool_words, RDMCE_PACK_POOL_MAX);
+  n.pool = std::min<uint64_t>(n.pool, RDMCE_PACK_POOL_MAX);
 #endif
-  return p->pool_words ? dalloc(&p->d_pool, p->pool_words) : hipSuccess;
-}
-
-// Allocates the packed search's arenas (once per plan, for 32 waves per CU):
-// all of them, or none, so that a run after one that failed here starts over.
-mce_status ensure_pack(mce_plan *p) {
-  if (p->pack_ready) return MCE_OK;
-  const hipError_t e = alloc_pack(p);
+  const uint64_t o_pool = take(8 * n.pool);
+  const hipError_t e = hipMalloc((void **)&p->d_pack, bytes);
   if (e != hipSuccess) {
-    free_pack(p);
+    p->d_pack = nullptr;
     (void)hipGetLastError();  // or the next launch would report it
     return fail(MCE_ERR_DEVICE, std::string("packed search memory: ") + hipGetErrorString(e));
   }
-  p->pack_ready = true;
+  auto at = [&](bool has, uint64_t o) { return has ? p->d_pack + o : nullptr; };
+  p->d_pk_stack = (uint64_t *)at(true, o_stack);
+  p->d_mail = (uint64_t *)at(n.mail_waves, o_mail);
+  p->d_pk_idle = (unsigned long long *)at(n.mail_waves, o_idle);
+  for (uint32_t v = 0; v < (uint32_t)kPackVariants; ++v) p->d_wide[v] = (uint64_t *)at(v < n.lists, o_wide + v * list);
+  for (int k = 0; k < 2; ++k) p->d_wide_h[k] = (uint64_t *)at(true, o_wide_h + k * list);
+  p->d_pk_plist = (uint32_t *)at(p->opt.want_list, o_ids);
+  p->d_pool = (uint64_t *)at(n.pool, o_pool);
+  p->pk = n;
   return MCE_OK;
-}
-
-uint32_t pack_waves(const mce_plan *p) {
-  return (uint32_t)std::min<uint64_t>(p->pack_waves_alloc, std::max<uint64_t>(1, (uint64_t)p->cus * p->pack_wpc));
 }
 
 // Ranges zeroed before a run: counters and results ...
@@ -910,11 +974,6 @@ hipError_t collect(const mce_plan *p, hipStream_t s) {
   return launch_collect(p->d_work + kSumsAt, p->d_work + kHistAt, p->d_ctr, p->d_hist, p->hist_len, s);
 }
 
-// Whether a level can ever be exposed: |P| >= share_bound takes a root with
-// that many candidates (at most the largest out-degree), or an eager root.
-bool can_share(const mce_plan *p, const KArgs &a) {
-  return a.share_bound > 0 && ((uint64_t)a.share_bound <= p->max_out || a.eager);
-}
 // Waves of the one-root-per-wave kernel: those beyond the root count could
 // only take shared tasks.
 uint32_t mce_waves(const mce_plan *p, KArgs &a) {
@@ -939,40 +998,33 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
   f.add(p->d_work, kWorkWords);
   if (p->d_root_nodes) f.add(p->d_root_nodes, p->n_roots);
   if (p->d_root_cycles) f.add(p->d_root_cycles, p->n_roots);
-  if (p->pack) f.add(p->d_pk_idle, (p->pack_waves_alloc + 63) / 64);
+  if (p->pack && p->d_pk_idle) f.add(p->d_pk_idle, (p->pk.mail_waves + 63) / 64);
   hipError_t e = launch_fill_zero(f, s);
   if (e != hipSuccess) return e;
   if (!p->pack) {
     e = launch_mce(a, mce_waves(p, a), (uint32_t)p->waves_per_cu, s);
     return e == hipSuccess ? collect(p, s) : e;
   }
-  const uint64_t units = a.pk_gstart ? a.pk_ngroups : a.n_dispatch;
   const bool share = can_share(p, a);
-  const bool batch = a.root_graph != nullptr;
-  for (int v = 0; v < kPackVariants && e == hipSuccess; ++v) {
+  const int launches = pack_launches(p, a);
+  for (int v = 0; v < launches && v < kPackVariants && e == hipSuccess; ++v) {
+    const PackShape sh = pack_shape(p, a, v);
     const uint32_t nw = kPackNW[v], nx = kPackNX[v];
     KArgs b = a;
     b.pk_stack = p->d_pk_stack;
-    b.pk_cap = p->pk_stack_words / pack_rec_words(nw, nx);
+    b.pk_cap = p->pk.stack / pack_rec_words(nw, nx);
     b.pk_thr = (uint32_t)(b.pk_cap - 64 * (std::min<uint64_t>(64ull * nw, p->max_out) + 3));
 #ifdef RDMCE_PACK_THR_MAX  // test builds: reach the depth-first expansion on small graphs
     b.pk_thr = std::min<uint32_t>(b.pk_thr, RDMCE_PACK_THR_MAX);
 #endif
-    // the wider variants' slots are 3.5 and 5.3 times larger: half and a
-    // quarter as many; and no more than let the requested waves per CU all be
-    // resident in its LDS (a wave that waited for LDS started late)
-    uint32_t slots = std::max<uint32_t>(1, p->pack_slots >> v);
-    while (slots > 1 && (pack_lds_bytes(nw, nx, slots, batch) > p->lds_per_block_max ||
-                         pack_lds_bytes(nw, nx, slots, batch) * (uint64_t)p->pack_wpc > p->lds_per_cu))
-      --slots;
-    b.pk_slots = slots;
+    b.pk_slots = sh.slots;
     b.pk_plist = p->d_pk_plist;
     b.wide = p->d_wide[v];
     b.n_wide = p->d_ctr + kNWide0 + v;
     b.heavy = p->d_wide[kPackVariants - 1];
     b.n_heavy = p->d_ctr + kNWide0 + kPackVariants - 1;
     b.pk_pool = p->d_pool;
-    b.pk_pool_words = p->pool_words;
+    b.pk_pool_words = p->pk.pool;
     b.pk_pool_used = p->d_ctr + kPoolUsed;
     // wide roots leave with a copy of their vertex bitmap, from which the
     // next launches derive them
@@ -986,24 +1038,15 @@ hipError_t enqueue_run(const mce_plan *p, const KArgs &a0, hipStream_t s) {
       b.n_dispatch_dev = p->d_ctr + kNWide0 + v - 1;
       b.next_root = p->d_work + v * kNextWords;
     }
-    // Waves: those that fit a CU's LDS and the registers of the variant that
-    // launch_pack picks (a wave that has to wait starts late); without sharing, no more than the runs
-    // the first launch hands out (the others' list lengths are not known here).
-    uint64_t fit = std::max<uint64_t>(1, p->lds_per_cu / pack_lds_bytes(nw, nx, slots, batch));
-    if (v == 2 || (v == 1 && p->pack_wpc <= 16)) fit = std::min<uint64_t>(fit, 12);
-    uint32_t pw = (uint32_t)std::min<uint64_t>(pack_waves(p), fit * p->cus);
-    if (v == 0 && !share) pw = (uint32_t)std::min<uint64_t>(pw, std::max<uint64_t>(units, 1));
     b.state = p->d_work + kStateAt + v * kStateWords;
     b.pk_share = share;
-    b.pk_nwaves = pw;
+    b.pk_nwaves = sh.waves;
     b.pk_idle = p->d_pk_idle;
     b.pk_mail = p->d_mail;
-    e = launch_pack(b, v, pw, (uint32_t)p->pack_wpc, s);
-    // No root of this graph is too wide for this variant: |P0| is at most the
-    // largest out-degree, |X0'| the largest degree.
-    if (p->max_out <= 64 * nw && p->max_deg <= 64 * nx && !a.eager) return e == hipSuccess ? collect(p, s) : e;
+    e = launch_pack(b, v, sh.waves, (uint32_t)p->pack_wpc, s);
   }
   if (e != hipSuccess) return e;
+  if (launches <= kPackVariants) return collect(p, s);
   KArgs c = a;
   c.perm = p->d_wide[kPackVariants - 1];
   c.reverse = 0;
@@ -1050,7 +1093,7 @@ mce_status run_core(mce_plan *p, const KArgs &a0, bool allow_graph, RunOut &ro) 
     return MCE_OK;
   }
   if (p->pack) {
-    mce_status st = ensure_pack(p);
+    mce_status st = ensure_pack(p, a);
     if (st) return st;
   }
   const bool use_graph = allow_graph && p->opt.use_graph;

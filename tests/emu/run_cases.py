@@ -236,6 +236,38 @@ def cases():
                 return f"after allocation {k} failed: {err}"
             if left:
                 return None if k > 1 else "a first run without an allocation"
+    def pack_memory():
+        # a packed solve of a graph of small roots takes memory for the
+        # variant and the waves it launches: less than 12-word records for 32
+        # waves a CU would take
+        rg = graph(random_graph(200, 0.03, 5))
+        ref = oracle_for(rg)
+        ro, co = rg.GetRowOffset(), rg.GetColIdx()
+        out = max(int(ro[v + 1] - ro[v]) - int(np.searchsorted(co[ro[v]:ro[v + 1]], v, side="right"))
+                  for v in range(rg.GetNumVertices()))
+        total = ctypes.c_ulonglong.in_dll(R.lib(), "emu_malloc_bytes")
+        p = R.Plan(rg, waves_per_cu=wpc, pack=True, want_root_stats=True)
+        before = total.value
+        err = same(p.run(), ref)
+        took = total.value - before
+        err = err or same(p.run(), ref) or (None if total.value - before == took else "a second run allocates")
+        p.free()
+        bound = 32 * 8 * 12 * (256 + 64 * (out + 3))
+        return err or (None if took <= bound else f"{took} bytes for the packed search, {bound} expected at most")
+    yield "pack memory", pack_memory
+
+    def pack_grows(kw):
+        # the autotuner asks for more waves and, where it was off, for sharing:
+        # the plan's memory follows, also under a captured replay
+        rg = graph(dense_core_graph(40, 4, 60, 0.05, 3))
+        ref = oracle_for(rg)
+        p = R.Plan(rg, waves_per_cu=wpc, pack=True, pack_waves_per_cu=1, pack_slots=1, want_root_stats=True, **kw)
+        err = same(p.run(), ref)
+        p.autotune(4)
+        err = err or same(p.run(), ref) or same(p.run(), ref)
+        p.free()
+        return err
+    yield "pack grows", lambda: pack_grows({}) or pack_grows({"share_bound": -1, "use_graph": True})
     yield "pack out of memory", lambda: pack_out_of_memory(False) or pack_out_of_memory(True)
 
 
