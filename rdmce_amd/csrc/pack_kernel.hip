@@ -67,8 +67,12 @@ namespace {
 // community graph, ms: looks every 4 passes 12.7 / 27.1, 8 12.5 / 24.0, 16
 // 13.7 / 23.8 (each gift copies a subproblem, and the taker starts with part
 // of a pass).
+#ifdef RDMCE_PACK_EAGER_GIFTS  // test builds: gifts on small graphs, counted by kind in the results' sharing fields
+constexpr uint32_t kPackPoll = 1, kPackSpare = 2;
+#else
 constexpr uint32_t kPackPoll = 8;
 constexpr uint32_t kPackSpare = 32;
+#endif
 
 template <int NW, int NX>
 struct PackCfg {
@@ -820,6 +824,10 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
       given += ~empty ? (uint32_t)__builtin_ctzll(~empty) : 64u;
       flag = 1 | ((uint64_t)n << 8) | ((uint64_t)cands << 32);
     }
+#ifdef RDMCE_PACK_EAGER_GIFTS
+    acc.published += range;
+    acc.owner += split;
+#endif
     state_add(a, (uint32_t)to, kWorking - kLooking);
     mail_stored();  // the mail is there before its flag
     if (l == 0) st_mail(out, flag);

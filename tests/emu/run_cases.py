@@ -268,6 +268,46 @@ def cases():
         p.free()
         return err
     yield "pack grows", lambda: pack_grows({}) or pack_grows({"share_bound": -1, "use_graph": True})
+    # Work handed to idle waves, in the build that looks for them after every
+    # pass and counts gifts of runs and of a record's candidates in
+    # published_levels and owner_tasks (elsewhere these cases prove nothing).
+    def pack_gifts(rg, want, lists=False, **kw):
+        vertex = kw.get("root_mode") == R.ROOT_VERTEX
+        og = OracleGraph.from_csr(rg.GetRowOffset(), rg.GetColIdx(), rg.GetLabels(), rg.GetDegeneracy())
+        if "root_order" in kw:
+            ref = og.mce_roots(kw["root_order"], root_mode=1 if vertex else 2)
+        else:
+            ref = og.mce(root_mode=1 if vertex else 2, root_nodes=True, list_cap=1 << 20)
+        p = R.Plan(rg, waves_per_cu=wpc, pack=True, pack_waves_per_cu=4, share_bound=1, want_list=lists,
+                   want_root_stats=True, **kw)
+        seen = {"runs": 0, "candidates": 0, "records": 0}
+        for _ in range(6):  # who is idle when differs from run to run
+            o = p.run()
+            err = same(o, ref, lists=lists, nodes="root_order" not in kw)
+            if err:
+                return err
+            seen["runs"] += o.published_levels
+            seen["candidates"] += o.owner_tasks
+            seen["records"] += o.shared_tasks - o.published_levels - o.owner_tasks
+            if all(seen[k] > 0 for k in want):
+                break
+        p.free()
+        return None if all(seen[k] > 0 for k in want) else f"gifts {seen}, expected {want}"
+    gg = graph(random_graph(60, 0.7, 2))
+    yield "pack gifts edge roots", lambda: pack_gifts(gg, ["runs", "records"])
+    yield "pack gifts clique lists", lambda: pack_gifts(gg, ["runs", "records"], lists=True)
+    yield "pack gifts vertex roots", lambda: pack_gifts(gg, ["records"], root_mode=R.ROOT_VERTEX)
+    heavy = np.array([np.argmax(oracle_for(gg, root_mode=1).root_nodes)], dtype=np.uint64)
+    yield "pack gifts one root", lambda: pack_gifts(gg, ["records"], root_mode=R.ROOT_VERTEX, root_order=heavy)
+
+    def pack_gifts_wide_top():
+        # vertex 0 with 100 later neighbours that are not adjacent: one record
+        # with 100 candidates, of which a pass takes 64
+        rg = R.Graph.from_edges([(0, v) for v in range(1, 101)])
+        first = np.zeros(1, dtype=np.uint64)
+        return (pack_gifts(rg, ["candidates"], root_mode=R.ROOT_VERTEX, root_order=first)
+                or pack_gifts(rg, ["candidates"], lists=True, root_mode=R.ROOT_VERTEX))
+    yield "pack gifts wide top", pack_gifts_wide_top
     yield "pack out of memory", lambda: pack_out_of_memory(False) or pack_out_of_memory(True)
 
 
