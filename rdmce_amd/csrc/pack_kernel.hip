@@ -729,7 +729,10 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
   auto give = [&]() {
     const KArgs &a = cold_args(w.a);
     const uint32_t l = cold_lane();
-    const bool range = gend - gcur >= 2;
+    // The last unbuilt root goes before records of a deep stack do: records
+    // that were given away stay in it as empty ones, and a root built on top of
+    // those would need its own 64 records per level beyond pk_thr.
+    const bool range = gend - gcur >= (top > a.pk_thr ? 1u : 2u);
     uint64_t dm = 0, sel_m = 0;
     uint32_t ci = 0, s0 = 0, cands = 0, mid = 0;
     bool split = false, take = false;
@@ -791,7 +794,7 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
     uint64_t *out = a.pk_mail + (uint64_t)to * kPackMailWords;
     uint64_t flag;
     if (range) {  // the upper half of the run's unbuilt roots
-      const uint64_t at = gcur + (gend - gcur + 1) / 2;
+      const uint64_t at = gend - gcur > 1 ? gcur + (gend - gcur + 1) / 2 : gcur;
       if (l == 0) {
         st_mail(out + 1, at);
         st_mail(out + 2, gend);
@@ -943,6 +946,9 @@ __device__ __forceinline__ void pack_main(const KArgs &a) {
                                    map32);
         }
       }
+#ifdef RDMCE_PACK_EAGER_GIFTS  // test builds: the stack's bound counts on this
+      if (top > a.pk_thr + 64 && l == 0) atomicOr(a.err, kErrPackStack);
+#endif
       const uint64_t i = gcur++;
       const uint64_t canon = bcast64(a.perm ? a.perm[i] : (a.reverse ? n_dispatch - 1 - i : i));
       if (a.eager && bcast32(a.eager[i])) {  // split before launch: to the one-root-per-wave kernel

@@ -308,6 +308,19 @@ def cases():
         return (pack_gifts(rg, ["candidates"], root_mode=R.ROOT_VERTEX, root_order=first)
                 or pack_gifts(rg, ["candidates"], lists=True, root_mode=R.ROOT_VERTEX))
     yield "pack gifts wide top", pack_gifts_wide_top
+
+    def pack_gifts_last_root():
+        # a run of three heavy roots, of which two are searched at once: while
+        # their stack is deep, the third is given away before records are
+        rg = graph(random_graph(64, 0.8, 3))
+        n = oracle_for(rg).root_nodes.astype(np.int64)
+        v0 = (rg.roots(R.ROOT_EDGE) >> np.uint64(32)).astype(np.int64)
+        best = max(set(v0.tolist()), key=lambda v: np.sort(n[v0 == v])[-3:].sum())
+        ids = np.nonzero(v0 == best)[0]
+        ids = ids[np.argsort(-n[ids])][:3].astype(np.uint64)
+        return pack_gifts(rg, ["runs", "records"], root_order=ids, runs=np.array([0, 3], dtype=np.uint64),
+                          pack_slots=2)
+    yield "pack gifts last root", pack_gifts_last_root
     yield "pack out of memory", lambda: pack_out_of_memory(False) or pack_out_of_memory(True)
 
 
