@@ -289,8 +289,8 @@ void mce_cost_model_free(mce_cost_model *m);
 /* For callers that cannot allocate device memory: code under HIP graph       */
 /* capture, tight serving loops, harnesses that forbid hipMalloc.  Every      */
 /* scratch buffer lives in one static device array of                          */
-/* MCE_NOALLOC_SCRATCH_BYTES per device, held until the process ends; calls    */
-/* that overlap on one device race on it.                                      */
+/* MCE_NOALLOC_SCRATCH_BYTES (and 51 KB of counters) per device, held until    */
+/* the process ends; calls that overlap on one device race on it.              */
 /* ------------------------------------------------------------------------ */
 #define MCE_NOALLOC_SCRATCH_BYTES (64ull << 20)
 #define MCE_NOALLOC_ERR_SCRATCH (1ull << 31)

@@ -22,18 +22,21 @@ using namespace rdmce;
 namespace {
 
 constexpr uint64_t kScratchBytes = MCE_NOALLOC_SCRATCH_BYTES;
-static __device__ __align__(256) uint8_t scratch[kScratchBytes];
+// Counters kept in copies (u64 each: dispatch, work state, sums, clique
+// sizes), behind the scratch proper: how much of that a graph leaves for the
+// waves decides which graphs and roots fit.
+enum Copies { cNext, cState = cNext + kShards * kShardWords, cSums = cState + kStateShards * kShardWords,
+              cHistSh = cSums + kShards * kShardWords, cNumCopies = cHistSh + kShards * kLdsHist };
+static __device__ __align__(256) uint8_t scratch[kScratchBytes + 8 * cNumCopies];
 
 constexpr int kMaxDevices = 64;
 constexpr uint32_t kWavesPerCu = 4;     // few waves, large per-wave regions
 constexpr uint32_t kDeferCap = 1024;
 constexpr uint32_t kScanThreads = 1024;
 
-// Counters in the array (u64 each): the collected sums (Sum), the others,
-// then those kept in copies (dispatch, work state, sums, clique sizes).
+// Counters in the scratch (u64 each): the collected sums (Sum), then the others.
 enum Ctr { cCount = sCount, cHash = sHash, cNodes = sNodes, cList = kNumSums, cNDeferred, cDeferNeed, cDeferStackNeed,
-           cErr, cNext = 32, cState = cNext + kShards * kShardWords, cSums = cState + kStateShards * kShardWords,
-           cHistSh = cSums + kShards * kShardWords, cNum = cHistSh + kShards * kLdsHist };
+           cErr, cNum };
 
 std::mutex g_mu;
 uint8_t *g_scratch[kMaxDevices] = {};
@@ -174,12 +177,14 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
 
   hipStream_t s = (hipStream_t)stream;
   unsigned long long *ctr = (unsigned long long *)(base + o_ctr);
+  unsigned long long *copies = (unsigned long long *)(base + kScratchBytes);
   unsigned long long *hist = (unsigned long long *)(base + o_hist);
   uint64_t *outoff = (uint64_t *)(base + o_outoff), *rfirst = (uint64_t *)(base + o_rfirst);
   uint64_t *roots = (uint64_t *)(base + o_roots);
   // Resets with a fill kernel (no memset nodes if the caller captures this).
   FillList f;
   f.add(ctr, cNum);
+  f.add(copies, cNumCopies);
   f.add(hist, hist_len);
   f.add(base + o_recs, sizeof(ShareRec) / 8 * (uint64_t)waves);
   f.add(base + o_users, (waves + 2) / 2);
@@ -205,10 +210,10 @@ extern "C" mce_status mce_solve_device_csr_noalloc(int32_t device, uint64_t n, u
     a.n_dispatch = m;
     a.reverse = 1;  // high core first, BkPivotBitBalance.cuh:429-431
     a.root_mode = MCE_ROOT_EDGE;
-    a.next_root = ctr + cNext;
-    a.state = ctr + cState;
-    a.sums = ctr + cSums;
-    a.hist_sh = ctr + cHistSh;
+    a.next_root = copies + cNext;
+    a.state = copies + cState;
+    a.sums = copies + cSums;
+    a.hist_sh = copies + cHistSh;
     a.list_cursor = ctr + cList;
     a.n_deferred = ctr + cNDeferred;
     a.deferred_need = ctr + cDeferNeed;
