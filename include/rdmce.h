@@ -111,7 +111,9 @@ typedef struct mce_options {
   int32_t root_mode;         /* MCE_ROOT_EDGE (default) or MCE_ROOT_VERTEX */
   int32_t waves_per_cu;      /* resident wavefronts per CU (1..32; 0 = 16), WARP_PER_SM analogue; also picks the
                                 kernel compiled for that occupancy (<=16, <=20, <=24, <=32) */
-  int32_t share_bound;       /* TASK_SHARE_BOUND: |P| at which a level is exposed; 0 = 24; <0 = off */
+  int32_t share_bound;       /* TASK_SHARE_BOUND: |P| at which a level is exposed; 0 = 24; <0 = off.  Packed
+                                search: waves give work away where some root has that many candidates (or is
+                                flagged eager); <0 turns that off as well */
   int32_t want_list;         /* 1 = return the clique list */
   int32_t want_root_stats;   /* 1 = return per-root node counts and wave cycles */
   int32_t schedule;          /* MCE_SCHED_* */
@@ -157,7 +159,8 @@ typedef struct mce_result {
   uint64_t *root_cycles;     /* per canonical root: wave cycles spent (want_root_stats) */
   uint64_t total_nodes;
   uint64_t deferred_roots;   /* roots re-run in the large-scratch pass */
-  uint64_t shared_tasks;     /* subtrees handed between wavefronts */
+  uint64_t shared_tasks;     /* subtrees handed between wavefronts (packed search: gifts taken, each a
+                                range of roots or part of a record stack) */
   double kernel_ms;          /* device time of the enumeration kernels (HIP events) */
   double total_ms;           /* wall time of the call */
   int32_t passes;
