@@ -177,7 +177,6 @@ struct Acc {
   unsigned long long words;
   unsigned long long build;
   unsigned long long scan;  // per lane: adjacency entries of the bitmap rows' runs
-  unsigned long long lwords;  // per lane: more of `words`
   unsigned long long nodes;
   uint32_t shared, published, owner;  // sharing: see Sum
 };
@@ -187,9 +186,6 @@ __device__ __forceinline__ unsigned int ld_relaxed(unsigned int *p) {
 }
 __device__ __forceinline__ unsigned long long ld_relaxed(unsigned long long *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ unsigned int ld_acquire(unsigned int *p) {
-  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Sleeps about 256 * n cycles (s_sleep takes an immediate operand).
 __device__ __forceinline__ void nap(uint32_t n) {
