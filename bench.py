@@ -156,8 +156,8 @@ def roofline(out, kernel_ms: float, workload: str, plain=None):
     return {"bound": bound, "achieved": achieved, "peak": peak, "unit": unit, "frac": t_lb / t,
             "traffic": read_profile(f"pack_{workload.replace('-', '_')}_pmc", "traffic_bytes_per_step"),
             "t_lb_ms": t_lb * 1e3, "build_bytes": b_build,
-            "build_bytes_denominator": "per-root builds (one-root-per-wave kernel, same roots)"
-            if plain is not None else "the measured kernels' own builds",
+            "build_bytes_denominator": "per-root builds (one-root-per-wave kernel, same roots); the packed search "
+            "shares builds between roots, so frac can pass 1: see own_build" if plain is not None else "the measured kernels' own builds",
             "search_bytes": b_search, "search_ops": ops,
             "ceilings_ms": {k: v[0] * 1e3 for k, v in ceil.items()},
             "frac_of_peak": {k: v[1] / v[2] for k, v in ceil.items()},
